@@ -22,6 +22,7 @@ SOURCES = [
     "mesh/batch.cpp",
     "mesh/gmsh.cpp",
     "mesh/reorder.cpp",
+    "device/ilu_plan.cpp",
     "device/fv_kernels.hip",
     "device/keps_kernels.hip",
     "device/transient_kernels.hip",

@@ -8,6 +8,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <numeric>
 #include <stdexcept>
 
 #include "common.hpp"
@@ -692,21 +693,10 @@ void fill_info(const KResult& r, s355_solve_info* info) {
 
 void Context::ensure_ilu() {
   if (have_levels_) return;
-  std::vector<int> lrows, urows;
-  ilu_levels(dm.Nc, mesh.rowptr.data(), mesh.col.data(), mesh.diag.data(), lrows, levels_.lptr, urows, levels_.uptr);
-  levels_.lrows = upload(allocs_, lrows, stream);
-  levels_.urows = upload(allocs_, urows, stream);
-  // positions of each row in the two level orders (the sweeps' z spaces)
-  std::vector<int> lpos(dm.Nc), upos(dm.Nc), l2u(dm.Nc);
-  for (int p = 0; p < dm.Nc; ++p) {
-    lpos[lrows[p]] = p;
-    upos[urows[p]] = p;
-  }
-  for (int p = 0; p < dm.Nc; ++p) l2u[p] = upos[lrows[p]];
-  levels_.lpos = upload(allocs_, lpos, stream);
   {
-    std::vector<int> sptr, sp, sd, su, sr, sq;
-    ilu_steps(dm.Nc, mesh.rowptr.data(), mesh.col.data(), mesh.diag.data(), lrows, sptr, sp, sd, su, sr, sq);
+    std::vector<int> rows, sptr, sp, sd, su, sr, sq;
+    ilu_levels(dm.Nc, mesh.rowptr.data(), mesh.col.data(), mesh.diag.data(), rows, levels_.lptr);
+    ilu_steps(dm.Nc, mesh.rowptr.data(), mesh.col.data(), mesh.diag.data(), rows, sptr, sp, sd, su, sr, sq);
     levels_.steps.ptr = upload(allocs_, sptr, stream);
     levels_.steps.p = upload(allocs_, sp, stream);
     levels_.steps.d = upload(allocs_, sd, stream);
@@ -715,29 +705,56 @@ void Context::ensure_ilu() {
     levels_.steps.q = upload(allocs_, sq, stream);
     sync();  // host staging vectors go out of scope
   }
-  levels_.l2u = upload(allocs_, l2u, stream);
-  levels_.upos = upload(allocs_, upos, stream);
-  // level-ELL copies of the factors for the sweeps
-  for (int up = 0; up < 2; ++up) {
-    IluEll& e = up ? levels_.uell : levels_.lell;
-    std::vector<int> ecol, esrc, len, dsrc;
-    ilu_ell(dm.Nc, mesh.rowptr.data(), mesh.col.data(), mesh.diag.data(), up ? urows : lrows,
-            up ? levels_.uptr : levels_.lptr, up ? upos : lpos, up != 0, e.off, ecol, esrc, len, dsrc);
-    e.slots = esrc.size();
-    e.col = upload(allocs_, ecol, stream);
-    e.src = upload(allocs_, esrc, stream);
-    e.len = upload(allocs_, len, stream);
-    if (up) e.dsrc = upload(allocs_, dsrc, stream);
+  auto put = [&](IluSweep& w, const IluPlan& p, bool up) {
+    w.n = p.n;
+    w.subs = p.subs;
+    w.group = p.group;
+    w.dptr = p.dptr;
+    w.slots = p.col.size();
+    w.len = upload(allocs_, p.len, stream);
+    w.slot0 = upload(allocs_, p.slot0, stream);
+    w.stride = upload(allocs_, p.stride, stream);
+    w.col = upload(allocs_, p.col, stream);
+    w.src = upload(allocs_, p.src, stream);
+    w.later = upload(allocs_, p.later, stream);
+    w.sptr = upload(allocs_, p.sptr, stream);
+    w.p = upload(allocs_, p.p, stream);
+    w.uptr = upload(allocs_, p.uptr, stream);
+    w.r = upload(allocs_, p.r, stream);
+    w.q = upload(allocs_, p.q, stream);
+    if (up) {
+      std::vector<int> dsrc(p.n);
+      for (int k = 0; k < p.n; ++k) {
+        const int d = mesh.diag[p.rows[k]];
+        dsrc[k] = p.depth[k] ? -1 - d : d;
+      }
+      w.dsrc = upload(allocs_, dsrc, stream);
+      sync();
+    }
+  };
+  {
+    std::vector<int> natural(dm.Nc);
+    std::iota(natural.begin(), natural.end(), 0);
+    const IluPlan lower = ilu_plan(dm.Nc, mesh.rowptr.data(), mesh.col.data(), mesh.diag.data(), false, natural,
+                                   lay.cell);
+    put(levels_.lower, lower, false);
+    const IluPlan upper = ilu_plan(dm.Nc, mesh.rowptr.data(), mesh.col.data(), mesh.diag.data(), true, lower.rows,
+                                   lay.cell);
+    put(levels_.upper, upper, true);
+    std::vector<int> l2u(dm.Nc);
+    for (int q = 0; q < dm.Nc; ++q) l2u[q] = upper.pos[lower.rows[q]];
+    levels_.lpos = upload(allocs_, lower.pos, stream);
+    levels_.l2u = upload(allocs_, l2u, stream);
+    levels_.upos = upload(allocs_, upper.pos, stream);
     sync();  // host staging vectors go out of scope
   }
   kwork_.lu = alloc<double>(dm.nnz);
-  kwork_.ilu_lval = alloc<double>(levels_.lell.slots);
-  kwork_.ilu_uval = alloc<double>(levels_.uell.slots);
-  kwork_.ilu_dval = alloc<double>(dm.Nc);
-  kwork_.ilu_zl = alloc<double>(dm.Nc);
-  kwork_.ilu_zu = alloc<double>(dm.Nc);
+  kwork_.ilu_lcoef = alloc<double>(levels_.lower.slots);
+  kwork_.ilu_ucoef = alloc<double>(levels_.upper.slots);
+  kwork_.ilu_own = alloc<double>(dm.Nc);
+  kwork_.ilu_zl = alloc<double>(2 * static_cast<size_t>(dm.Nc));
+  kwork_.ilu_zu = alloc<double>(2 * static_cast<size_t>(dm.Nc));
   kwork_.ilu = &levels_;
-  sync();  // host staging of the level lists
   have_levels_ = true;
 }
 
@@ -783,12 +800,12 @@ int Context::run_solve(int which, const double* b, double* x, const s355_ksp_opt
     // FP32 inner solves on the rounded matrix inside FP64 refinement
     ensure_mixed();
     kwork32_.ilu = kwork_.ilu;
-    if (kwork32_.ilu && !kwork32_.ilu_lval) {
-      kwork32_.ilu_lval = alloc<float>(levels_.lell.slots);
-      kwork32_.ilu_uval = alloc<float>(levels_.uell.slots);
-      kwork32_.ilu_dval = alloc<float>(dm.Nc);
-      kwork32_.ilu_zl = alloc<float>(dm.Nc);
-      kwork32_.ilu_zu = alloc<float>(dm.Nc);
+    if (kwork32_.ilu && !kwork32_.ilu_lcoef) {
+      kwork32_.ilu_lcoef = alloc<float>(levels_.lower.slots);
+      kwork32_.ilu_ucoef = alloc<float>(levels_.upper.slots);
+      kwork32_.ilu_own = alloc<float>(dm.Nc);
+      kwork32_.ilu_zl = alloc<float>(2 * static_cast<size_t>(dm.Nc));
+      kwork32_.ilu_zu = alloc<float>(2 * static_cast<size_t>(dm.Nc));
     }
     CsrView<float> A{dm.Nc, dm.rowptr, dm.col, dm.diag, a32_, dm.nnz};
     CsrView<double> A64{dm.Nc, dm.rowptr, dm.col, dm.diag, val, dm.nnz};

@@ -1,0 +1,245 @@
+#include "ilu_plan.hpp"
+
+#include <algorithm>
+#include <memory>
+#include <stdexcept>
+
+#include "../mesh/parallel.hpp"
+
+namespace s355 {
+namespace {
+
+constexpr long kMost = 0x7fffffffL;
+
+// n ints without filling them
+struct Ints {
+  std::unique_ptr<int[]> p;
+  explicit Ints(size_t n) : p(new int[n ? n : 1]) {}
+  int& operator[](size_t i) { return p[i]; }
+};
+
+}  // namespace
+
+IluPlan ilu_plan(int n, const int* rowptr, const int* col, const int* diag, bool upper, const std::vector<int>& order,
+                 const std::vector<int>& cases, int merge_levels, int merge_rows) {
+  if (n > kMost / 2) throw std::invalid_argument("ILU(0) sweeps above 32-bit indices");
+  if (merge_levels < 1 || merge_levels > kMergeLevels) throw std::invalid_argument("ilu_plan: merge_levels");
+  // the merged rows' terms fit 32-bit indices below this many rows on any mesh
+  // of hexahedra and tetrahedra; above it the levels are large anyway
+  if (n > (1 << 26)) merge_levels = 1;
+  IluPlan out;
+  out.n = n;
+  auto first = [&](int i) { return upper ? diag[i] + 1 : rowptr[i]; };
+  auto last = [&](int i) { return upper ? rowptr[i + 1] : diag[i]; };
+
+  std::vector<int> lev(n), grp(n), dep(n), most(n);  // most: terms of a row at most, its own input among them
+  for (int k = 0; k < n; ++k) {
+    const int i = upper ? n - 1 - k : k;
+    int l = 0;
+    for (int e = first(i); e < last(i); ++e) l = std::max(l, lev[col[e]] + 1);
+    lev[i] = l;
+  }
+  // groups, case by case; dlist: the rows of each depth
+  std::vector<std::vector<int>> dlist(merge_levels);
+  int ngroup = 0;
+  for (size_t c = 0; c + 1 < cases.size(); ++c) {
+    const int a = cases[c], e = cases[c + 1];
+    if (e <= a) continue;
+    int nlev = 0;
+    for (int i = a; i < e; ++i) nlev = std::max(nlev, lev[i] + 1);
+    std::vector<int> lptr(nlev + 1, 0), lrows(e - a);
+    for (int i = a; i < e; ++i) ++lptr[lev[i] + 1];
+    for (int l = 0; l < nlev; ++l) lptr[l + 1] += lptr[l];
+    {
+      std::vector<int> at(lptr.begin(), lptr.end() - 1);
+      for (int i = a; i < e; ++i) lrows[at[lev[i]]++] = i;
+    }
+    int g = -1, begin = 0;  // the open group and its first level
+    for (int l = 0; l < nlev; ++l) {
+      bool joins = g >= 0 && l - begin < merge_levels && lptr[l + 1] - lptr[begin] <= merge_rows;
+      for (int k = lptr[l]; joins && k < lptr[l + 1]; ++k) {
+        const int i = lrows[k];
+        int m = 1;
+        for (int x = first(i); x < last(i); ++x) m += lev[col[x]] >= begin ? most[col[x]] : 1;
+        most[i] = m;
+        joins = m <= kMergeTerms;
+      }
+      if (!joins) {
+        ++g;
+        begin = l;
+        for (int k = lptr[l]; k < lptr[l + 1]; ++k) most[lrows[k]] = 1 + last(lrows[k]) - first(lrows[k]);
+      }
+      const int d = l - begin;
+      for (int k = lptr[l]; k < lptr[l + 1]; ++k) {
+        grp[lrows[k]] = g;
+        dep[lrows[k]] = d;
+      }
+      dlist[d].insert(dlist[d].end(), lrows.begin() + lptr[l], lrows.begin() + lptr[l + 1]);
+    }
+    ngroup = std::max(ngroup, g + 1);
+  }
+
+  // the terms of every row, depth by depth.  Code j: the input of row j, n + j:
+  // the result of row j.  Row i's terms are at start[i], count[i] of them; so
+  // are, for a row below depth 0, its pairs (term of the row, term of the row
+  // referred to, -1 its own input), one run per reference in CSR order.
+  std::vector<long> start(static_cast<size_t>(n) + 1, 0);
+  for (int i = 0; i < n; ++i) start[i + 1] = start[i] + most[i];
+  Ints code(start[n]), src(start[n]), pr(start[n]), pq(start[n]);
+  std::vector<int> count(n), nstep(n, 0), npair(n, 0);
+  for (int d = 0; d < merge_levels; ++d) {
+    const std::vector<int>& list = dlist[d];
+    parallel_for(
+        static_cast<long>(list.size()),
+        [&](long k) {
+          const int i = list[k];
+          const long s = start[i];
+          int m = 0, pairs = 0, steps = 0;
+          auto term = [&](int c) {
+            int u = 0;
+            while (u < m && code[s + u] != c) ++u;
+            if (u == m) {
+              code[s + m] = c;
+              src[s + m] = -1;
+              ++m;
+            }
+            return u;
+          };
+          for (int x = first(i); x < last(i); ++x) {
+            const int j = col[x];
+            if (grp[j] != grp[i]) {
+              src[s + term(n + j)] = x;
+              continue;
+            }
+            ++steps;
+            for (int y = -1; y < count[j]; ++y) {  // -1: row j's own input
+              pr[s + pairs] = term(y < 0 ? j : code[start[j] + y]);
+              pq[s + pairs] = y;
+              ++pairs;
+            }
+          }
+          count[i] = m;
+          nstep[i] = steps;
+          npair[i] = pairs;
+        },
+        1 << 12);
+  }
+
+  // sweep order: by (group, class), keeping the order given
+  auto key = [&](int i) {
+    int c = 0;
+    while (count[i] > kTermWidth[c]) ++c;
+    return static_cast<long>(grp[i]) * kTermClasses + c;
+  };
+  const long nkey = static_cast<long>(ngroup) * kTermClasses;
+  std::vector<int> kptr(nkey + 1, 0), width(nkey, 0);
+  for (int i = 0; i < n; ++i) {
+    const long k = key(i);
+    ++kptr[k + 1];
+    width[k] = std::max(width[k], count[i]);
+  }
+  for (long k = 0; k < nkey; ++k) kptr[k + 1] += kptr[k];
+  out.rows.resize(n);
+  out.pos.resize(n);
+  {
+    std::vector<int> at(kptr.begin(), kptr.end() - 1);
+    for (int i : order) {
+      const int p = at[key(i)]++;
+      out.rows[p] = i;
+      out.pos[i] = p;
+    }
+  }
+  long slots = 0;
+  out.group.assign(1, 0);
+  out.len.resize(n);
+  out.slot0.resize(n);
+  out.stride.resize(n);
+  out.depth.resize(n);
+  for (int g = 0; g < ngroup; ++g) {
+    for (int c = 0; c < kTermClasses; ++c) {
+      const long k = static_cast<long>(g) * kTermClasses + c;
+      const int p0 = kptr[k], nr = kptr[k + 1] - p0;
+      if (nr == 0) continue;
+      if (c + 1 < kTermClasses)
+        width[k] = kTermWidth[c];
+      else
+        width[k] = (width[k] + kTermBatch - 1) / kTermBatch * kTermBatch;
+      out.subs.push_back(IluSub{slots, p0, nr, width[k], c});
+      if (slots + static_cast<long>(width[k]) * nr > kMost)
+        throw std::invalid_argument("ILU(0) sweep slots above 32-bit indices");
+      for (int p = p0; p < p0 + nr; ++p) {
+        out.slot0[p] = static_cast<int>(slots + (p - p0));
+        out.stride[p] = nr;
+      }
+      slots += static_cast<long>(width[k]) * nr;
+    }
+    out.group.push_back(static_cast<int>(out.subs.size()));
+  }
+  out.col.resize(slots);
+  out.src.resize(slots);
+  for (const IluSub& sub : out.subs)
+    parallel_for(
+        sub.nrows,
+        [&](long k) {
+          const int p = sub.p0 + static_cast<int>(k), i = out.rows[p];
+          out.len[p] = count[i];
+          out.depth[p] = dep[i];
+          for (int u = 0; u < sub.width; ++u) {
+            const size_t at = static_cast<size_t>(sub.off) + static_cast<size_t>(u) * sub.nrows + k;
+            if (u < count[i]) {
+              const int c = code[start[i] + u];
+              out.col[at] = c < n ? out.pos[c] : n + out.pos[c - n];
+              out.src[at] = src[start[i] + u];
+            } else {
+              out.col[at] = p;
+              out.src[at] = -1;
+            }
+          }
+        },
+        1 << 13);
+
+  // the steps of the rows below depth 0
+  out.dptr.assign(1, 0);
+  for (int d = 1; d < merge_levels; ++d) {
+    for (int p = 0; p < n; ++p)
+      if (out.depth[p] == d) out.later.push_back(p);
+    out.dptr.push_back(static_cast<int>(out.later.size()));
+  }
+  const size_t nl = out.later.size();
+  out.sptr.assign(nl + 1, 0);
+  std::vector<long> pairs(nl + 1, 0);
+  long steps = 0;
+  for (size_t k = 0; k < nl; ++k) {
+    const int i = out.rows[out.later[k]];
+    steps += nstep[i];
+    pairs[k + 1] = pairs[k] + npair[i];
+    if (steps > kMost || pairs[k + 1] > kMost) throw std::invalid_argument("ILU(0) sweep steps above 32-bit indices");
+    out.sptr[k + 1] = static_cast<int>(steps);
+  }
+  out.p.resize(steps);
+  out.uptr.assign(static_cast<size_t>(steps) + 1, 0);
+  out.r.resize(pairs[nl]);
+  out.q.resize(pairs[nl]);
+  parallel_for(
+      static_cast<long>(nl),
+      [&](long k) {
+        const int pi = out.later[k], i = out.rows[pi];
+        int x0 = out.sptr[k];
+        long at = pairs[k], from = start[i];
+        for (int x = first(i); x < last(i); ++x) {
+          const int j = col[x];
+          if (grp[j] != grp[i]) continue;
+          const int pj = out.pos[j];
+          out.p[x0] = x;
+          for (int y = -1; y < count[j]; ++y, ++at, ++from) {
+            out.r[at] = out.slot0[pi] + pr[from] * out.stride[pi];
+            out.q[at] = pq[from] < 0 ? -1 - pj : out.slot0[pj] + pq[from] * out.stride[pj];
+          }
+          out.uptr[++x0] = static_cast<int>(at);
+        }
+      },
+      1 << 12);
+  return out;
+}
+
+}  // namespace s355

@@ -46,10 +46,10 @@ __global__ void __launch_bounds__(kBlock) k_jacobi_setup(CsrView<T> A, T* inv) {
   inv[i] = static_cast<T>(d != 0.0 ? 1.0 / d : 1.0);
 }
 
-// Workgroup size of a level launch of the ILU(0) factorisation and sweeps: a
-// level below 64 K rows launches one-wave workgroups, so its rows spread over
+// Workgroup size of a launch of the ILU(0) factorisation and sweeps: a
+// launch below 64 K rows has one-wave workgroups, so its rows spread over
 // all CUs (each row is a chain of dependent loads, not a share of bandwidth);
-// larger levels keep 256-thread workgroups.
+// larger launches keep 256-thread workgroups.
 inline int level_block(int nrows) { return nrows < (kBlock << 8) ? kWave : kBlock; }
 
 // ---- ILU(0), natural ordering, one thread per row of a level.  IKJ
@@ -73,72 +73,142 @@ __global__ void __launch_bounds__(kBlock) k_ilu_factor(T* __restrict__ lu, IluSt
   }
 }
 
-// One level of the lower (z = L^-1 z) or upper (z = U^-1 z) sweep on the
-// level-ELL copy, in place in level space: the level's k-th row sits at
-// position p0 + k of the sweep's order, where its input is found, its result
-// is stored and the column ids of later levels point.  Row k has L entries
-// among the level's `width` slots (padding: value 0, column = the row's own
-// position, so every slot's gather is in bounds).  All width slots' values
-// and column ids load before the state check; then the row's input and the
-// gathers of z; the entries are subtracted in entry order, the padding never.
-constexpr int kEllBatch = 8;
-template <class T, bool Upper>
-__global__ void __launch_bounds__(kBlock) k_ilu_sweep_ell(const int* __restrict__ len, const int* __restrict__ ecol,
-                                                          const T* __restrict__ eval, const T* __restrict__ dval,
-                                                          long base, int p0, int nrows, int width, T* zs,
-                                                          const KState* st) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= nrows) return;
-  const int L = len[k];
-  const int w0 = width < kEllBatch ? width : kEllBatch;
-  T v[kEllBatch], zv[kEllBatch];
-  int c[kEllBatch];
+// One group of a sweep (see ilu_plan.hpp): each row sums its terms over the
+// sweep's inputs and the earlier groups' results, one thread per row, in
+// place of a launch per level.  A level of a few thousand rows is bound by
+// the launch and the chain slots -> gathers -> store, so all of a row's
+// slots load before any is used and all its gathers before any is added: the
+// rows of a launch come in classes of term counts, each a run of workgroups
+// compiled for its padded width, its loads unconditional (guarded ones wait
+// for each other).  A longer row than the widest class takes batches.
+struct IluLaunch {
+  // per class; blk0: its first workgroup (empty classes: nrows 0, where the
+  // next class starts)
+  long off[kTermClasses];
+  int p0[kTermClasses], nrows[kTermClasses], width[kTermClasses], blk0[kTermClasses];
+};
+
+template <class T, int W>
+__device__ __forceinline__ T ilu_row(const int* __restrict__ col, const T* __restrict__ coef, const T* buf, size_t q0,
+                                     int nrows, int L, T s) {
+  T v[W], x[W];
+  int c[W];
 #pragma unroll
-  for (int u = 0; u < kEllBatch; ++u)
-    if (u < w0) {
-      const size_t q = static_cast<size_t>(base) + static_cast<size_t>(u) * nrows + k;
-      v[u] = eval[q];
-      c[u] = ecol[q];
-    }
-  T d = T(1);
-  if constexpr (Upper) d = dval[k];
-  if (st && st->reason) return;
-  T s = zs[p0 + k];
-#pragma unroll
-  for (int u = 0; u < kEllBatch; ++u)
-    if (u < w0) zv[u] = zs[c[u]];
-#pragma unroll
-  for (int u = 0; u < kEllBatch; ++u)
-    if (u < L) s -= v[u] * zv[u];
-  // rows longer than one batch (polyhedral cells): the rest, batch by batch
-  for (int j0 = kEllBatch; j0 < L; j0 += kEllBatch) {
-#pragma unroll
-    for (int u = 0; u < kEllBatch; ++u)
-      if (j0 + u < L) {
-        const size_t q = static_cast<size_t>(base) + static_cast<size_t>(j0 + u) * nrows + k;
-        v[u] = eval[q];
-        c[u] = ecol[q];
-      }
-#pragma unroll
-    for (int u = 0; u < kEllBatch; ++u)
-      if (j0 + u < L) zv[u] = zs[c[u]];
-#pragma unroll
-    for (int u = 0; u < kEllBatch; ++u)
-      if (j0 + u < L) s -= v[u] * zv[u];
+  for (int u = 0; u < W; ++u) {
+    v[u] = coef[q0 + static_cast<size_t>(u) * nrows];
+    c[u] = col[q0 + static_cast<size_t>(u) * nrows];
   }
-  if constexpr (Upper)
-    zs[p0 + k] = s / d;
-  else
-    zs[p0 + k] = s;
+#pragma unroll
+  for (int u = 0; u < W; ++u) x[u] = buf[c[u]];  // padding: the row's own input
+#pragma unroll
+  for (int u = 0; u < W; ++u) s = u < L ? s + v[u] * x[u] : s;
+  return s;
 }
 
-// The moves between the natural order and the sweeps' level orders (Tag
-// only names the move in kernel traces).  Inside a lower level rows keep
-// their natural order, inside an upper level their lower-level order, so the
-// rows of a run of consecutive source positions that fall in one level of
-// the destination order are consecutive there: a workgroup reading (or
-// writing) a contiguous range writes (reads) one short contiguous run per
-// level, and consecutive workgroups on one XCD extend the same runs in its L2.
+// (own: the coefficient of each row's own input, null: 1)
+template <class T, bool Wide>
+__global__ void __launch_bounds__(kBlock) k_ilu_group(IluLaunch g, const int* __restrict__ len,
+                                                      const int* __restrict__ col, const T* __restrict__ coef,
+                                                      const T* __restrict__ own, T* buf, int n, const KState* st) {
+  // the workgroup's class, by constant indices (the launch stays in registers)
+  const int blk = blockIdx.x;
+  int cls = 0, p0 = g.p0[0], nrows = g.nrows[0], width = g.width[0], blk0 = 0;
+  long off = g.off[0];
+#pragma unroll
+  for (int c = 1; c < (Wide ? kTermClasses : kNarrowClasses); ++c)
+    if (blk >= g.blk0[c]) {
+      cls = c;
+      p0 = g.p0[c];
+      nrows = g.nrows[c];
+      width = g.width[c];
+      blk0 = g.blk0[c];
+      off = g.off[c];
+    }
+  const int k = (blk - blk0) * static_cast<int>(blockDim.x) + threadIdx.x;
+  if (k >= nrows) return;
+  if (st && st->reason) return;
+  const int p = p0 + k, L = len[p];
+  const size_t q0 = static_cast<size_t>(off) + k;
+  T z = buf[p];
+  if (own) z *= own[p];
+  if (cls == 0) {
+    z = ilu_row<T, kTermWidth[0]>(col, coef, buf, q0, nrows, L, z);
+  } else if (cls == 1) {
+    z = ilu_row<T, kTermWidth[1]>(col, coef, buf, q0, nrows, L, z);
+  } else if (cls == 2) {
+    z = ilu_row<T, kTermWidth[2]>(col, coef, buf, q0, nrows, L, z);
+  } else if constexpr (Wide) {
+    switch (cls) {
+      case 3: z = ilu_row<T, kTermWidth[3]>(col, coef, buf, q0, nrows, L, z); break;
+      case 4: z = ilu_row<T, kTermWidth[4]>(col, coef, buf, q0, nrows, L, z); break;
+      case 5: z = ilu_row<T, kTermWidth[5]>(col, coef, buf, q0, nrows, L, z); break;
+      default:
+        for (int j = 0; j < width; j += kTermBatch)
+          z = ilu_row<T, kTermBatch>(col, coef, buf, q0 + static_cast<size_t>(j) * nrows, nrows, L - j, z);
+        break;
+    }
+  }
+  buf[static_cast<size_t>(n) + p] = z;
+}
+
+// The coefficients of a sweep from the factors: those of the rows at depth 0
+// (no reference to their own group), and the direct terms of the others.
+// (own: 1 / pivot in the upper sweep)
+template <class T, bool Upper>
+__global__ void __launch_bounds__(kBlock) k_ilu_coef(int n, const int* __restrict__ len, const int* __restrict__ slot0,
+                                                     const int* __restrict__ stride, const int* __restrict__ src,
+                                                     const int* __restrict__ dsrc, const T* __restrict__ lu,
+                                                     T* __restrict__ coef, T* __restrict__ own) {
+  const int p = blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= n) return;
+  const int L = len[p];
+  const size_t q0 = slot0[p], step = stride[p];
+  // dsrc < 0: a row below depth 0, divided by its pivot once its terms are complete
+  const int dp = Upper ? dsrc[p] : -1;
+  const T d = dp >= 0 ? lu[dp] : T(1);
+  for (int u = 0; u < L; ++u) {
+    const int e = src[q0 + u * step];
+    const T c = e >= 0 ? -lu[e] : T(0);
+    coef[q0 + u * step] = dp >= 0 ? c / d : c;
+  }
+  if (dp >= 0) own[p] = T(1) / d;
+}
+
+// ... and the rows of one depth d > 0, whose references to rows of lower depths
+// are replaced by those rows' terms
+template <class T, bool Upper>
+__global__ void __launch_bounds__(kBlock) k_ilu_merge(int k0, int nrows, const int* __restrict__ later,
+                                                      const int* __restrict__ sptr, const int* __restrict__ sp,
+                                                      const int* __restrict__ uptr, const int* __restrict__ r,
+                                                      const int* __restrict__ q, const int* __restrict__ len,
+                                                      const int* __restrict__ slot0, const int* __restrict__ stride,
+                                                      const int* __restrict__ dsrc, const T* __restrict__ lu, T* coef,
+                                                      T* own) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= nrows) return;
+  const int k = k0 + t, p = later[k];
+  for (int x = sptr[k]; x < sptr[k + 1]; ++x) {
+    const T a = lu[sp[x]];
+    for (int u = uptr[x]; u < uptr[x + 1]; ++u) {
+      const int e = q[u];
+      coef[r[u]] -= a * (e >= 0 ? coef[e] : (Upper ? own[-1 - e] : T(1)));
+    }
+  }
+  if constexpr (Upper) {
+    const T d = lu[-1 - dsrc[p]];
+    const size_t q0 = slot0[p], step = stride[p];
+    for (int u = 0; u < len[p]; ++u) coef[q0 + u * step] /= d;
+    own[p] = T(1) / d;
+  }
+}
+
+// The moves between the natural order and the sweeps' orders (Tag only
+// names the move in kernel traces).  Inside one run of a launch's rows (same
+// group, depth and class) rows keep their natural order in the lower sweep and
+// their lower-sweep order in the upper, so the rows of a range of consecutive
+// source positions that fall in one run of the destination order are
+// consecutive there: a workgroup reading (or writing) a contiguous range
+// writes (reads) one short contiguous piece per run, and consecutive workgroups on one XCD extend the same runs in its L2.
 // scatter: dst[pos[q]] = src[q]
 template <class T, int Tag>
 __global__ void __launch_bounds__(kBlock) k_scatter(int n, const int* __restrict__ pos, const T* __restrict__ src,
@@ -196,32 +266,63 @@ __global__ void __launch_bounds__(kBlock) k_gather(const int* __restrict__ src, 
   out[q] = p >= 0 ? lu[p] : T(0);
 }
 
-// ILU(0) factors of A into lu (CSR), then their level-ELL copies into the
-// workspace's value buffers when those are set
+// the coefficients of one sweep from the factors lu
+template <class T, bool Upper>
+void ilu_coefficients(const IluSweep& w, const T* lu, T* coef, T* own, hipStream_t s) {
+  hipLaunchKernelGGL((k_ilu_coef<T, Upper>), dim3(grid_for(w.n)), dim3(kBlock), 0, s, w.n, w.len, w.slot0, w.stride,
+                     w.src, w.dsrc, lu, coef, own);
+  for (size_t d = 0; d + 1 < w.dptr.size(); ++d) {
+    const int nr = w.dptr[d + 1] - w.dptr[d];
+    if (nr == 0) continue;
+    const int b = level_block(nr);
+    hipLaunchKernelGGL((k_ilu_merge<T, Upper>), dim3(grid_for(nr, b)), dim3(b), 0, s, w.dptr[d], nr, w.later, w.sptr,
+                       w.p, w.uptr, w.r, w.q, w.len, w.slot0, w.stride, w.dsrc, lu, coef, own);
+  }
+}
+
+// ILU(0) factors of A into lu (CSR), then the sweeps' coefficients
 template <class T>
-void ilu_factor(const CsrView<T>& A, int nnz, const IluLevels& lv, T* lu, hipStream_t s, const KWork* w = nullptr) {
+void ilu_factor(const CsrView<T>& A, int nnz, const IluLevels& lv, T* lu, hipStream_t s, const KWork* w) {
   S355_HIP(hipMemcpyAsync(lu, A.val, sizeof(T) * static_cast<size_t>(nnz), hipMemcpyDeviceToDevice, s));
-  if (!lv.steps.ptr) throw std::invalid_argument("ILU(0) factorisation without its elimination steps");
+  if (!lv.steps.ptr || !w->ilu_lcoef || !w->ilu_ucoef || !w->ilu_own)
+    throw std::invalid_argument("ILU(0) factorisation without its plan");
   for (int l = 0; l < lv.nl(); ++l) {
     const int nr = lv.lptr[l + 1] - lv.lptr[l];
     if (nr == 0) continue;
     const int b = level_block(nr);
     hipLaunchKernelGGL((k_ilu_factor<T>), dim3(grid_for(nr, b)), dim3(b), 0, s, lu, lv.steps, lv.lptr[l], nr);
   }
-  if (w && w->ilu_lval && lv.lell.col) {
-    const size_t nrow = lv.uptr.back();
-    hipLaunchKernelGGL((k_gather<T>), dim3(grid_for(static_cast<long>(lv.lell.slots))), dim3(kBlock), 0, s,
-                       lv.lell.src, lv.lell.slots, lu, static_cast<T*>(w->ilu_lval));
-    hipLaunchKernelGGL((k_gather<T>), dim3(grid_for(static_cast<long>(lv.uell.slots))), dim3(kBlock), 0, s,
-                       lv.uell.src, lv.uell.slots, lu, static_cast<T*>(w->ilu_uval));
-    hipLaunchKernelGGL((k_gather<T>), dim3(grid_for(static_cast<long>(nrow))), dim3(kBlock), 0, s, lv.uell.dsrc, nrow,
-                       lu, static_cast<T*>(w->ilu_dval));
-  }
+  ilu_coefficients<T, false>(lv.lower, lu, static_cast<T*>(w->ilu_lcoef), nullptr, s);
+  ilu_coefficients<T, true>(lv.upper, lu, static_cast<T*>(w->ilu_ucoef), static_cast<T*>(w->ilu_own), s);
   S355_LAUNCH_CHECK();
 }
 
-// z = (LU)^-1 r ; r and z distinct.  With a graph cache the level sweeps
-// (one launch per level) are captured once per (factor, r, z) and replayed.
+// one sweep, group by group, on buf: n inputs, then n results
+template <class T>
+void ilu_sweep(const IluSweep& w, const T* coef, const T* own, T* buf, const KState* st, hipStream_t s) {
+  for (size_t g = 0; g + 1 < w.group.size(); ++g) {
+    IluLaunch a{};
+    int rows = 0, blocks = 0, k = w.group[g];
+    for (int x = k; x < w.group[g + 1]; ++x) rows += w.subs[x].nrows;
+    const int b = level_block(rows);
+    for (int c = 0; c < kTermClasses; ++c) {
+      a.blk0[c] = blocks;
+      if (k == w.group[g + 1] || w.subs[k].cls != c) continue;
+      const IluSub& u = w.subs[k++];
+      a.off[c] = u.off;
+      a.p0[c] = u.p0;
+      a.nrows[c] = u.nrows;
+      a.width[c] = u.width;
+      blocks += grid_for(u.nrows, b);
+    }
+    const bool wide = w.subs[w.group[g + 1] - 1].cls >= kNarrowClasses;
+    hipLaunchKernelGGL((wide ? k_ilu_group<T, true> : k_ilu_group<T, false>), dim3(blocks), dim3(b), 0, s, a, w.len,
+                       w.col, coef, own, buf, w.n, st);
+  }
+}
+
+// z = (LU)^-1 r ; r and z distinct.  With a graph cache the sweeps (one
+// launch per group) are captured once per (factor, r, z) and replayed.
 // With dot (CG) the last move also leaves the partial sums of (z, z) and
 // (z, r) per kBlock rows there (see k_gather_at).
 template <class T>
@@ -230,45 +331,29 @@ void ilu_apply(const CsrView<T>& A, const IluLevels& lv, const T* lu, const T* r
   if (graphs) {
     const std::vector<uintptr_t> key = {0x11u, reinterpret_cast<uintptr_t>(lu), reinterpret_cast<uintptr_t>(r),
                                         reinterpret_cast<uintptr_t>(z), reinterpret_cast<uintptr_t>(st),
-                                        reinterpret_cast<uintptr_t>(lv.lrows), sizeof(T),
-                                        reinterpret_cast<uintptr_t>(w ? w->ilu_lval : nullptr),
+                                        reinterpret_cast<uintptr_t>(lv.lpos), sizeof(T),
+                                        reinterpret_cast<uintptr_t>(w ? w->ilu_lcoef : nullptr),
                                         reinterpret_cast<uintptr_t>(dot)};
     hipGraphExec_t g = graphs->get(key, s, [&] { ilu_apply(A, lv, lu, r, z, st, s, nullptr, w, dot); });
     S355_HIP(hipGraphLaunch(g, s));
     return;
   }
-  if (!w || !w->ilu_lval || !w->ilu_zl || !w->ilu_zu || !lv.lell.col || !lv.lpos || !lv.l2u || !lv.upos)
-    throw std::invalid_argument("ILU(0) application without its level-ELL workspace");
-  const T* lval = static_cast<const T*>(w->ilu_lval);
-  const T* uval = static_cast<const T*>(w->ilu_uval);
-  const T* dval = static_cast<const T*>(w->ilu_dval);
+  if (!w || !w->ilu_lcoef || !w->ilu_zl || !w->ilu_zu || !lv.lower.col || !lv.lpos || !lv.l2u || !lv.upos)
+    throw std::invalid_argument("ILU(0) application without its sweep workspace");
   T* zl = static_cast<T*>(w->ilu_zl);
   T* zu = static_cast<T*>(w->ilu_zu);
-  auto width = [](const IluEll& e, int l, int nr) { return static_cast<int>((e.off[l + 1] - e.off[l]) / nr); };
   const int n = lv.lptr.back();
   const int gn = grid_for(n);
   // r into the lower order, the lower sweep, its result into the upper
   // order, the upper sweep, z back into the natural order
   hipLaunchKernelGGL((k_scatter<T, 0>), dim3(gn), dim3(kBlock), 0, s, n, lv.lpos, r, zl, st);
-  for (int l = 0; l < lv.nl(); ++l) {
-    const int p0 = lv.lptr[l], nr = lv.lptr[l + 1] - p0;
-    if (nr == 0) continue;
-    const int b = level_block(nr);
-    hipLaunchKernelGGL((k_ilu_sweep_ell<T, false>), dim3(grid_for(nr, b)), dim3(b), 0, s, lv.lell.len + p0,
-                       lv.lell.col, lval, nullptr, lv.lell.off[l], p0, nr, width(lv.lell, l, nr), zl, st);
-  }
-  hipLaunchKernelGGL((k_scatter<T, 1>), dim3(gn), dim3(kBlock), 0, s, n, lv.l2u, zl, zu, st);
-  for (int l = 0; l < lv.nu(); ++l) {
-    const int p0 = lv.uptr[l], nr = lv.uptr[l + 1] - p0;
-    if (nr == 0) continue;
-    const int b = level_block(nr);
-    hipLaunchKernelGGL((k_ilu_sweep_ell<T, true>), dim3(grid_for(nr, b)), dim3(b), 0, s, lv.uell.len + p0,
-                       lv.uell.col, uval, dval + p0, lv.uell.off[l], p0, nr, width(lv.uell, l, nr), zu, st);
-  }
+  ilu_sweep<T>(lv.lower, static_cast<const T*>(w->ilu_lcoef), static_cast<const T*>(nullptr), zl, st, s);
+  hipLaunchKernelGGL((k_scatter<T, 1>), dim3(gn), dim3(kBlock), 0, s, n, lv.l2u, zl + n, zu, st);
+  ilu_sweep<T>(lv.upper, static_cast<const T*>(w->ilu_ucoef), static_cast<const T*>(w->ilu_own), zu, st, s);
   if (dot)
-    hipLaunchKernelGGL((k_gather_at<T, 2, true>), dim3(gn), dim3(kBlock), 0, s, n, lv.upos, zu, z, st, r, dot);
+    hipLaunchKernelGGL((k_gather_at<T, 2, true>), dim3(gn), dim3(kBlock), 0, s, n, lv.upos, zu + n, z, st, r, dot);
   else
-    hipLaunchKernelGGL((k_gather_at<T, 2>), dim3(gn), dim3(kBlock), 0, s, n, lv.upos, zu, z, st, nullptr, nullptr);
+    hipLaunchKernelGGL((k_gather_at<T, 2>), dim3(gn), dim3(kBlock), 0, s, n, lv.upos, zu + n, z, st, nullptr, nullptr);
   S355_LAUNCH_CHECK();
 }
 
@@ -2578,46 +2663,6 @@ void jacobi_inverse(const CsrView<T>& A, T* inv, hipStream_t s) {
 template void jacobi_inverse<double>(const CsrView<double>&, double*, hipStream_t);
 template void jacobi_inverse<float>(const CsrView<float>&, float*, hipStream_t);
 
-void ilu_ell(int n, const int* rowptr, const int* col, const int* diag, const std::vector<int>& rows,
-             const std::vector<int>& ptr, const std::vector<int>& pos, bool upper, std::vector<long>& off,
-             std::vector<int>& ecol, std::vector<int>& esrc, std::vector<int>& len, std::vector<int>& dsrc) {
-  const int nlev = static_cast<int>(ptr.size()) - 1;
-  auto first = [&](int i) { return upper ? diag[i] + 1 : rowptr[i]; };
-  auto last = [&](int i) { return upper ? rowptr[i + 1] : diag[i]; };
-  off.assign(nlev + 1, 0);
-  len.assign(n, 0);
-  if (upper) dsrc.assign(n, 0);
-  for (int l = 0; l < nlev; ++l) {
-    int w = 0;
-    for (int k = ptr[l]; k < ptr[l + 1]; ++k) {
-      const int i = rows[k];
-      len[k] = last(i) - first(i);
-      w = std::max(w, len[k]);
-      if (upper) dsrc[k] = diag[i];
-    }
-    off[l + 1] = off[l] + static_cast<long>(w) * (ptr[l + 1] - ptr[l]);
-  }
-  if (off[nlev] > 0x7fffffffL) throw std::invalid_argument("ILU level-ELL copy above 32-bit indices");
-  ecol.assign(off[nlev], 0);
-  esrc.assign(off[nlev], -1);
-  for (int l = 0; l < nlev; ++l) {
-    const int nr = ptr[l + 1] - ptr[l];
-    for (int k = 0; k < nr; ++k) {
-      const int i = rows[ptr[l] + k];
-      const int w = static_cast<int>((off[l + 1] - off[l]) / std::max(nr, 1));
-      for (int j = 0; j < w; ++j) {
-        const size_t q = static_cast<size_t>(off[l]) + static_cast<size_t>(j) * nr + k;
-        if (j < len[ptr[l] + k]) {
-          ecol[q] = pos[col[first(i) + j]];
-          esrc[q] = first(i) + j;
-        } else {
-          ecol[q] = pos[i];
-        }
-      }
-    }
-  }
-}
-
 void ilu_steps(int n, const int* rowptr, const int* col, const int* diag, const std::vector<int>& rows,
                std::vector<int>& ptr, std::vector<int>& p, std::vector<int>& d, std::vector<int>& u,
                std::vector<int>& r, std::vector<int>& q) {
@@ -2657,8 +2702,8 @@ void ilu_steps(int n, const int* rowptr, const int* col, const int* diag, const 
   }
 }
 
-void ilu_levels(int n, const int* rowptr, const int* col, const int* diag, std::vector<int>& lrows,
-                std::vector<int>& lptr, std::vector<int>& urows, std::vector<int>& uptr) {
+void ilu_levels(int n, const int* rowptr, const int* col, const int* diag, std::vector<int>& rows,
+                std::vector<int>& ptr) {
   std::vector<int> lev(n, 0);
   int nl = 0;
   for (int i = 0; i < n; ++i) {
@@ -2667,30 +2712,12 @@ void ilu_levels(int n, const int* rowptr, const int* col, const int* diag, std::
     lev[i] = l;
     nl = std::max(nl, l + 1);
   }
-  // rows by level; inside a level in the order they come in `order`
-  auto group = [&](int nlev, const int* order, std::vector<int>& rows, std::vector<int>& ptr) {
-    ptr.assign(nlev + 1, 0);
-    for (int i = 0; i < n; ++i) ptr[lev[i] + 1]++;
-    for (int l = 0; l < nlev; ++l) ptr[l + 1] += ptr[l];
-    rows.assign(n, 0);
-    std::vector<int> pos(ptr.begin(), ptr.end() - 1);
-    for (int k = 0; k < n; ++k) {
-      const int i = order ? order[k] : k;
-      rows[pos[lev[i]]++] = i;
-    }
-  };
-  group(nl, nullptr, lrows, lptr);  // natural order inside a lower level
-  int nu = 0;
-  for (int i = n - 1; i >= 0; --i) {
-    int l = 0;
-    for (int p = diag[i] + 1; p < rowptr[i + 1]; ++p) l = std::max(l, lev[col[p]] + 1);
-    lev[i] = l;
-    nu = std::max(nu, l + 1);
-  }
-  // lower-level order inside an upper level: the rows of a run of one lower
-  // level that share an upper level stay consecutive in it, which keeps the
-  // move of the lower sweep's result into the upper order local
-  group(nu, lrows.data(), urows, uptr);
+  ptr.assign(nl + 1, 0);
+  for (int i = 0; i < n; ++i) ptr[lev[i] + 1]++;
+  for (int l = 0; l < nl; ++l) ptr[l + 1] += ptr[l];
+  rows.assign(n, 0);
+  std::vector<int> pos(ptr.begin(), ptr.end() - 1);
+  for (int i = 0; i < n; ++i) rows[pos[lev[i]]++] = i;
 }
 
 }  // namespace s355

@@ -15,6 +15,7 @@
 
 #include "../../../include/simple355.h"
 #include "common.hpp"
+#include "ilu_plan.hpp"
 
 namespace s355 {
 
@@ -119,33 +120,28 @@ void fill_ordered(int n, const int* rowptr, const int* src, const int* row_nat, 
 template <class T, class S>
 void sell_fill(const int* src, size_t nslots, const S* csr_val, T* out, hipStream_t s);
 
-// Level schedule of the CSR pattern for ILU(0) (natural ordering): rows of a
-// level depend only on rows of earlier levels.  Lower levels order the
-// forward sweep and the factorisation, upper levels the backward sweep.
-//
-// The sweeps read the factors from level-ELL copies: the strictly lower
-// (upper) entries of the rows of one level are stored column-major, entry j
-// of the level's k-th row at off[l] + j * nrows_l + k, so that a wave's loads
-// of values and column ids are contiguous; len gives each row's count (rows
-// keep their CSR entry order, so the sums equal those of a CSR row walk).
-//
-// Each sweep runs in place in level space: the row at position p of the
-// sweep's level lists finds its input and stores its value at p, and the ELL
-// column ids are such positions.  A level's loads and stores are then one
-// contiguous run, and its gathers land in the runs of earlier levels instead
-// of all over the vector.  One gather pass over the whole vector moves r
-// into the lower order, one moves the lower result into the upper order and
-// one moves z back into the natural order.
-struct IluEll {
-  std::vector<long> off;        // host: nlev + 1 slot offsets
-  const int* col = nullptr;     // device: level-space position of each slot's column
-  const int* src = nullptr;     // device: CSR position of each slot (-1 padding)
-  const int* len = nullptr;     // device: entries of each row, by position in the level lists
-  const int* dsrc = nullptr;    // device (upper only): CSR position of each row's diagonal
+// The ILU(0) preconditioner (natural ordering).  The factorisation takes
+// the rows level by level (rows of a level depend only on rows of earlier
+// levels); the sweeps take them by the groups of ilu_plan.hpp, each sweep on a
+// buffer of its n inputs and n results in its own row order.  One pass over
+// the whole vector moves r into the lower order, one moves the lower
+// result into the upper order and one moves z back into the natural order.
+
+// one sweep's plan: what the launches need on the host, the rest on the device
+// (names as in IluPlan)
+struct IluSweep {
+  int n = 0;
+  std::vector<IluSub> subs;
+  std::vector<int> group, dptr;
   size_t slots = 0;
+  const int *len = nullptr, *slot0 = nullptr, *stride = nullptr, *col = nullptr, *src = nullptr;
+  const int *later = nullptr, *sptr = nullptr, *p = nullptr, *uptr = nullptr, *r = nullptr, *q = nullptr;
+  // upper sweep: CSR position of the pivot of the row at each position at
+  // depth 0, and -1 minus it below
+  const int* dsrc = nullptr;
 };
 
-// The elimination steps of ILU(0) per row, rows in lower-level order: row
+// The elimination steps of ILU(0) per row, rows by level: row
 // position t has steps ptr[t] .. ptr[t+1]-1; step s divides the lower entry
 // p[s] by the pivot d[s] (the diagonal of row col[p]) and then applies the
 // slot pairs u[s] .. u[s+1]-1: lu[r] -= l * lu[q].
@@ -159,16 +155,13 @@ struct IluSteps {
 };
 
 struct IluLevels {
-  std::vector<int> lptr, uptr;  // host: level boundaries into lrows / urows
-  const int* lrows = nullptr;   // device: rows grouped by lower level
-  const int* urows = nullptr;   // device: rows grouped by upper level
-  const int* lpos = nullptr;    // device: lower-level position of each row
-  const int* l2u = nullptr;     // device: upper-level position of the row at each lower position
-  const int* upos = nullptr;    // device: upper-level position of each row
-  IluEll lell, uell;
+  std::vector<int> lptr;        // host: level boundaries of the factorisation's rows
+  const int* lpos = nullptr;    // device: lower-sweep position of each row
+  const int* l2u = nullptr;     // device: upper-sweep position of the row at each lower position
+  const int* upos = nullptr;    // device: upper-sweep position of each row
+  IluSweep lower, upper;
   IluSteps steps;
   int nl() const { return static_cast<int>(lptr.size()) - 1; }
-  int nu() const { return static_cast<int>(uptr.size()) - 1; }
 };
 
 // Host construction of the elimination steps (rows in the order of rows).
@@ -176,16 +169,10 @@ void ilu_steps(int n, const int* rowptr, const int* col, const int* diag, const 
                std::vector<int>& ptr, std::vector<int>& p, std::vector<int>& d, std::vector<int>& u,
                std::vector<int>& r, std::vector<int>& q);
 
-// Host computation of the level schedule.
-void ilu_levels(int n, const int* rowptr, const int* col, const int* diag, std::vector<int>& lrows,
-                std::vector<int>& lptr, std::vector<int>& urows, std::vector<int>& uptr);
-
-// Host construction of one level-ELL copy (upper: the strictly upper part and
-// the diagonal positions; else the strictly lower part).  pos[i] is the
-// position of row i in rows, the space the column ids are given in.
-void ilu_ell(int n, const int* rowptr, const int* col, const int* diag, const std::vector<int>& rows,
-             const std::vector<int>& ptr, const std::vector<int>& pos, bool upper, std::vector<long>& off,
-             std::vector<int>& ecol, std::vector<int>& esrc, std::vector<int>& len, std::vector<int>& dsrc);
+// Host computation of the factorisation's levels: the rows by level, in their
+// natural order inside one.
+void ilu_levels(int n, const int* rowptr, const int* col, const int* diag, std::vector<int>& rows,
+                std::vector<int>& ptr);
 
 struct KResult {
   int iters = 0, reason = 0;
@@ -242,10 +229,10 @@ struct KWork {
   void* r = nullptr;        // n elements of T: preconditioner input (CG: r, z, p, w use V[0..3])
   void* pcinv = nullptr;    // n elements of T (Jacobi inverse diagonal)
   void* lu = nullptr;       // nnz elements of T (ILU(0) factors), when ilu is set
-  void* ilu_lval = nullptr; // level-ELL factor values of T: lower slots, upper slots, diagonal per row
-  void* ilu_uval = nullptr;
-  void* ilu_dval = nullptr;
-  void* ilu_zl = nullptr;   // n elements of T each: the lower and upper sweeps' z in level space
+  void* ilu_lcoef = nullptr;  // coefficients of T per slot of the lower and the upper sweep
+  void* ilu_ucoef = nullptr;
+  void* ilu_own = nullptr;    // n elements of T: 1 / pivot by upper-sweep position
+  void* ilu_zl = nullptr;   // 2 n elements of T each: inputs and results of the lower and the upper sweep
   void* ilu_zu = nullptr;
   const IluLevels* ilu = nullptr;
   double* partial = nullptr;
