@@ -382,6 +382,7 @@ void Context::allocate_fields() {
   kwork_.pcinv = alloc<double>(Nc);
   kwork_.partial = partial_;
   kwork_.partial_len = partial_len_;
+  kwork_.norms = alloc<double>(2 * tiles1);
   kwork_.st = alloc<KState>(ncase);
   S355_HIP(hipHostMalloc(&host_pinned_, 4096 + 10 * sizeof(double) * ncase, hipHostMallocDefault));
   S355_HIP(hipHostMalloc(reinterpret_cast<void**>(&hdr_), sizeof(KHeader) * ncase, hipHostMallocDefault));
@@ -771,6 +772,7 @@ void Context::ensure_mixed() {
   kwork32_.pcinv = alloc<float>(Nc);
   kwork32_.partial = partial_;
   kwork32_.partial_len = partial_len_;
+  kwork32_.norms = kwork_.norms;
   kwork32_.st = kwork_.st;
   kwork32_.host = kwork_.host;
   kwork32_.ncase = kwork_.ncase;

@@ -1,11 +1,12 @@
 // Device GMRES(m) / CG for the SIMPLE solves (see krylov.hpp).
 //
-// One GMRES iteration is five launches: SpMV fused with the Jacobi apply,
-// a multi-dot against the basis, its fixed-order reduction, the Gram-Schmidt
-// update fused with the norm, and a one-block finalisation that updates the
-// Hessenberg column, applies the Givens rotations and runs the convergence
-// test.  Basis vectors are kept unnormalised (v_k = scale_k V_k); the scales
-// are folded into the coefficients, which saves a normalisation pass over N.
+// One GMRES iteration is four launches: SpMV fused with the Jacobi apply, a
+// multi-dot against the basis, the sums of its tiles together with the previous
+// step's finalisation (Hessenberg column, Givens rotations, convergence test),
+// and the Gram-Schmidt update fused with the norm; two on small systems (see
+// k_spmv_dots).  Basis vectors are kept unnormalised (v_k = scale_k V_k); the
+// scales are folded into the coefficients, which saves a normalisation pass
+// over N and lets a product start before its vector's norm is known.
 // Every kernel returns at once when the device state says the solve has
 // ended, so the host may launch iterations ahead and read the state back
 // only every few iterations.
@@ -28,11 +29,14 @@ constexpr int kConvergedRtol = 2, kConvergedAtol = 3, kDivergedNull = -2, kDiver
               kDivergedBreakdown = -5, kDivergedIndefinitePc = -8, kDivergedNanorinf = -9,
               kDivergedIndefiniteMat = -10;
 
-__device__ __forceinline__ int conv_check(const KState* st, double rnorm) {
+__device__ __forceinline__ int conv_check(double ttol, double abstol, double dtol, double rnorm0, double rnorm) {
   if (isnan(rnorm) || isinf(rnorm)) return kDivergedNanorinf;
-  if (rnorm <= st->ttol) return rnorm < st->abstol ? kConvergedAtol : kConvergedRtol;
-  if (rnorm >= st->dtol * st->rnorm0) return kDivergedDtol;
+  if (rnorm <= ttol) return rnorm < abstol ? kConvergedAtol : kConvergedRtol;
+  if (rnorm >= dtol * rnorm0) return kDivergedDtol;
   return 0;
+}
+__device__ __forceinline__ int conv_check(const KState* st, double rnorm) {
+  return conv_check(st->ttol, st->abstol, st->dtol, st->rnorm0, rnorm);
 }
 
 __device__ __forceinline__ double& Hm(KState* st, int ld, int r, int c) { return st->H[c * ld + r]; }
@@ -357,7 +361,8 @@ void ilu_apply(const CsrView<T>& A, const IluLevels& lv, const T* lu, const T* r
   S355_LAUNCH_CHECK();
 }
 
-// ---- y = scale * M^-1 A x
+// ---- y = M^-1 A x (of the unnormalised basis vector: its scale goes into the
+// coefficients, so a product does not wait for the norm's finalisation)
 // L consecutive lanes share a row (L = 4, 8 or 16, picked per matrix): their
 // loads of values and column ids are contiguous across the wavefront; a
 // shuffle tree in a fixed order sums the lanes.  With NT the matrix streams
@@ -408,8 +413,7 @@ __device__ __forceinline__ T row_dot(const CsrView<T>& A, const T* __restrict__ 
 
 template <class T, int L, bool NT>
 __global__ void __launch_bounds__(kBlock) k_spmv_pc(CsrView<T> A, Tiles t, const T* __restrict__ x,
-                                                    const T* __restrict__ inv, T* __restrict__ y, const KState* st,
-                                                    int it) {
+                                                    const T* __restrict__ inv, T* __restrict__ y, const KState* st) {
   const int g = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
   const int row = g / L, lane = g % L;
   // the lanes of one row share its case, so they leave together
@@ -419,7 +423,7 @@ __global__ void __launch_bounds__(kBlock) k_spmv_pc(CsrView<T> A, Tiles t, const
   if (lane == 0 && row < A.n) {
     double z = static_cast<double>(s);
     if (inv) z *= static_cast<double>(inv[row]);
-    y[row] = static_cast<T>(z * sc->scale[it]);
+    y[row] = static_cast<T>(z);
   }
 }
 
@@ -446,11 +450,11 @@ __device__ __forceinline__ int sell_col(const V& A, size_t q, int row) {
 }
 
 template <class T, bool NT, bool PC, int W, bool C16>
-__device__ __forceinline__ void sell_row(const SellView<T>& A, const Tiles& t, const T* __restrict__ x,
-                                         const T* __restrict__ inv, T* __restrict__ y, const KState* st, int it,
-                                         int sl, int pos, int qa, int q1, double scl_in = -1.0) {
+__device__ __forceinline__ T sell_row(const SellView<T>& A, const Tiles& t, const T* __restrict__ x,
+                                      const T* __restrict__ inv, const KState* st, int sl, int pos, int qa, int q1,
+                                      int& row) {
   constexpr int B = W > 0 ? W : kSellBatch;
-  const int row = A.row ? A.row[pos] : pos;
+  row = A.row ? A.row[pos] : pos;
   int q0 = qa + (pos & 63);
   T v[B], xv[B];
   int c[B];
@@ -464,17 +468,21 @@ __device__ __forceinline__ void sell_row(const SellView<T>& A, const Tiles& t, c
     int cs = A.scase[sl];
     if (cs < 0) cs = t.case_of(row);
     sc = st + cs;
-    if (sc->reason) return;
+    if (sc->reason) {
+      row = -1;
+      return T(0);
+    }
   }
 #pragma unroll
   for (int u = 0; u < B; ++u) {
     v[u] = ld_stream<T, NT>(A.val + q0 + 64 * u);
     c[u] = sell_col<NT, C16>(A, q0 + 64 * u, row);
   }
-  if (sc->reason) return;
+  if (sc->reason) {
+    row = -1;
+    return T(0);
+  }
   // used after the slots (PC: Jacobi, inv is set)
-  // the basis vector's scale: from the state, or given (positive)
-  const double scl = scl_in > 0.0 ? scl_in : sc->scale[it];
   T invr = T(1);
   if constexpr (PC) invr = inv[row];
   T acc = T(0);
@@ -501,37 +509,39 @@ __device__ __forceinline__ void sell_row(const SellView<T>& A, const Tiles& t, c
   }
   double z = static_cast<double>(acc);
   if constexpr (PC) z *= static_cast<double>(invr);
-  y[row] = static_cast<T>(z * scl);
+  return static_cast<T>(z);
 }
 
-// one row of slice sl by the slice's width (wave-uniform)
+// one row of slice sl by the slice's width (wave-uniform); row -1: its case
+// has finished, no value
 template <class T, bool NT, bool PC, bool C16>
-__device__ __forceinline__ void sell_row_any(const SellView<T>& A, const Tiles& t, const T* __restrict__ x,
-                                             const T* __restrict__ inv, T* __restrict__ y, const KState* st, int it,
-                                             int sl, int pos, int qa, int q1, double scl = -1.0) {
+__device__ __forceinline__ T sell_row_any(const SellView<T>& A, const Tiles& t, const T* __restrict__ x,
+                                          const T* __restrict__ inv, const KState* st, int sl, int pos, int qa, int q1,
+                                          int& row) {
   switch ((q1 - qa) >> 6) {
-    case 1: sell_row<T, NT, PC, 1, C16>(A, t, x, inv, y, st, it, sl, pos, qa, q1, scl); break;
-    case 2: sell_row<T, NT, PC, 2, C16>(A, t, x, inv, y, st, it, sl, pos, qa, q1, scl); break;
-    case 3: sell_row<T, NT, PC, 3, C16>(A, t, x, inv, y, st, it, sl, pos, qa, q1, scl); break;
-    case 4: sell_row<T, NT, PC, 4, C16>(A, t, x, inv, y, st, it, sl, pos, qa, q1, scl); break;
-    case 5: sell_row<T, NT, PC, 5, C16>(A, t, x, inv, y, st, it, sl, pos, qa, q1, scl); break;
-    case 6: sell_row<T, NT, PC, 6, C16>(A, t, x, inv, y, st, it, sl, pos, qa, q1, scl); break;
-    case 7: sell_row<T, NT, PC, 7, C16>(A, t, x, inv, y, st, it, sl, pos, qa, q1, scl); break;
-    case 8: sell_row<T, NT, PC, 8, C16>(A, t, x, inv, y, st, it, sl, pos, qa, q1, scl); break;
-    default: sell_row<T, NT, PC, 0, C16>(A, t, x, inv, y, st, it, sl, pos, qa, q1, scl); break;
+    case 1: return sell_row<T, NT, PC, 1, C16>(A, t, x, inv, st, sl, pos, qa, q1, row);
+    case 2: return sell_row<T, NT, PC, 2, C16>(A, t, x, inv, st, sl, pos, qa, q1, row);
+    case 3: return sell_row<T, NT, PC, 3, C16>(A, t, x, inv, st, sl, pos, qa, q1, row);
+    case 4: return sell_row<T, NT, PC, 4, C16>(A, t, x, inv, st, sl, pos, qa, q1, row);
+    case 5: return sell_row<T, NT, PC, 5, C16>(A, t, x, inv, st, sl, pos, qa, q1, row);
+    case 6: return sell_row<T, NT, PC, 6, C16>(A, t, x, inv, st, sl, pos, qa, q1, row);
+    case 7: return sell_row<T, NT, PC, 7, C16>(A, t, x, inv, st, sl, pos, qa, q1, row);
+    case 8: return sell_row<T, NT, PC, 8, C16>(A, t, x, inv, st, sl, pos, qa, q1, row);
+    default: return sell_row<T, NT, PC, 0, C16>(A, t, x, inv, st, sl, pos, qa, q1, row);
   }
 }
 
 template <class T, bool NT, bool PC, bool C16 = false>
 __global__ void __launch_bounds__(kBlock) k_spmv_sell(SellView<T> A, Tiles t, const T* __restrict__ x,
-                                                      const T* __restrict__ inv, T* __restrict__ y, const KState* st,
-                                                      int it) {
+                                                      const T* __restrict__ inv, T* __restrict__ y, const KState* st) {
   const int pos = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
   if (pos >= A.n) return;
   // a wave is one slice (64 consecutive positions), so the slice index and
   // width are wave-uniform and the slice bounds load through the scalar cache
   const int sl = __builtin_amdgcn_readfirstlane(pos >> 6);
-  sell_row_any<T, NT, PC, C16>(A, t, x, inv, y, st, it, sl, pos, A.ptr[sl], A.ptr[sl + 1]);
+  int row;
+  const T z = sell_row_any<T, NT, PC, C16>(A, t, x, inv, st, sl, pos, A.ptr[sl], A.ptr[sl + 1], row);
+  if (row >= 0) y[row] = z;
 }
 
 // Two adjacent slices per wave, one row of each per lane (one case, FP32 on
@@ -541,7 +551,7 @@ __global__ void __launch_bounds__(kBlock) k_spmv_sell(SellView<T> A, Tiles t, co
 // never added (adjacent slices of a sorted window rarely differ in width).
 template <class T, bool NT, bool PC, int W, bool C16>
 __device__ __forceinline__ void sell_rows2(const SellView<T>& A, const T* __restrict__ x, const T* __restrict__ inv,
-                                           T* __restrict__ y, const KState* st, int it, int sl, int lane, int qa0,
+                                           T* __restrict__ y, const KState* st, int sl, int lane, int qa0,
                                            int qa1, int q11) {
   const int w0 = (qa1 - qa0) >> 6, w1 = (q11 - qa1) >> 6;
   const int pos0 = sl * 64 + lane, pos1 = pos0 + 64;
@@ -560,7 +570,6 @@ __device__ __forceinline__ void sell_rows2(const SellView<T>& A, const T* __rest
     c1[u] = sell_col<NT, C16>(A, qb, row1);
   }
   if (st->reason) return;
-  const double scl = st->scale[it];
   T i0 = T(1), i1 = T(1);
   if constexpr (PC) {
     i0 = inv[row0];
@@ -582,14 +591,14 @@ __device__ __forceinline__ void sell_rows2(const SellView<T>& A, const T* __rest
     z0 *= static_cast<double>(i0);
     z1 *= static_cast<double>(i1);
   }
-  y[row0] = static_cast<T>(z0 * scl);
-  if (ok1) y[row1] = static_cast<T>(z1 * scl);
+  y[row0] = static_cast<T>(z0);
+  if (ok1) y[row1] = static_cast<T>(z1);
 }
 
 template <class T, bool NT, bool PC, bool C16 = false>
 __global__ void __launch_bounds__(kBlock) k_spmv_sell2(SellView<T> A, Tiles t, const T* __restrict__ x,
-                                                       const T* __restrict__ inv, T* __restrict__ y, const KState* st,
-                                                       int it) {
+                                                       const T* __restrict__ inv, T* __restrict__ y,
+                                                       const KState* st) {
   // wave w takes slices 2w and 2w + 1
   const int wv = xcd_block(blockIdx.x, gridDim.x) * (kBlock / kWave) + static_cast<int>(threadIdx.x) / kWave;
   const int sl = __builtin_amdgcn_readfirstlane(2 * wv), lane = threadIdx.x & (kWave - 1);
@@ -598,26 +607,34 @@ __global__ void __launch_bounds__(kBlock) k_spmv_sell2(SellView<T> A, Tiles t, c
   if (sl + 1 >= nsl) {
     // an odd last slice: the one-slice body
     const int pos = sl * 64 + lane;
-    if (pos < A.n) sell_row_any<T, NT, PC, C16>(A, t, x, inv, y, st, it, sl, pos, A.ptr[sl], A.ptr[sl + 1]);
+    if (pos < A.n) {
+      int row;
+      const T z = sell_row_any<T, NT, PC, C16>(A, t, x, inv, st, sl, pos, A.ptr[sl], A.ptr[sl + 1], row);
+      if (row >= 0) y[row] = z;
+    }
     return;
   }
   const int qa0 = A.ptr[sl], qa1 = A.ptr[sl + 1], q11 = A.ptr[sl + 2];
   const int wmax = max((qa1 - qa0) >> 6, (q11 - qa1) >> 6);
   switch (wmax) {
-    case 1: sell_rows2<T, NT, PC, 1, C16>(A, x, inv, y, st, it, sl, lane, qa0, qa1, q11); break;
-    case 2: sell_rows2<T, NT, PC, 2, C16>(A, x, inv, y, st, it, sl, lane, qa0, qa1, q11); break;
-    case 3: sell_rows2<T, NT, PC, 3, C16>(A, x, inv, y, st, it, sl, lane, qa0, qa1, q11); break;
-    case 4: sell_rows2<T, NT, PC, 4, C16>(A, x, inv, y, st, it, sl, lane, qa0, qa1, q11); break;
-    case 5: sell_rows2<T, NT, PC, 5, C16>(A, x, inv, y, st, it, sl, lane, qa0, qa1, q11); break;
-    case 6: sell_rows2<T, NT, PC, 6, C16>(A, x, inv, y, st, it, sl, lane, qa0, qa1, q11); break;
-    case 7: sell_rows2<T, NT, PC, 7, C16>(A, x, inv, y, st, it, sl, lane, qa0, qa1, q11); break;
-    case 8: sell_rows2<T, NT, PC, 8, C16>(A, x, inv, y, st, it, sl, lane, qa0, qa1, q11); break;
+    case 1: sell_rows2<T, NT, PC, 1, C16>(A, x, inv, y, st, sl, lane, qa0, qa1, q11); break;
+    case 2: sell_rows2<T, NT, PC, 2, C16>(A, x, inv, y, st, sl, lane, qa0, qa1, q11); break;
+    case 3: sell_rows2<T, NT, PC, 3, C16>(A, x, inv, y, st, sl, lane, qa0, qa1, q11); break;
+    case 4: sell_rows2<T, NT, PC, 4, C16>(A, x, inv, y, st, sl, lane, qa0, qa1, q11); break;
+    case 5: sell_rows2<T, NT, PC, 5, C16>(A, x, inv, y, st, sl, lane, qa0, qa1, q11); break;
+    case 6: sell_rows2<T, NT, PC, 6, C16>(A, x, inv, y, st, sl, lane, qa0, qa1, q11); break;
+    case 7: sell_rows2<T, NT, PC, 7, C16>(A, x, inv, y, st, sl, lane, qa0, qa1, q11); break;
+    case 8: sell_rows2<T, NT, PC, 8, C16>(A, x, inv, y, st, sl, lane, qa0, qa1, q11); break;
     default: {
       // a slice wider than one batch: each slice with the one-slice body
       // for its own width
       for (int k = 0; k < 2; ++k) {
         const int s2 = sl + k, pos = s2 * 64 + lane;
-        if (pos < A.n) sell_row_any<T, NT, PC, C16>(A, t, x, inv, y, st, it, s2, pos, A.ptr[s2], A.ptr[s2 + 1]);
+        if (pos < A.n) {
+          int row;
+          const T z = sell_row_any<T, NT, PC, C16>(A, t, x, inv, st, s2, pos, A.ptr[s2], A.ptr[s2 + 1], row);
+          if (row >= 0) y[row] = z;
+        }
       }
       break;
     }
@@ -643,70 +660,69 @@ inline int spmv_variant(int lanes, int nt, int sell_v) {
 
 template <class T, int L>
 void launch_spmv_l(bool nt, const CsrView<T>& A, const Tiles& t, const T* x, const T* inv, T* y, const KState* st,
-                   int it, hipStream_t s) {
+                   hipStream_t s) {
   const int g = grid_for(static_cast<long>(A.n) * L);
   if (nt)
-    hipLaunchKernelGGL((k_spmv_pc<T, L, true>), dim3(g), dim3(kBlock), 0, s, A, t, x, inv, y, st, it);
+    hipLaunchKernelGGL((k_spmv_pc<T, L, true>), dim3(g), dim3(kBlock), 0, s, A, t, x, inv, y, st);
   else
-    hipLaunchKernelGGL((k_spmv_pc<T, L, false>), dim3(g), dim3(kBlock), 0, s, A, t, x, inv, y, st, it);
+    hipLaunchKernelGGL((k_spmv_pc<T, L, false>), dim3(g), dim3(kBlock), 0, s, A, t, x, inv, y, st);
 }
 
 // the SELL-64 product: two slices per wave when the view says so (FP32, one
 // case), else one
 template <class T, bool NT, bool PC, bool C16>
-void launch_sell(const SellView<T>& sell, const Tiles& t, const T* x, const T* inv, T* y, const KState* st, int it,
-                 hipStream_t s) {
+void launch_sell(const SellView<T>& sell, const Tiles& t, const T* x, const T* inv, T* y, const KState* st, hipStream_t s) {
   if constexpr (std::is_same<T, float>::value) {
     if (sell.two) {
       // two slices per wave: kBlock / kWave waves per block
       const int nsl = (sell.n + 63) / 64;
       const int g2 = grid_for((nsl + 1) / 2, kBlock / kWave);
-      hipLaunchKernelGGL((k_spmv_sell2<T, NT, PC, C16>), dim3(g2), dim3(kBlock), 0, s, sell, t, x, inv, y, st, it);
+      hipLaunchKernelGGL((k_spmv_sell2<T, NT, PC, C16>), dim3(g2), dim3(kBlock), 0, s, sell, t, x, inv, y, st);
       return;
     }
   }
   hipLaunchKernelGGL((k_spmv_sell<T, NT, PC, C16>), dim3(grid_for(sell.n)), dim3(kBlock), 0, s, sell, t, x, inv, y,
-                     st, it);
+                     st);
 }
 
 template <class T, bool NT, bool PC>
-void launch_sell_c(const SellView<T>& sell, const Tiles& t, const T* x, const T* inv, T* y, const KState* st, int it,
+void launch_sell_c(const SellView<T>& sell, const Tiles& t, const T* x, const T* inv, T* y, const KState* st,
                    hipStream_t s) {
   if (sell.col16) {
     // 16-bit column offsets exist for the FP32 inner order only
     if constexpr (std::is_same<T, float>::value)
-      launch_sell<T, NT, PC, true>(sell, t, x, inv, y, st, it, s);
+      launch_sell<T, NT, PC, true>(sell, t, x, inv, y, st, s);
     else
       throw std::logic_error("16-bit SELL columns in an FP64 product");
   } else {
-    launch_sell<T, NT, PC, false>(sell, t, x, inv, y, st, it, s);
+    launch_sell<T, NT, PC, false>(sell, t, x, inv, y, st, s);
   }
 }
 
-// y = scale M^-1 A x with the CSR kernel at L lanes per row, or with the
+// y = M^-1 A x with the CSR kernel at L lanes per row, or with the
 // SELL-64 copy for L = 0 (sell must then be set)
 template <class T>
 void launch_spmv(int L, int nt, const CsrView<T>& A, const SellView<T>& sell, const Tiles& t, const T* x, const T* inv,
-                 T* y, const KState* st, int it, hipStream_t s) {
+                 T* y, const KState* st, hipStream_t s) {
   switch (L) {
     case 0: {
       if (!sell.ptr) throw std::logic_error("SELL-64 SpMV without a SELL copy");
       if (sell.n != A.n) throw std::logic_error("SELL-64 copy of another size");
       if (nt && inv)
-        launch_sell_c<T, true, true>(sell, t, x, inv, y, st, it, s);
+        launch_sell_c<T, true, true>(sell, t, x, inv, y, st, s);
       else if (nt)
-        launch_sell_c<T, true, false>(sell, t, x, inv, y, st, it, s);
+        launch_sell_c<T, true, false>(sell, t, x, inv, y, st, s);
       else if (inv)
-        launch_sell_c<T, false, true>(sell, t, x, inv, y, st, it, s);
+        launch_sell_c<T, false, true>(sell, t, x, inv, y, st, s);
       else
-        launch_sell_c<T, false, false>(sell, t, x, inv, y, st, it, s);
+        launch_sell_c<T, false, false>(sell, t, x, inv, y, st, s);
       break;
     }
-    case 1: launch_spmv_l<T, 1>(nt != 0, A, t, x, inv, y, st, it, s); break;
-    case 2: launch_spmv_l<T, 2>(nt != 0, A, t, x, inv, y, st, it, s); break;
-    case 4: launch_spmv_l<T, 4>(nt != 0, A, t, x, inv, y, st, it, s); break;
-    case 16: launch_spmv_l<T, 16>(nt != 0, A, t, x, inv, y, st, it, s); break;
-    default: launch_spmv_l<T, 8>(nt != 0, A, t, x, inv, y, st, it, s); break;
+    case 1: launch_spmv_l<T, 1>(nt != 0, A, t, x, inv, y, st, s); break;
+    case 2: launch_spmv_l<T, 2>(nt != 0, A, t, x, inv, y, st, s); break;
+    case 4: launch_spmv_l<T, 4>(nt != 0, A, t, x, inv, y, st, s); break;
+    case 16: launch_spmv_l<T, 16>(nt != 0, A, t, x, inv, y, st, s); break;
+    default: launch_spmv_l<T, 8>(nt != 0, A, t, x, inv, y, st, s); break;
   }
 }
 
@@ -722,6 +738,7 @@ SellView<T> sell_of(const KWork& w, int n, int variant = -1) {
     v.col16 = w.sell[sv].col16;
     v.val = static_cast<const T*>(w.sell_vals[sv]);
     v.scase = w.sell[sv].scase;
+    v.tiled = !v.row || kSellSigma[sv] <= kBlock;
     v.two = std::is_same<T, float>::value && !v.scase && (w.sell2 > 0 || (w.sell2 < 0 && n >= (1 << 20))) ? 1 : 0;
   }
   return v;
@@ -898,12 +915,18 @@ __device__ __forceinline__ void axpy_all(const T* __restrict__ V, size_t ld, int
 // for the last chunk's few vectors too.  The sums are the same either way.
 template <class T, int R, bool Batch>
 __global__ void __launch_bounds__(kBlock) k_mdot(const T* __restrict__ V, size_t ld, Tiles t, int it,
-                                                 double* __restrict__ partial, int pstride, const KState* st,
-                                                 int cpb) {
+                                                 double* __restrict__ partial, int pstride, KState* st, int cpb) {
   using S = GsShape<T, R>;
   int a, e, c;
   t.range(blockIdx.x, a, e, c);
-  if (st[c].reason) return;
+  const int reason = st[c].reason;
+  if (threadIdx.x == 0 && blockIdx.y == 0) {
+    // for the next launch, which may change reason while it runs
+    int t0, t1;
+    t.tiles_of(c, t0, t1);
+    if (static_cast<int>(blockIdx.x) == t0) st[c].ended = reason;
+  }
+  if (reason) return;
   // each wave's sum of every k of the block, reduced over the waves once
   __shared__ double lds[kBlock / kWave][8 * ((kMaxRestart + 8) / 8)];
   const size_t end = static_cast<size_t>(e);
@@ -989,23 +1012,7 @@ __device__ __forceinline__ void strided_sum2(const double* __restrict__ p, int n
   }
 }
 
-// ---- hcol[k] = scale_k * sum over the case's tiles of partial[k][b]
-// (block (k, case))
-__global__ void __launch_bounds__(kBlock) k_mdot_final(const double* partial, Tiles t, int pstride, KState* st) {
-  KState* s = st + blockIdx.y;
-  if (s->reason) return;
-  __shared__ double lds[kBlock / kWave];
-  const int k = blockIdx.x;
-  int t0, t1;
-  t.tiles_of(blockIdx.y, t0, t1);
-  double v = 0.0;
-  const double* pk = partial + static_cast<size_t>(k) * t.ntile;  // column k: contiguous over tiles
-  v = strided_sum(pk, t0, t1);
-  v = block_sum(v, lds);
-  if (threadIdx.x == 0) s->hcol[k] = v * s->scale[k];
-}
-
-// ---- w -= sum_k hcol_k scale_k V_k ; partial ||w||^2 per tile.  With Batch
+// ---- w = scale_it w - sum_k hcol_k scale_k V_k ; ||w||^2 per tile into norms.  With Batch
 // (grids too small to hide memory latency with many waves) each thread
 // issues the loads of up to 8 basis vectors before it uses any; otherwise it
 // streams them one after the other and the resident waves hide the latency
@@ -1013,7 +1020,7 @@ __global__ void __launch_bounds__(kBlock) k_mdot_final(const double* partial, Ti
 // order either way.
 template <class T, int R, bool Batch>
 __global__ void __launch_bounds__(kBlock) k_maxpy_norm(T* __restrict__ V, size_t ld, Tiles t, int it,
-                                                       double* __restrict__ partial, const KState* st) {
+                                                       double* __restrict__ norms, const KState* st) {
   using S = GsShape<T, R>;
   int a, e, c;
   t.range(blockIdx.x, a, e, c);
@@ -1021,7 +1028,8 @@ __global__ void __launch_bounds__(kBlock) k_maxpy_norm(T* __restrict__ V, size_t
   if (sc->reason) return;
   __shared__ double cf[kMaxRestart + 1];
   __shared__ double lds[kBlock / kWave];
-  for (int k = threadIdx.x; k <= it; k += kBlock) cf[k] = sc->hcol[k] * sc->scale[k];
+  for (int k = threadIdx.x; k <= it; k += kBlock) cf[k] = sc->hcol[it & 1][k] * sc->scale[k];
+  const double sw = sc->scale[it];
   __syncthreads();
   const size_t end = static_cast<size_t>(e);
   const bool vec = S::vec_ok(a, ld);
@@ -1033,6 +1041,8 @@ __global__ void __launch_bounds__(kBlock) k_maxpy_norm(T* __restrict__ V, size_t
     const size_t i0 = S::row0(a, q);
     double sacc[S::VW];
     load_chunk<T, S::VW>(w, i0, end, vec, sacc);
+#pragma unroll
+    for (int u = 0; u < S::VW; ++u) sacc[u] *= sw;
     if (whole) {
       axpy_all<T, S::VW, true>(V, ld, it + 1, i0, cf, sacc);
     } else {
@@ -1052,157 +1062,348 @@ __global__ void __launch_bounds__(kBlock) k_maxpy_norm(T* __restrict__ V, size_t
     store_chunk<T, S::VW>(w, i0, end, vec, out);
   }
   nrm = block_sum(nrm, lds);
-  if (threadIdx.x == 0) partial[blockIdx.x] = nrm;
+  if (threadIdx.x == 0) norms[blockIdx.x] = nrm;
 }
 
 // ---- Hessenberg column, Givens rotations, convergence test of step it of
-// one case, by one block.  The column and the previous rotations are staged
-// in LDS, so the serial rotation sweep of thread 0 runs out of LDS rather
-// than global memory.  Staging: every thread, before a barrier that
-// publishes col/cc/ss.
-__device__ __forceinline__ void arnoldi_stage(const KState* s_, int it, double* col, double* cc, double* ss) {
-  for (int j = threadIdx.x; j <= it; j += kBlock) {
-    col[j] = s_->hcol[j];
-    cc[j] = s_->cc[j];
-    ss[j] = s_->ss[j];
-  }
-}
+// one case, by one block, from the norms of its tiles.  The column and the
+// previous rotations are staged in LDS and the scalars that thread 0 needs load
+// with them, so its serial rotation sweep waits for no global load.
+struct ArnoldiScalars {
+  double g_it, rnorm, ttol, abstol, dtol, rnorm0;
+  int its, maxit;
+};
 
 // The rest, once staged and published: s (thread 0) is the squared norm of
 // the new basis vector.  Every thread of the block calls it.
-__device__ void arnoldi_close(double s, int it, int m, KState* s_, double* col, double* cc, double* ss) {
+__device__ void arnoldi_close(double s, int it, int m, KState* s_, const ArnoldiScalars& q, double* col, double* cc,
+                              double* ss) {
   const int ld = m + 1;
   if (threadIdx.x == 0) {
     const double tt = sqrt(s);
     col[it + 1] = tt;
     s_->scale[it + 1] = tt != 0.0 ? 1.0 / tt : 1.0;
-    const double g_it = s_->grs[it];
-    double hapbnd = fabs(tt / g_it);
+    double hapbnd = fabs(tt / q.g_it);
     if (hapbnd > 1.e-30) hapbnd = 1.e-30;
     const bool hapend = tt < hapbnd;
+    double carry = col[0];  // col[j] as the rotations before j left it
+    double c1 = cc[0], s1 = ss[0], h1 = it > 0 ? col[1] : 0.0;
     for (int j = 1; j <= it; ++j) {
-      const double t0v = col[j - 1];
-      col[j - 1] = cc[j - 1] * t0v + ss[j - 1] * col[j];
-      col[j] = cc[j - 1] * col[j] - ss[j - 1] * t0v;
+      // the next rotation's operands load while this one's products run
+      const int jn = j < it ? j : j - 1;
+      const double c2 = cc[jn], s2 = ss[jn], h2 = col[jn + 1];
+      col[j - 1] = c1 * carry + s1 * h1;
+      carry = c1 * h1 - s1 * carry;
+      c1 = c2;
+      s1 = s2;
+      h1 = h2;
     }
     double res;
     int reason = 0;
     if (!hapend) {
-      const double hv = col[it], hn = col[it + 1];
+      const double hv = carry, hn = tt;
       const double tr = sqrt(hv * hv + hn * hn);
       if (tr == 0.0) {
         reason = kDivergedNull;
-        res = s_->rnorm;
+        res = q.rnorm;
+        col[it] = carry;
       } else {
         const double c = hv / tr, sn = hn / tr;
         s_->cc[it] = c;
         s_->ss[it] = sn;
-        s_->grs[it + 1] = -(sn * g_it);
-        s_->grs[it] = c * g_it;
+        const double g1 = -(sn * q.g_it);
+        s_->grs[it + 1] = g1;
+        s_->grs[it] = c * q.g_it;
         col[it] = c * hv + sn * hn;
-        res = fabs(s_->grs[it + 1]);
+        res = fabs(g1);
       }
     } else {
       res = 0.0;
+      col[it] = carry;
     }
     s_->it = it + 1;
-    s_->its += 1;
+    s_->its = q.its + 1;
     s_->rnorm = res;
     if (!reason) {
-      reason = conv_check(s_, res);
+      reason = conv_check(q.ttol, q.abstol, q.dtol, q.rnorm0, res);
       if (hapend && !reason) reason = kDivergedBreakdown;
     }
-    if (!reason && s_->its >= s_->maxit) reason = kDivergedIts;
+    if (!reason && q.its + 1 >= q.maxit) reason = kDivergedIts;
     s_->reason = reason;
   }
   __syncthreads();
   for (int j = threadIdx.x; j <= it + 1; j += kBlock) Hm(s_, ld, j, it) = col[j];
 }
 
-// one block per case, from the partial norms of the case's tiles
-__global__ void __launch_bounds__(kBlock) k_arnoldi_finalize(const double* partial, Tiles t, int it, int m,
-                                                             KState* st) {
-  KState* s_ = st + blockIdx.x;
-  if (s_->reason) return;
+// step it of one case from the norms of its tiles, by one block
+__device__ void arnoldi_finalize(const double* norms, const Tiles& t, int c, int it, int m, KState* s_) {
   __shared__ double lds[kBlock / kWave];
   __shared__ double col[kMaxRestart + 2], cc[kMaxRestart + 1], ss[kMaxRestart + 1];
   int t0, t1;
-  t.tiles_of(blockIdx.x, t0, t1);
-  double s = strided_sum(partial, t0, t1);
-  arnoldi_stage(s_, it, col, cc, ss);
+  t.tiles_of(c, t0, t1);
+  for (int j = threadIdx.x; j <= it; j += kBlock) {
+    col[j] = s_->hcol[it & 1][j];
+    cc[j] = s_->cc[j];
+    ss[j] = s_->ss[j];
+  }
+  const ArnoldiScalars q = {s_->grs[it], s_->rnorm,  s_->ttol, s_->abstol, s_->dtol,
+                            s_->rnorm0,  s_->its, s_->maxit};
+  double s = strided_sum(norms, t0, t1);
   s = block_sum(s, lds);  // contains the barrier that publishes col/cc/ss
-  arnoldi_close(s, it, m, s_, col, cc, ss);
+  arnoldi_close(s, it, m, s_, q, col, cc, ss);
 }
 
-// The SELL-64 product of step it > 0 of one case together with the
-// finalisation of step it - 1, which would otherwise be a launch of its own
-// between them (small systems, where launches, not bytes, set the time).
-// Every block sums the tile norms of basis vector it (step it - 1 made it),
-// in the finalisation's order, for that vector's scale; block 0 also
-// completes step it - 1.  The other blocks may read the state before or
-// after block 0 ends the solve there: the rows they then write belong to a
-// basis vector that is never used.  The tile norms stay valid until the next
-// kernel (the multi-dot of step it writes over them).
-template <class T, bool NT, bool PC, bool C16>
-__global__ void __launch_bounds__(kBlock) k_spmv_sell_fin(SellView<T> A, Tiles t, const T* __restrict__ x,
-                                                          const T* __restrict__ inv, T* __restrict__ y, KState* st,
-                                                          const double* partial, int it, int m) {
-  __shared__ double lds[kBlock / kWave];
-  __shared__ double col[kMaxRestart + 2], cc[kMaxRestart + 1], ss[kMaxRestart + 1];
-  __shared__ double scl;
-  // block 0 alone writes the state in this launch, after its first barrier,
-  // so its threads all read the same value here
-  const bool fin = blockIdx.x == 0 && !st->reason;
-  int t0, t1;
-  t.tiles_of(0, t0, t1);
-  double s = strided_sum(partial, t0, t1);
-  if (fin) arnoldi_stage(st, it - 1, col, cc, ss);
-  s = block_sum(s, lds);
-  if (threadIdx.x == 0) {
-    const double tt = sqrt(s);
-    scl = tt != 0.0 ? 1.0 / tt : 1.0;
+// ... as a launch of its own (one block per case): the last step of a cycle
+__global__ void __launch_bounds__(kBlock) k_arnoldi_finalize(const double* norms, Tiles t, int it, int m, KState* st) {
+  KState* s_ = st + blockIdx.x;
+  if (s_->reason) return;
+  arnoldi_finalize(norms, t, blockIdx.x, it, m, s_);
+}
+
+// ---- hcol[k] = scale_k scale_it * sum over the case's tiles of dots[k][b]
+// (block (k, case), k = 0..it), and with fin the finalisation of step it - 1
+// (block (it + 1, case)), which so costs no launch of its own: the product of
+// step it and its dots use the unscaled basis vector and do not wait for it.
+// The blocks form scale_it themselves from the tile norms (in the
+// finalisation's order, the same bits); hcol and the norms alternate between
+// two arrays by step, so the finalisation reads what nobody writes here, and
+// whether the solve had ended is read from the multi-dot's copy.  Where the
+// finalisation ends it now, the column is never used.  With the finalisation
+// as a launch between the update and the next product (4.8 us a step) the
+// pressure solves of the channel took 374.6 ms (2.53 M rows, FP32 cycles), 98.2
+// (748 K), 75.4 (546 K, FP64); beside the sums 361.6, 93.1, 71.0.
+__global__ void __launch_bounds__(kBlock) k_orth(const double* dots, const double* norms, Tiles t, int it, int m,
+                                                 int fin, KState* st) {
+  KState* s = st + blockIdx.y;
+  if (s->ended) return;
+  const int k = blockIdx.x;
+  if (k > it) {
+    arnoldi_finalize(norms, t, blockIdx.y, it - 1, m, s);
+    return;
   }
-  if (fin)
-    arnoldi_close(s, it - 1, m, st, col, cc, ss);
-  else
+  __shared__ double lds[kBlock / kWave], lds2[kBlock / kWave];
+  int t0, t1;
+  t.tiles_of(blockIdx.y, t0, t1);
+  double v = strided_sum(dots + static_cast<size_t>(k) * t.ntile, t0, t1);  // column k: contiguous over tiles
+  double n2 = fin ? strided_sum(norms, t0, t1) : 0.0;
+  v = block_sum(v, lds);
+  if (fin) n2 = block_sum(n2, lds2);
+  if (threadIdx.x == 0) {
+    double sw;
+    if (fin) {
+      const double tt = sqrt(n2);
+      sw = tt != 0.0 ? 1.0 / tt : 1.0;
+    } else {
+      sw = s->scale[it];
+    }
+    s->hcol[it & 1][k] = v * (k == it ? sw : s->scale[k]) * sw;
+  }
+}
+
+// ---- one case of at most kBlock tiles of kBlock rows, without ILU, on the
+// SELL-64 copy: an Arnoldi step in two launches.  Such a step moves a few MB
+// that the L2s hold, and a launch costs 1.6-2 us before its first load
+// returns, so what sets the time is the number of launches and the chain of
+// loads in each (32,768 rows, FP64, step 15 of 30: product 5.0 with the
+// finalisation, dots 3.8, sums 3.0, update 3.9 us as four launches; 4.5 and 5.9
+// as two, and four SIMPLE steps of the cavity 40.3 -> 29.9 ms).  Above kBlock
+// tiles every block's own sums of all tiles cost more than the launch.
+
+// The product w = M^-1 A V_it, and its dots with V_0..V_it: a block's rows are
+// one tile, so each thread still holds its w.  The first 8 basis vectors load
+// ahead of the product, each further 8 ahead of the sums before it.  With a
+// row map (64-row windows) the rows come back to their own threads through
+// LDS.  The sums are those of k_mdot with one row per thread, bit for bit.
+template <class T, bool NT, bool PC, bool C16>
+__global__ void __launch_bounds__(kBlock) k_spmv_dots(SellView<T> A, Tiles t, T* V, size_t ld,
+                                                      const T* __restrict__ inv, KState* st, int it,
+                                                      double* __restrict__ dots) {
+  const int reason = st->reason;  // (used once the first loads are on their way)
+  __shared__ T wrow[kBlock];
+  __shared__ double lds[kBlock / kWave][8 * ((kMaxRestart + 8) / 8)];
+  const int b = xcd_block(blockIdx.x, gridDim.x);
+  const int a = b * kBlock, pos = a + static_cast<int>(threadIdx.x);
+  const bool in = pos < A.n;
+  const T* vp = V + (in ? pos : A.n - 1);  // past the end: any element, times w = 0
+  T e[8];
+#pragma unroll
+  for (int u = 0; u < 8; ++u) e[u] = vp[static_cast<size_t>(min(u, it)) * ld];
+  T w = T(0);
+  if (in) {
+    const int sl = __builtin_amdgcn_readfirstlane(pos >> 6);
+    int row;  // -1 where the solve has ended
+    w = sell_row_any<T, NT, PC, C16>(A, t, V + static_cast<size_t>(it) * ld, inv, st, sl, pos, A.ptr[sl],
+                                     A.ptr[sl + 1], row);
+    if (A.row && row >= 0) wrow[row - a] = w;
+  }
+  // for the next launch, which may change reason while it runs
+  if (blockIdx.x == 0 && threadIdx.x == 0) st->ended = reason;
+  if (reason) return;
+  if (A.row) {
     __syncthreads();
-  const int pos = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
-  if (pos >= A.n) return;
-  const int sl = __builtin_amdgcn_readfirstlane(pos >> 6);
-  sell_row_any<T, NT, PC, C16>(A, t, x, inv, y, st, it, sl, pos, A.ptr[sl], A.ptr[sl + 1], scl);
+    w = in ? wrow[threadIdx.x] : T(0);
+  }
+  if (in) V[static_cast<size_t>(it + 1) * ld + pos] = w;
+  const double wd = static_cast<double>(w);
+  const int lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
+  for (int k0 = 0; k0 <= it; k0 += 8) {
+    T next[8];
+    const bool more = k0 + 8 <= it;
+    if (more) {
+#pragma unroll
+      for (int u = 0; u < 8; ++u) next[u] = vp[static_cast<size_t>(min(k0 + 8 + u, it)) * ld];
+    }
+    double acc[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) acc[u] = k0 + u <= it ? 0.0 + wd * static_cast<double>(e[u]) : 0.0;
+    const double sk = wave_sum8(acc);
+    if ((lane & 7) == 0) lds[wid][k0 + (lane >> 3)] = sk;
+    if (more) {
+#pragma unroll
+      for (int u = 0; u < 8; ++u) e[u] = next[u];
+    }
+  }
+  __syncthreads();
+  for (int j = threadIdx.x; j <= it; j += kBlock) {
+    double s = 0.0;
+#pragma unroll
+    for (int q = 0; q < kBlock / kWave; ++q) s += lds[q][j];
+    dots[static_cast<size_t>(j) * t.ntile + b] = s;
+  }
+}
+
+// wave sums (four 64-tile pieces of up to kBlock tiles each, in tile order) of
+// 8 columns of tile values, the columns' sums in lanes 8 k ..; the order is
+// that of strided_sum and block_sum
+__device__ __forceinline__ double tile_sums8(const double* p, int ntile, int k0, int kn) {
+  const int lane = threadIdx.x & (kWave - 1);
+  double x[4][8];
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int k = min(k0 + u, kn - 1), b = min(64 * c + lane, ntile - 1);
+      x[c][u] = 64 * c < ntile ? p[static_cast<size_t>(k) * ntile + b] : 0.0;
+    }
+  double s = 0.0;
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    if (64 * c >= ntile) break;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) x[c][u] = 64 * c + lane < ntile ? x[c][u] : 0.0;
+    s += wave_sum8(x[c]);
+  }
+  return s;
+}
+
+// the same for one column, its sum in every lane
+__device__ __forceinline__ double tile_sum(const double* p, int ntile) {
+  const int lane = threadIdx.x & (kWave - 1);
+  double x[8];
+#pragma unroll
+  for (int c = 0; c < 8; ++c) x[c] = c < 4 && 64 * c + lane < ntile ? p[min(64 * c + lane, ntile - 1)] : 0.0;
+  const double v = wave_sum8(x);
+  double s = 0.0;
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+    if (64 * c < ntile) s += __shfl(v, 8 * c, kWave);
+  return s;
+}
+
+// The rest of the step: every block sums the tiles' dots and norms itself (the
+// order and bits of k_orth), then updates its tile as k_maxpy_norm does.  The
+// block past the tiles finalises step it - 1 (fin).
+template <class T>
+__global__ void __launch_bounds__(kBlock) k_orth_update(T* V, size_t ld, Tiles t, const double* __restrict__ dots,
+                                                        const double* norms, double* norms_out, int it, int m, int fin,
+                                                        KState* st) {
+  const int ended = st->ended;  // (used once the first loads are on their way)
+  if (static_cast<int>(blockIdx.x) == t.ntile) {
+    if (!ended) arnoldi_finalize(norms, t, 0, it - 1, m, st);
+    return;
+  }
+  __shared__ double cf[kMaxRestart + 1 + 8];
+  __shared__ double lds[kBlock / kWave];
+  const int a = blockIdx.x * kBlock, row = a + static_cast<int>(threadIdx.x);
+  const bool in = row < t.n;
+  T* vp = V + (in ? row : t.n - 1);
+  T e[8];
+#pragma unroll
+  for (int u = 0; u < 8; ++u) e[u] = vp[static_cast<size_t>(min(u, it)) * ld];
+  const T wv = in ? vp[static_cast<size_t>(it + 1) * ld] : T(0);
+  const int lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
+  double sw;
+  if (fin) {
+    const double tt = sqrt(tile_sum(norms, t.ntile));
+    sw = tt != 0.0 ? 1.0 / tt : 1.0;
+  } else {
+    sw = st->scale[it];
+  }
+  for (int k0 = 8 * wid; k0 <= it; k0 += 8 * (kBlock / kWave)) {
+    const double v = tile_sums8(dots, t.ntile, k0, it + 1);
+    if (ended) return;
+    const int k = k0 + (lane >> 3);
+    if ((lane & 7) == 0 && k <= it) {
+      const double sk = k == it ? sw : st->scale[k];
+      const double h = v * sk * sw;
+      if (blockIdx.x == 0) st->hcol[it & 1][k] = h;
+      cf[k] = h * sk;
+    }
+  }
+  if (ended) return;
+  __syncthreads();
+  double acc = static_cast<double>(wv) * sw;
+  for (int k0 = 0; k0 <= it; k0 += 8) {
+    T next[8];
+    const bool more = k0 + 8 <= it;
+    if (more) {
+#pragma unroll
+      for (int u = 0; u < 8; ++u) next[u] = vp[static_cast<size_t>(min(k0 + 8 + u, it)) * ld];
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (k0 + u <= it) acc -= cf[k0 + u] * static_cast<double>(e[u]);
+    if (more) {
+#pragma unroll
+      for (int u = 0; u < 8; ++u) e[u] = next[u];
+    }
+  }
+  const T out = static_cast<T>(acc);
+  double nrm = in ? 0.0 + static_cast<double>(out) * static_cast<double>(out) : 0.0;
+  if (in) vp[static_cast<size_t>(it + 1) * ld] = out;
+  nrm = block_sum(nrm, lds);
+  if (threadIdx.x == 0) norms_out[blockIdx.x] = nrm;
 }
 
 template <class T, bool NT, bool PC>
-void launch_sell_fin_c(const SellView<T>& sell, const Tiles& t, const T* x, const T* inv, T* y, KState* st,
-                       const double* partial, int it, int m, hipStream_t s) {
-  const int g = grid_for(sell.n);
+void launch_spmv_dots_c(const SellView<T>& sell, const Tiles& t, T* V, size_t ld, const T* inv, KState* st,
+                        int it, double* dots, hipStream_t s) {
   if (sell.col16) {
     if constexpr (std::is_same<T, float>::value)
-      hipLaunchKernelGGL((k_spmv_sell_fin<T, NT, PC, true>), dim3(g), dim3(kBlock), 0, s, sell, t, x, inv, y, st,
-                         partial, it, m);
+      hipLaunchKernelGGL((k_spmv_dots<T, NT, PC, true>), dim3(t.ntile), dim3(kBlock), 0, s, sell, t, V, ld, inv, st,
+                         it, dots);
     else
       throw std::logic_error("16-bit SELL columns in an FP64 product");
   } else {
-    hipLaunchKernelGGL((k_spmv_sell_fin<T, NT, PC, false>), dim3(g), dim3(kBlock), 0, s, sell, t, x, inv, y, st,
-                       partial, it, m);
+    hipLaunchKernelGGL((k_spmv_dots<T, NT, PC, false>), dim3(t.ntile), dim3(kBlock), 0, s, sell, t, V, ld, inv, st,
+                       it, dots);
   }
 }
 
-// y = scale M^-1 A x on the one-slice SELL-64 copy with the finalisation of
-// step it - 1 (one case, no ILU)
+// V_it+1 = M^-1 A V_it on the one-slice SELL-64 copy and its dots (t: tiles of kBlock rows)
 template <class T>
-void launch_sell_fin(int nt, const SellView<T>& sell, const Tiles& t, const T* x, const T* inv, T* y, KState* st,
-                     const double* partial, int it, int m, hipStream_t s) {
-  if (!sell.ptr || sell.two || sell.scase) throw std::logic_error("fused SELL-64 product on another layout");
-  if (it < 1) throw std::logic_error("fused SELL-64 product without a previous step");
+void launch_spmv_dots(int nt, const SellView<T>& sell, const Tiles& t, T* V, size_t ld, const T* inv,
+                      KState* st, int it, double* dots, hipStream_t s) {
+  if (!sell.ptr || sell.two || sell.scase || !sell.tiled || t.tile != kBlock || t.ntile > kBlock || t.n != sell.n)
+    throw std::logic_error("product with dots on another layout");
   if (nt && inv)
-    launch_sell_fin_c<T, true, true>(sell, t, x, inv, y, st, partial, it, m, s);
+    launch_spmv_dots_c<T, true, true>(sell, t, V, ld, inv, st, it, dots, s);
   else if (nt)
-    launch_sell_fin_c<T, true, false>(sell, t, x, inv, y, st, partial, it, m, s);
+    launch_spmv_dots_c<T, true, false>(sell, t, V, ld, inv, st, it, dots, s);
   else if (inv)
-    launch_sell_fin_c<T, false, true>(sell, t, x, inv, y, st, partial, it, m, s);
+    launch_spmv_dots_c<T, false, true>(sell, t, V, ld, inv, st, it, dots, s);
   else
-    launch_sell_fin_c<T, false, false>(sell, t, x, inv, y, st, partial, it, m, s);
+    launch_spmv_dots_c<T, false, false>(sell, t, V, ld, inv, st, it, dots, s);
 }
 
 // ---- back substitution R y = g on the completed columns of each case, y_j
@@ -1432,6 +1633,7 @@ __global__ void k_init_states(KState* st, int ncase, int maxit, double rtol, dou
     s->reason = 0;
     s->maxit = maxit;
     s->done = 0;
+    s->ended = 0;
     s->cycles = 0;
     s->rnorm = s->rnorm0 = s->ttol = s->snorm = 0.0;
     s->rtol = rtol;
@@ -1622,7 +1824,7 @@ constexpr int kBatchTiles = 1024;
 template <class T>
 struct Dispatch {
   template <int R>
-  static void mdot_r(const T* V, size_t ld, const Tiles& t, int it, double* partial, int pstride, const KState* st,
+  static void mdot_r(const T* V, size_t ld, const Tiles& t, int it, double* partial, int pstride, KState* st,
                      hipStream_t s) {
     // below kMdotBlocks tiles, the chunks of 8 dot products go to separate blocks
     const int chunks = (it + 8) / 8;
@@ -1637,11 +1839,11 @@ struct Dispatch {
                          st, cpb);
   }
   template <int R>
-  static void maxpy_r(T* V, size_t ld, const Tiles& t, int it, double* partial, const KState* st, hipStream_t s) {
+  static void maxpy_r(T* V, size_t ld, const Tiles& t, int it, double* norms, const KState* st, hipStream_t s) {
     if (t.ntile < kBatchTiles)
-      hipLaunchKernelGGL((k_maxpy_norm<T, R, true>), dim3(t.ntile), dim3(kBlock), 0, s, V, ld, t, it, partial, st);
+      hipLaunchKernelGGL((k_maxpy_norm<T, R, true>), dim3(t.ntile), dim3(kBlock), 0, s, V, ld, t, it, norms, st);
     else
-      hipLaunchKernelGGL((k_maxpy_norm<T, R, false>), dim3(t.ntile), dim3(kBlock), 0, s, V, ld, t, it, partial, st);
+      hipLaunchKernelGGL((k_maxpy_norm<T, R, false>), dim3(t.ntile), dim3(kBlock), 0, s, V, ld, t, it, norms, st);
   }
   template <int R, class X>
   static void update_r(const T* V, size_t ld, const Tiles& t, X* x, const KState* st, const int* xrow,
@@ -1652,7 +1854,7 @@ struct Dispatch {
       hipLaunchKernelGGL((k_update_x<T, X, R, false>), dim3(t.ntile), dim3(kBlock), 0, s, V, ld, t, x, st, xrow);
   }
   static void mdot(int R, const T* V, size_t ld, const Tiles& t, int it, double* partial, int pstride,
-                   const KState* st, hipStream_t s) {
+                   KState* st, hipStream_t s) {
     switch (R) {
       case 16: mdot_r<16>(V, ld, t, it, partial, pstride, st, s); break;
       case 8: mdot_r<8>(V, ld, t, it, partial, pstride, st, s); break;
@@ -1661,14 +1863,14 @@ struct Dispatch {
       default: mdot_r<1>(V, ld, t, it, partial, pstride, st, s); break;
     }
   }
-  static void maxpy(int R, T* V, size_t ld, const Tiles& t, int it, double* partial, const KState* st,
+  static void maxpy(int R, T* V, size_t ld, const Tiles& t, int it, double* norms, const KState* st,
                     hipStream_t s) {
     switch (R) {
-      case 16: maxpy_r<16>(V, ld, t, it, partial, st, s); break;
-      case 8: maxpy_r<8>(V, ld, t, it, partial, st, s); break;
-      case 4: maxpy_r<4>(V, ld, t, it, partial, st, s); break;
-      case 2: maxpy_r<2>(V, ld, t, it, partial, st, s); break;
-      default: maxpy_r<1>(V, ld, t, it, partial, st, s); break;
+      case 16: maxpy_r<16>(V, ld, t, it, norms, st, s); break;
+      case 8: maxpy_r<8>(V, ld, t, it, norms, st, s); break;
+      case 4: maxpy_r<4>(V, ld, t, it, norms, st, s); break;
+      case 2: maxpy_r<2>(V, ld, t, it, norms, st, s); break;
+      default: maxpy_r<1>(V, ld, t, it, norms, st, s); break;
     }
   }
   template <class X>
@@ -1759,6 +1961,15 @@ KResult collect(KWork& w, bool mixed) {
 // estimate passes the test ends early and the restart residual decides.
 // inv_x (mixed Jacobi only) holds the FP64 inverse diagonal.  Cases run their
 // cycles in lockstep; a case that has finished drops out of every kernel.
+// Whether a solve without ILU takes the two launches of k_spmv_dots per step:
+// one case of at most kBlock tiles of one row per thread on a SELL-64 copy
+// whose windows lie inside a tile.
+template <class T>
+bool two_launch_steps(const KWork& w, const SellView<T>& sell, int L, int R) {
+  return w.ncase == 1 && w.tiles[0].ntile <= kBlock && L == 0 && R == 1 && sell.ptr && sell.tiled && !sell.two &&
+         !sell.scase;
+}
+
 template <class T, class X>
 KResult gmres(const CsrView<T>& A, const CsrView<X>& Ares, const X* b, X* x, const s355_ksp_opts& o, bool zero_guess,
               KWork& w, X* inv_x, hipStream_t s) {
@@ -1808,6 +2019,7 @@ KResult gmres(const CsrView<T>& A, const CsrView<X>& Ares, const X* b, X* x, con
   }
   init_states(w, o, s);
   const int pstride = m + 1;
+  if (!w.norms) throw std::runtime_error("gmres: no norm buffer");
   if (static_cast<size_t>(tl.ntile) * pstride > w.partial_len) throw std::runtime_error("gmres: partial buffer too small");
   if (!zero_guess) {
     if (lu) {
@@ -1844,42 +2056,43 @@ KResult gmres(const CsrView<T>& A, const CsrView<X>& Ares, const X* b, X* x, con
                        zero_guess ? 1 : 0, mixed ? 1 : 0);
     S355_LAUNCH_CHECK();
   };
-  // One case on a small system (at most kBlock tiles) without ILU, where
-  // launches rather than bytes set the time: the finalisation of step it - 1
-  // runs inside the SELL product of step it.  It is pending after each step
-  // and launched on its own when the product does not take it (before a
-  // state read, at the cycle's end, before a timed product).
-  const bool fuse_fin = nc == 1 && tl.ntile <= kBlock && !lu && L == 0 && !sell.two && !sell.scase;
+  // One case on a small system without ILU: two launches per step (see
+  // k_spmv_dots), the same bits as the four.  An SpMV that is timed on its own
+  // takes the four.
+  const bool small = two_launch_steps<T>(w, sell, L, R) && !lu;
+  // the tile norms of the newest basis vector alternate between two arrays; the
+  // finalisation of step it - 1 runs beside step it, the cycle's last on its own
+  double* const norms[2] = {w.norms, w.norms + w.tiles[0].ntile};
   int fin_pending = -1;
   auto flush_fin = [&] {
     if (fin_pending < 0) return;
-    hipLaunchKernelGGL(k_arnoldi_finalize, dim3(nc), dim3(kBlock), 0, s, w.partial, tl, fin_pending, m, w.st);
+    hipLaunchKernelGGL(k_arnoldi_finalize, dim3(nc), dim3(kBlock), 0, s, norms[fin_pending & 1], tl, fin_pending, m,
+                       w.st);
     S355_LAUNCH_CHECK();
     fin_pending = -1;
   };
   auto enqueue_iteration = [&](int it, bool timed) {
     hipEvent_t e0 = nullptr, e1 = nullptr;
     const bool rec = timed && w.timer && (w.timer->seen++ % w.timer->every) == 0 && w.timer->take(e0, e1);
-    const bool fused = fuse_fin && !rec && it > 0 && fin_pending == it - 1;
-    if (!fused) flush_fin();
-    if (rec) S355_HIP(hipEventRecord(e0, s));
-    if (lu) {
-      launch_spmv<T>(L, w.nt, A, sell, tl, V + it * ld, static_cast<const T*>(nullptr), tmp, w.st, it, s);
-    } else if (fused) {
-      launch_sell_fin<T>(w.nt, sell, tl, V + it * ld, inv, V + (it + 1) * ld, w.st, w.partial, it, m, s);
-      fin_pending = -1;
+    const int fin = fin_pending >= 0 && fin_pending == it - 1 ? 1 : 0;
+    const double* before = norms[(it + 1) & 1];
+    if (small && !rec) {
+      launch_spmv_dots<T>(w.nt, sell, tl, V, ld, inv, w.st, it, w.partial, s);
+      hipLaunchKernelGGL((k_orth_update<T>), dim3(tl.ntile + fin), dim3(kBlock), 0, s, V, ld, tl, w.partial, before,
+                         norms[it & 1], it, m, fin, w.st);
     } else {
-      launch_spmv<T>(L, w.nt, A, sell, tl, V + it * ld, inv, V + (it + 1) * ld, w.st, it, s);
+      if (rec) S355_HIP(hipEventRecord(e0, s));
+      if (lu)
+        launch_spmv<T>(L, w.nt, A, sell, tl, V + it * ld, static_cast<const T*>(nullptr), tmp, w.st, s);
+      else
+        launch_spmv<T>(L, w.nt, A, sell, tl, V + it * ld, inv, V + (it + 1) * ld, w.st, s);
+      if (rec) S355_HIP(hipEventRecord(e1, s));
+      if (lu) ilu_apply(A, *w.ilu, lu, tmp, V + (it + 1) * ld, ilu_st, s, w.graphs, &w);
+      Dispatch<T>::mdot(R, V, ld, tl, it, w.partial, pstride, w.st, s);
+      hipLaunchKernelGGL(k_orth, dim3(it + 1 + fin, nc), dim3(kBlock), 0, s, w.partial, before, tl, it, m, fin, w.st);
+      Dispatch<T>::maxpy(R, V, ld, tl, it, norms[it & 1], w.st, s);
     }
-    if (rec) S355_HIP(hipEventRecord(e1, s));
-    if (lu) ilu_apply(A, *w.ilu, lu, tmp, V + (it + 1) * ld, ilu_st, s, w.graphs, &w);
-    Dispatch<T>::mdot(R, V, ld, tl, it, w.partial, pstride, w.st, s);
-    hipLaunchKernelGGL(k_mdot_final, dim3(it + 1, nc), dim3(kBlock), 0, s, w.partial, tl, pstride, w.st);
-    Dispatch<T>::maxpy(R, V, ld, tl, it, w.partial, w.st, s);
-    if (fuse_fin)
-      fin_pending = it;
-    else
-      hipLaunchKernelGGL(k_arnoldi_finalize, dim3(nc), dim3(kBlock), 0, s, w.partial, tl, it, m, w.st);
+    fin_pending = it;
     S355_LAUNCH_CHECK();
   };
   auto enqueue_end = [&] {
@@ -1921,6 +2134,7 @@ KResult gmres(const CsrView<T>& A, const CsrView<X>& Ares, const X* b, X* x, con
       if (first_c && ksplit < m) {
         launch(1, [&] {
           enqueue_restart(true, zero_guess);
+          fin_pending = -1;
           for (int it = 0; it < ksplit; ++it) enqueue_iteration(it, false);
           flush_fin();
         });
@@ -1969,7 +2183,7 @@ KResult gmres(const CsrView<T>& A, const CsrView<X>& Ares, const X* b, X* x, con
       ++it;
       ++its;
       if (it % check_every == 0 && it < m) {
-        flush_fin();
+        // (the state lags a step: its last finalisation runs beside the next step)
         read_headers(w, s);
         if (all_stopped(w)) break;
       }
@@ -2052,7 +2266,7 @@ KResult cg(const CsrView<T>& A, const T* b, T* x, const s355_ksp_opts& o, bool z
 
 __global__ void k_bench_init(KState* st, int ncase) {
   for (int c = threadIdx.x; c < ncase; c += blockDim.x) {
-    st[c].reason = 0;
+    st[c].reason = st[c].ended = 0;
     st[c].scale[0] = 1.0;
     st[c].scale[1] = 1.0;
   }
@@ -2246,13 +2460,14 @@ void autotune(const CsrView<T>& A, KWork& w, int m, hipStream_t s) {
   hipLaunchKernelGGL(k_bench_init, dim3(1), dim3(kBlock), 0, s, w.st, w.ncase);
   S355_LAUNCH_CHECK();
   const T* none = nullptr;
-  // One small case: the solve runs the SELL product of step j together with
-  // the finalisation of step j - 1, and any other product beside a launch of
-  // its own, so every candidate is timed with that finalisation (and a reset
-  // of the state, the same for all).  The shapes are tuned once for every
-  // solve of the context: an ILU(0) solve, which keeps the two apart, then
-  // runs the shape timed with the saving it does not take.
-  const bool with_fin = w.ncase == 1 && w.tiles[0].ntile <= kBlock && m >= 2;
+  // One small case takes the SELL-64 copy with windows inside a tile and one
+  // row per thread, two launches a step, whatever the four launches of other
+  // shapes measure here: only the matrix loads are left to choose.  (The
+  // shapes serve every solve of the context, ILU(0) solves too.)
+  int tiled = -1;
+  if (w.ncase == 1 && w.tiles[0].ntile <= kBlock)
+    for (int sv = kSellVariants - 1; sv >= 0; --sv)
+      if (two_launch_steps<T>(w, sell_of<T>(w, n, sv), 0, 1)) tiled = sv;
   TuneReport rep;
   int best_l = 8, best_nt = 0;
   double best = 1e300;
@@ -2261,6 +2476,7 @@ void autotune(const CsrView<T>& A, KWork& w, int m, hipStream_t s) {
     for (int sv = 0; sv < (L == 0 ? kSellVariants : 1); ++sv) {
       const SellView<T> sell = sell_of<T>(w, n, sv);
       if (L == 0 && !sell.ptr) continue;
+      if (tiled >= 0 && (L != 0 || sv != tiled)) continue;
       if (L == 0) {
         // values of this window's copy from the CSR matrix being tuned on
         const SellPat& pt = w.sell[sv];
@@ -2270,19 +2486,10 @@ void autotune(const CsrView<T>& A, KWork& w, int m, hipStream_t s) {
       for (int nt : {0, 1}) {
         const double ms = time_ms(
             [&] {
-              if (with_fin) {
-                // (a finalisation may end the timing solve: the state is reset first)
-                hipLaunchKernelGGL(k_bench_init, dim3(1), dim3(kBlock), 0, s, w.st, w.ncase);
-                if (L == 0 && !sell.two) {
-                  launch_sell_fin<T>(nt, sell, w.tiles[0], V, none, V + ld, w.st, w.partial, 1, m, s);
-                } else {
-                  launch_spmv<T>(L, nt, A, sell, w.tiles[0], V, none, V + ld, w.st, 1, s);
-                  hipLaunchKernelGGL(k_arnoldi_finalize, dim3(1), dim3(kBlock), 0, s, w.partial, w.tiles[0], 0, m,
-                                     w.st);
-                }
-              } else {
-                launch_spmv<T>(L, nt, A, sell, w.tiles[0], V, none, V + ld, w.st, 0, s);
-              }
+              if (tiled >= 0)
+                launch_spmv_dots<T>(nt, sell, w.tiles[0], V, ld, none, w.st, m / 2, w.partial, s);
+              else
+                launch_spmv<T>(L, nt, A, sell, w.tiles[0], V, none, V + ld, w.st, s);
             },
             5, s);
         rep.spmv_ms[spmv_variant(L, nt, sv)] = ms;
@@ -2304,7 +2511,7 @@ void autotune(const CsrView<T>& A, KWork& w, int m, hipStream_t s) {
         double ms2[2];
         for (int two = 0; two < 2; ++two) {
           sell.two = two;
-          ms2[two] = time_ms([&] { launch_spmv<T>(0, best_nt, A, sell, w.tiles[0], V, none, V + ld, w.st, 0, s); },
+          ms2[two] = time_ms([&] { launch_spmv<T>(0, best_nt, A, sell, w.tiles[0], V, none, V + ld, w.st, s); },
                              5, s);
         }
         w.sell2 = ms2[1] < ms2[0] ? 1 : 0;
@@ -2313,23 +2520,25 @@ void autotune(const CsrView<T>& A, KWork& w, int m, hipStream_t s) {
   }
   // the Gram-Schmidt launches of three Arnoldi steps across the cycle (a
   // quarter, half and three quarters of the restart length) at every tile
-  // size; the tile count also sets the work of the final reduction.  The
-  // state is running again first (a finalisation above may have ended it,
-  // and the kernels of an ended solve return at once).
-  hipLaunchKernelGGL(k_bench_init, dim3(1), dim3(kBlock), 0, s, w.st, w.ncase);
-  S355_LAUNCH_CHECK();
+  // size; the tile count also sets the work of the final reduction
   const int it = m / 2;
   int best_r = pick_r(n, sizeof(T));
   best = 1e300;
   for (int R : {1, 2, 4, 8, 16}) {
     const Tiles& t = w.tiles[log2_r(R)];
     if (static_cast<size_t>(t.ntile) * (m + 1) > w.partial_len) continue;
+    if (tiled >= 0 && R != 1) continue;
     const double ms = time_ms(
         [&] {
           for (int j : {m / 4, m / 2, (3 * m) / 4}) {
+            if (tiled >= 0) {
+              hipLaunchKernelGGL((k_orth_update<T>), dim3(t.ntile), dim3(kBlock), 0, s, V, ld, t, w.partial, w.norms,
+                                 w.norms + t.ntile, j, m, 0, w.st);
+              continue;
+            }
             Dispatch<T>::mdot(R, V, ld, t, j, w.partial, m + 1, w.st, s);
-            hipLaunchKernelGGL(k_mdot_final, dim3(j + 1, w.ncase), dim3(kBlock), 0, s, w.partial, t, m + 1, w.st);
-            Dispatch<T>::maxpy(R, V, ld, t, j, w.partial, w.st, s);
+            hipLaunchKernelGGL(k_orth, dim3(j + 1, w.ncase), dim3(kBlock), 0, s, w.partial, w.norms, t, j, m, 0, w.st);
+            Dispatch<T>::maxpy(R, V, ld, t, j, w.norms, w.st, s);
           }
         },
         5, s) / 3.0;
@@ -2471,7 +2680,7 @@ double bench_spmv(const CsrView<T>& A, const T* x, T* y, const T* inv, KWork& w,
   const Tiles& t = w.tiles[0];
   const SellView<T> sell = sell_of<T>(w, A.n);
   const int L = (w.lanes == 0 && !sell.ptr) ? 8 : w.lanes;
-  launch_spmv<T>(L, w.nt, A, sell, t, x, inv, y, w.st, 0, s);
+  launch_spmv<T>(L, w.nt, A, sell, t, x, inv, y, w.st, s);
   S355_LAUNCH_CHECK();
   hipEvent_t e0, e1;
   S355_HIP(hipEventCreate(&e0));
@@ -2482,7 +2691,7 @@ double bench_spmv(const CsrView<T>& A, const T* x, T* y, const T* inv, KWork& w,
     // does inside a Krylov iteration whose other kernels stream the basis
     if (flush) fill_zero(flush, flush_bytes, s);
     S355_HIP(hipEventRecord(e0, s));
-    launch_spmv<T>(L, w.nt, A, sell, t, x, inv, y, w.st, 0, s);
+    launch_spmv<T>(L, w.nt, A, sell, t, x, inv, y, w.st, s);
     S355_HIP(hipEventRecord(e1, s));
     S355_HIP(hipEventSynchronize(e1));
     float ms = 0.f;

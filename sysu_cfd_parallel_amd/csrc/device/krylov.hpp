@@ -31,20 +31,22 @@ struct KState {
   int maxit;
   int done;    // the case's solve has ended (reason final)
   int cycles;  // restart cycles started
+  int ended;   // reason as the last multi-dot found it (see k_orth)
+  int pad0;
   double rnorm, rnorm0, ttol, snorm;
   double rtol, abstol, dtol;
   double pad;
   double H[(kMaxRestart + 1) * (kMaxRestart + 1)];  // column-major, H(r,c) = H[c*(m+1)+r]
   double cc[kMaxRestart + 1], ss[kMaxRestart + 1], grs[kMaxRestart + 2];
   double scale[kMaxRestart + 1];  // basis vector k = scale[k] * V[k]
-  double hcol[kMaxRestart + 1];
+  double hcol[2][kMaxRestart + 1];  // Hessenberg column of step it in hcol[it & 1]
   double y[kMaxRestart + 1];
   // CG scalars
   double beta, betaold, dpi, dpiold, alpha;
 };
 
 struct KHeader {
-  int it, its, reason, maxit, done, cycles;
+  int it, its, reason, maxit, done, cycles, ended, pad0;
   double rnorm, rnorm0, ttol, snorm;
 };
 static_assert(offsetof(KState, rnorm) == offsetof(KHeader, rnorm), "KHeader mirrors the head of KState");
@@ -79,6 +81,7 @@ struct SellView {
   const T* val = nullptr;
   const int* scase = nullptr;  // batches: case of each slice, -1 when its rows span two cases
   int two = 0;                 // FP32, one case: two slices per wave
+  bool tiled = false;          // the rows of 256 positions are 256 consecutive rows
 };
 
 // SELL windows the autotuner chooses from: a short window keeps the rows of
@@ -190,10 +193,10 @@ struct GraphCache {
 
 // Timings taken by autotune(): SpMV per variant v = 2 k + nt (k = 0..4: CSR
 // with 1, 2, 4, 8, 16 lanes per row, k = 5..7: SELL-64 with window 64, 512,
-// 4096; nt: non-temporal matrix loads; on one case of at most kBlock tiles
-// with the Arnoldi finalisation the solve runs beside or inside the product)
-// and one Gram-Schmidt step (multi-dot + update at iteration gs_it)
-// per rows-per-thread 1, 2, 4, 8, 16; -1 = not timed.
+// 4096; nt: non-temporal matrix loads) and one Gram-Schmidt step (multi-dot +
+// update at iteration gs_it) per rows-per-thread 1, 2, 4, 8, 16; -1 = not timed.
+// One case of at most kBlock tiles: the product with its dots, and the rest of
+// the step, in the one shape such a system takes.
 struct TuneReport {
   // CSR lanes 1, 2, 4, 8, 16 then SELL-64 with windows 64, 512, 4096, each
   // temporal / non-temporal
@@ -237,6 +240,7 @@ struct KWork {
   const IluLevels* ilu = nullptr;
   double* partial = nullptr;
   size_t partial_len = 0;
+  double* norms = nullptr;  // 2 x the tiles of kBlock rows: ||w||^2 per tile of the last two Arnoldi steps
   int lanes = 8;            // CSR SpMV lanes per row (1, 2, 4, 8, 16); 0 = SELL-64 SpMV
   int nt = 0;               // SpMV loads the matrix non-temporally
   int sell_v = kSellDefault;  // SELL window in use (index into kSellSigma) when lanes == 0
