@@ -103,12 +103,46 @@ struct Tiles {
   }
 };
 
-// Butterfly sum over the 64 lanes of a wavefront; every lane ends with the
-// same value, produced by the same fixed pairing order.
-template <class T>
-__device__ __forceinline__ T wave_sum(T v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, kWave);
+// Values of other lanes without the LDS exchange a __shfl_xor takes (about 60
+// cycles each): swapped half-waves and half-rows, rotations and quad
+// permutations inside a row of 16.
+__device__ __forceinline__ void swap32(double& a, double& b) {
+  // a: its lower half and b's lower half; b: a's upper half and its upper half
+  const auto lo = __builtin_amdgcn_permlane32_swap(__double2loint(a), __double2loint(b), false, false);
+  const auto hi = __builtin_amdgcn_permlane32_swap(__double2hiint(a), __double2hiint(b), false, false);
+  a = __hiloint2double(hi[0], lo[0]);
+  b = __hiloint2double(hi[1], lo[1]);
+}
+__device__ __forceinline__ void swap16(double& a, double& b) {
+  // the same for the even and odd rows of 16
+  const auto lo = __builtin_amdgcn_permlane16_swap(__double2loint(a), __double2loint(b), false, false);
+  const auto hi = __builtin_amdgcn_permlane16_swap(__double2hiint(a), __double2hiint(b), false, false);
+  a = __hiloint2double(hi[0], lo[0]);
+  b = __hiloint2double(hi[1], lo[1]);
+}
+template <int Ctrl>
+__device__ __forceinline__ double dpp(double v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), Ctrl, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), Ctrl, 0xf, 0xf, true);
+  return __hiloint2double(hi, lo);
+}
+constexpr int kDppXor8 = 0x128;  // row_ror:8
+constexpr int kDppXor2 = 0x4e;   // quad_perm [2, 3, 0, 1]
+constexpr int kDppXor1 = 0xb1;   // quad_perm [1, 0, 3, 2]
+
+// Butterfly sum over the 64 lanes of a wavefront (xor 32, 16, 8, 4, 2, 1); every
+// lane ends with the same value, produced by the same fixed pairing order.
+__device__ __forceinline__ double wave_sum(double v) {
+  double w = v;
+  swap32(v, w);
+  v += w;
+  w = v;
+  swap16(v, w);
+  v += w;
+  v += dpp<kDppXor8>(v);
+  v += __shfl_xor(v, 4, kWave);
+  v += dpp<kDppXor2>(v);
+  v += dpp<kDppXor1>(v);
   return v;
 }
 
@@ -116,26 +150,27 @@ __device__ __forceinline__ T wave_sum(T v) {
 // the result for k ending in lanes 8k .. 8k + 7.  Each exchange step halves
 // the values a lane carries (xor 32, 16, 8: it keeps half of them, adds its
 // partner's copies of that half), then the last value takes a full butterfly
-// over the low three lane bits: 10 exchanges instead of 48 for eight
-// wave_sum calls.  The pairing order is fixed, so the sums are reproducible.
+// over the low three lane bits.  The pairing order is fixed and that of
+// wave_sum, so the sums are reproducible.
 __device__ __forceinline__ double wave_sum8(const double (&a)[8]) {
-  const int lane = threadIdx.x & (kWave - 1);
   double b[4], c[2];
-  const bool h5 = lane & 32, h4 = lane & 16, h3 = lane & 8;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    const double send = h5 ? a[j] : a[4 + j];
-    b[j] = (h5 ? a[4 + j] : a[j]) + __shfl_xor(send, 32, kWave);
+    double x = a[j], y = a[4 + j];
+    swap32(x, y);
+    b[j] = x + y;
   }
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
-    const double send = h4 ? b[j] : b[2 + j];
-    c[j] = (h4 ? b[2 + j] : b[j]) + __shfl_xor(send, 16, kWave);
+    double x = b[j], y = b[2 + j];
+    swap16(x, y);
+    c[j] = x + y;
   }
-  const double send = h3 ? c[0] : c[1];
-  double v = (h3 ? c[1] : c[0]) + __shfl_xor(send, 8, kWave);
-#pragma unroll
-  for (int off = 4; off > 0; off >>= 1) v += __shfl_xor(v, off, kWave);
+  const bool h3 = threadIdx.x & 8;
+  double v = (h3 ? c[1] : c[0]) + dpp<kDppXor8>(h3 ? c[0] : c[1]);
+  v += __shfl_xor(v, 4, kWave);
+  v += dpp<kDppXor2>(v);
+  v += dpp<kDppXor1>(v);
   return v;
 }
 
