@@ -94,22 +94,23 @@ Context::~Context() { free_all(); }
 
 Tiles Context::make_tiles(const std::vector<int>& case_row, int tile) {
   Tiles t;
+  const int nc = static_cast<int>(case_row.size()) - 1;
   t.n = case_row.back();
   t.tile = tile;
-  t.ncase = ncase;
-  if (ncase == 1) {
+  t.ncase = nc;
+  if (nc == 1) {
     t.ntile = std::max(1, (t.n + tile - 1) / tile);
     return t;
   }
-  std::vector<int> lo, tc, ct(ncase + 1);
-  for (int c = 0; c < ncase; ++c) {
+  std::vector<int> lo, tc, ct(nc + 1);
+  for (int c = 0; c < nc; ++c) {
     ct[c] = static_cast<int>(lo.size());
     for (int r = case_row[c]; r < case_row[c + 1]; r += tile) {
       lo.push_back(r);
       tc.push_back(c);
     }
   }
-  ct[ncase] = static_cast<int>(lo.size());
+  ct[nc] = static_cast<int>(lo.size());
   t.ntile = static_cast<int>(lo.size());
   lo.push_back(t.n);
   t.lo = upload(allocs_, lo, stream);
@@ -135,6 +136,8 @@ void Context::free_all() {
   for (void* p : allocs_) hipFree(p);
   allocs_.clear();
   if (host_pinned_) hipHostFree(host_pinned_);
+  if (triple_.host) hipHostFree(triple_.host);
+  triple_.host = nullptr;
   host_pinned_ = nullptr;
   if (hdr_) hipHostFree(hdr_);
   hdr_ = nullptr;
@@ -787,16 +790,21 @@ void Context::ensure_mixed() {
   ir_.host = reinterpret_cast<double*>(static_cast<char*>(host_pinned_) + 3584);
 }
 
+// same: the matrix is the previous call's, unchanged, and so are its copies and
+// its preconditioner; rep = 3: b and x hold the three momentum components'
+// right-hand sides and solutions, solved together, records in slots 0..2
 int Context::run_solve(int which, const double* b, double* x, const s355_ksp_opts& o, bool zero_guess,
-                       s355_solve_info* info, int slot) {
+                       s355_solve_info* info, int slot, bool same, int rep) {
   const double* val = which == 0 ? df.Au : (which == 1 ? df.Ap : df.As);
   KResult r;
   if (par.graphs && !graphs_) graphs_ = std::make_unique<GraphCache>();
   kwork_.graphs = par.graphs ? graphs_.get() : nullptr;
   kwork32_.graphs = kwork_.graphs;
-  kwork_.per_case = &case_info[slot];
-  kwork32_.per_case = &case_info[slot];
-  case_info[slot].assign(ncase, KResult{});
+  std::vector<KResult> together;
+  kwork_.per_case = rep > 1 ? &together : &case_info[slot];
+  kwork32_.per_case = kwork_.per_case;
+  kwork_.prepared = kwork32_.prepared = same;
+  if (rep == 1) case_info[slot].assign(ncase, KResult{});
   if (o.pc == S355_PC_ILU0) ensure_ilu();
   if (par.precision == S355_MIXED) {
     // FP32 inner solves on the rounded matrix inside FP64 refinement
@@ -813,25 +821,34 @@ int Context::run_solve(int which, const double* b, double* x, const s355_ksp_opt
     CsrView<double> A64{dm.Nc, dm.rowptr, dm.col, dm.diag, val, dm.nnz};
     const bool tune = par.autotune && o.type == S355_KSP_GMRES && !kwork32_.tuned;
     const bool ordered = use_order(o);
-    if (!ordered) convert_to_float(val, a32_, dm.nnz, stream);  // the inner order fills its own copy
+    if (!ordered && !same) convert_to_float(val, a32_, dm.nnz, stream);  // the inner order fills its own copy
     if (ordered) {
       // the Arnoldi cycle on the rows in the inner order, tuned there
-      fill_order(val, o.pc == S355_PC_JACOBI);
+      if (!same) fill_order(val, o.pc == S355_PC_JACOBI);
       CsrView<float> Ao{dm.Nc, ord_rowptr_, ord_col_, ord_diag_, a32o_, dm.nnz};
       if (tune) tune_ordered(Ao, std::min(o.restart, kMaxRestart));
-      KWork w = ordered_work(false);
+      KWork w = ordered_work(false, same);
+      if (rep > 1) w = triple_work(w, true);
       r = ir_solve(A64, Ao, b, x, o, zero_guess, par.ir_max, par.ir_inner_rtol, w, ir_, stream);
     } else {
-      if (o.type == S355_KSP_GMRES && (tune || kwork32_.lanes == 0)) prepare_sell(val, true, tune);
+      if (o.type == S355_KSP_GMRES && !same && (tune || kwork32_.lanes == 0)) prepare_sell(val, true, tune);
       if (tune) autotune<float>(A, kwork32_, std::min(o.restart, kMaxRestart), stream);
-      r = ir_solve(A64, A, b, x, o, zero_guess, par.ir_max, par.ir_inner_rtol, kwork32_, ir_, stream);
+      KWork w3;
+      if (rep > 1) w3 = triple_work(kwork32_, true);
+      r = ir_solve(A64, A, b, x, o, zero_guess, par.ir_max, par.ir_inner_rtol, rep > 1 ? w3 : kwork32_, ir_, stream);
     }
   } else {
     CsrView<double> A{dm.Nc, dm.rowptr, dm.col, dm.diag, val, dm.nnz};
     const bool tune = par.autotune && o.type == S355_KSP_GMRES && !kwork_.tuned;
-    if (o.type == S355_KSP_GMRES && (tune || kwork_.lanes == 0)) prepare_sell(val, false, tune);
+    if (o.type == S355_KSP_GMRES && !same && (tune || kwork_.lanes == 0)) prepare_sell(val, false, tune);
     if (tune) autotune<double>(A, kwork_, std::min(o.restart, kMaxRestart), stream);
-    r = krylov_solve<double>(A, b, x, o, zero_guess, kwork_, stream);
+    KWork w3;
+    if (rep > 1) w3 = triple_work(kwork_, false);
+    r = krylov_solve<double>(A, b, x, o, zero_guess, rep > 1 ? w3 : kwork_, stream);
+  }
+  if (rep > 1) {
+    for (int k = 0; k < rep; ++k) fill_info(together[k], info + k);
+    return r.reason < 0 ? S355_NOT_CONVERGED : S355_OK;
   }
   if (ncase == 1) case_info[slot].assign(1, r);
   fill_info(r, info);
@@ -847,14 +864,92 @@ int Context::solve_velocity(double rtol, int maxit, s355_solve_info info[3]) {
   // MPIStructure.cpp:279-283 leaves V and W unsolved).
   const double* b[3] = {df.bu, df.bv, df.bw};
   double* x[3] = {df.U, df.V, df.W};
+  if (ncase == 1 && o.type == S355_KSP_GMRES && dm.Nc > 0 && dm.Nc <= kTripleRows) {
+    // the three components as one solve with three right-hand sides: they share
+    // every launch (see triple_work), each with its own state and the bits of
+    // its own solve
+    const size_t n = dm.Nc;
+    ensure_triple();
+    launch_copy3(dm.Nc, df.bu, df.bv, df.bw, b3_, b3_ + n, b3_ + 2 * n, stream);
+    launch_copy3(dm.Nc, df.U, df.V, df.W, x3_, x3_ + n, x3_ + 2 * n, stream);
+    rc = run_solve(0, b3_, x3_, o, false, info, 0, false, 3);
+    for (int k = 0; k < 3; ++k) {
+      S355_HIP(hipMemcpyAsync(x[k], x3_ + k * n, n * sizeof(double), hipMemcpyDeviceToDevice, stream));
+      KResult r;
+      r.iters = info[k].iters;
+      r.reason = info[k].reason;
+      r.rnorm = info[k].rnorm;
+      r.rnorm0 = info[k].rnorm0;
+      r.refinements = info[k].refinements;
+      case_info[k].assign(1, r);
+      if (r.reason >= 0) continue;
+      for (int j = k + 1; j < 3; ++j) info[j] = s355_solve_info{0, 0, 0.0, 0.0, 0, 0};  // left as they were
+      break;
+    }
+    return rc;
+  }
   for (int k = 0; k < 3; ++k) {
-    rc = run_solve(0, b[k], x[k], o, false, &info[k], k);
+    rc = run_solve(0, b[k], x[k], o, false, &info[k], k, k > 0);
     if (rc != S355_OK) {
       for (int j = k + 1; j < 3; ++j) info[j] = s355_solve_info{0, 0, 0.0, 0.0, 0, 0};
       return rc;
     }
   }
   return rc;
+}
+
+void Context::ensure_triple() {
+  if (x3_) return;
+  const size_t n = dm.Nc, ld = (3 * n + 7) / 8 * 8;
+  x3_ = alloc<double>(ld);
+  b3_ = alloc<double>(ld);
+  const std::vector<int> rows = {0, dm.Nc, 2 * dm.Nc, 3 * dm.Nc};
+  for (int r = 0; r < 5; ++r) triple_.tiles[r] = make_tiles(rows, kBlock << r);
+  const size_t tiles1 = triple_.tiles[0].ntile;
+  triple_.partial_len = tiles1 * (max_restart_ + 1);
+  triple_.partial = alloc<double>(triple_.partial_len);
+  triple_.norms = alloc<double>(2 * tiles1);
+  triple_.st = alloc<KState>(3);
+  S355_HIP(hipHostMalloc(reinterpret_cast<void**>(&triple_.host), sizeof(KHeader) * 3, hipHostMallocDefault));
+  // sized for FP64 vectors, which the mixed path's FP32 ones then fit
+  const size_t elem = par.precision == S355_MIXED ? sizeof(float) : sizeof(double);
+  triple_elem_ = elem;
+  triple_.V = alloc<char>((static_cast<size_t>(max_restart_) + 1) * ld * elem);
+  triple_.r = alloc<char>(ld * elem);
+}
+
+// The workspace of the three momentum components' solve: the shapes, matrix
+// copies and preconditioner of w, the vectors and states of three cases.
+KWork Context::triple_work(const KWork& w, bool fp32) {
+  const size_t n = dm.Nc, elem = fp32 ? sizeof(float) : sizeof(double);
+  if (elem > triple_elem_) {  // the precision was changed
+    triple_.V = alloc<char>((static_cast<size_t>(max_restart_) + 1) * ((3 * n + 7) / 8 * 8) * elem);
+    triple_.r = alloc<char>((3 * n + 7) / 8 * 8 * elem);
+    triple_.ilu_zl = nullptr;
+    triple_elem_ = elem;
+  }
+  KWork t = w;
+  t.n = 3 * dm.Nc;
+  t.ncase = t.rep = 3;
+  t.ld = (3 * n + 7) / 8 * 8;
+  for (int r = 0; r < 5; ++r) t.tiles[r] = triple_.tiles[r];
+  t.V = triple_.V;
+  t.r = triple_.r;
+  t.partial = triple_.partial;
+  t.partial_len = triple_.partial_len;
+  t.norms = triple_.norms;
+  t.st = triple_.st;
+  t.host = triple_.host;
+  t.timer = nullptr;  // products of three vectors are not what it times
+  if (w.ilu) {
+    if (!triple_.ilu_zl) {
+      triple_.ilu_zl = alloc<char>(6 * n * triple_elem_);
+      triple_.ilu_zu = alloc<char>(6 * n * triple_elem_);
+    }
+    t.ilu_zl = triple_.ilu_zl;
+    t.ilu_zu = triple_.ilu_zu;
+  }
+  return t;
 }
 
 void Context::cal_ru_face() { launch_ruface(dm, df, stream); }
@@ -1178,14 +1273,14 @@ void Context::fill_order(const double* csr_val, bool jacobi) {
 // fill_order): the shapes of the FP32 workspace, the ordered SELL copies (of
 // the window in use, or all of them) filled from the ordered CSR, and the
 // position maps.
-KWork Context::ordered_work(bool all) {
+KWork Context::ordered_work(bool all, bool filled) {
   KWork w = kwork32_;
   for (int v = 0; v < kSellVariants; ++v) {
     w.sell[v] = osell_[v];
     w.sell_vals[v] = nullptr;
     if (all || (w.lanes == 0 && v == w.sell_v)) {
       if (!osell32_[v]) osell32_[v] = alloc<float>(osell_[v].slots);
-      sell_fill<float, float>(osell_[v].src, osell_[v].slots, a32o_, osell32_[v], stream);
+      if (!filled) sell_fill<float, float>(osell_[v].src, osell_[v].slots, a32o_, osell32_[v], stream);
       w.sell_vals[v] = osell32_[v];
     }
   }

@@ -106,7 +106,9 @@ class Context {
   void allocate_fields();
   void free_all();
   int run_solve(int which_matrix, const double* b, double* x, const s355_ksp_opts& o, bool zero_guess,
-                s355_solve_info* info, int slot);
+                s355_solve_info* info, int slot, bool same = false, int rep = 1);
+  void ensure_triple();
+  KWork triple_work(const KWork& w, bool fp32);
   Tiles make_tiles(const std::vector<int>& case_row, int tile);
   void ensure_mixed();
   void ensure_ilu();
@@ -123,7 +125,7 @@ class Context {
   bool fp32_assembly() const { return par.precision == S355_MIXED && par.assembly_fp32 == 1; }
   void ensure_order();
   void fill_order(const double* csr_val, bool jacobi);
-  KWork ordered_work(bool all);
+  KWork ordered_work(bool all, bool filled = false);
   void tune_ordered(const CsrView<float>& Ao, int m);
 
   std::vector<void*> allocs_;
@@ -143,6 +145,11 @@ class Context {
   float* a32_ = nullptr;
   KWork kwork32_{};
   IrWork ir_{};
+  // the three momentum components solved together: vectors and states, sized by
+  // triple_elem_ bytes an element
+  KWork triple_{};
+  size_t triple_elem_ = 0;
+  double *x3_ = nullptr, *b3_ = nullptr;
   // inner order of mixed GMRES: rows in reverse Cuthill-McKee order
   bool have_order_ = false, order_ok_ = false;
   int order_kind_ = 0;  // params.inner_order the order was built for

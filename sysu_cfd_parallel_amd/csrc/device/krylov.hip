@@ -114,6 +114,7 @@ template <class T, bool Wide>
 __global__ void __launch_bounds__(kBlock) k_ilu_group(IluLaunch g, const int* __restrict__ len,
                                                       const int* __restrict__ col, const T* __restrict__ coef,
                                                       const T* __restrict__ own, T* buf, int n, const KState* st) {
+  buf += blockIdx.y * 2 * static_cast<size_t>(n);  // right-hand side blockIdx.y
   // the workgroup's class, by constant indices (the launch stays in registers)
   const int blk = blockIdx.x;
   int cls = 0, p0 = g.p0[0], nrows = g.nrows[0], width = g.width[0], blk0 = 0;
@@ -130,7 +131,7 @@ __global__ void __launch_bounds__(kBlock) k_ilu_group(IluLaunch g, const int* __
     }
   const int k = (blk - blk0) * static_cast<int>(blockDim.x) + threadIdx.x;
   if (k >= nrows) return;
-  if (st && st->reason) return;
+  if (st && st[blockIdx.y].reason) return;
   const int p = p0 + k, L = len[p];
   const size_t q0 = static_cast<size_t>(off) + k;
   T z = buf[p];
@@ -214,14 +215,17 @@ __global__ void __launch_bounds__(kBlock) k_ilu_merge(int k0, int nrows, const i
 // consecutive there: a workgroup reading (or writing) a contiguous range
 // writes (reads) one short contiguous piece per run, and consecutive workgroups on one XCD extend the same runs in its L2.
 // scatter: dst[pos[q]] = src[q]
+// (right-hand side blockIdx.y at src + blockIdx.y * ssrc, dst + blockIdx.y * sdst)
 template <class T, int Tag>
 __global__ void __launch_bounds__(kBlock) k_scatter(int n, const int* __restrict__ pos, const T* __restrict__ src,
-                                                    T* __restrict__ dst, const KState* st) {
+                                                    size_t ssrc, T* __restrict__ dst, size_t sdst, const KState* st) {
+  src += blockIdx.y * ssrc;
+  dst += blockIdx.y * sdst;
   const int q = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
   if (q >= n) return;
   const int p = pos[q];
   const T v = src[q];
-  if (st && st->reason) return;
+  if (st && st[blockIdx.y].reason) return;
   dst[p] = v;
 }
 
@@ -233,12 +237,14 @@ template <class T, int Tag, bool Dot = false>
 __global__ void __launch_bounds__(kBlock) k_gather_at(int n, const int* __restrict__ idx, const T* __restrict__ src,
                                                       T* __restrict__ dst, const KState* st,
                                                       const T* __restrict__ r = nullptr, double* partial = nullptr) {
+  src += blockIdx.y * 2 * static_cast<size_t>(n);
+  dst += blockIdx.y * static_cast<size_t>(n);
   const int b = xcd_block(blockIdx.x, gridDim.x);
   const int q = b * blockDim.x + threadIdx.x;
   if constexpr (!Dot) {
     if (q >= n) return;
     const int p = idx[q];
-    if (st && st->reason) return;
+    if (st && st[blockIdx.y].reason) return;
     dst[q] = src[p];
   } else {
     __shared__ double lds[kBlock / kWave];
@@ -303,7 +309,7 @@ void ilu_factor(const CsrView<T>& A, int nnz, const IluLevels& lv, T* lu, hipStr
 
 // one sweep, group by group, on buf: n inputs, then n results
 template <class T>
-void ilu_sweep(const IluSweep& w, const T* coef, const T* own, T* buf, const KState* st, hipStream_t s) {
+void ilu_sweep(const IluSweep& w, const T* coef, const T* own, T* buf, const KState* st, int rep, hipStream_t s) {
   for (size_t g = 0; g + 1 < w.group.size(); ++g) {
     IluLaunch a{};
     int rows = 0, blocks = 0, k = w.group[g];
@@ -320,12 +326,13 @@ void ilu_sweep(const IluSweep& w, const T* coef, const T* own, T* buf, const KSt
       blocks += grid_for(u.nrows, b);
     }
     const bool wide = w.subs[w.group[g + 1] - 1].cls >= kNarrowClasses;
-    hipLaunchKernelGGL((wide ? k_ilu_group<T, true> : k_ilu_group<T, false>), dim3(blocks), dim3(b), 0, s, a, w.len,
+    hipLaunchKernelGGL((wide ? k_ilu_group<T, true> : k_ilu_group<T, false>), dim3(blocks, rep), dim3(b), 0, s, a, w.len,
                        w.col, coef, own, buf, w.n, st);
   }
 }
 
-// z = (LU)^-1 r ; r and z distinct.  With a graph cache the sweeps (one
+// z = (LU)^-1 r ; r and z distinct (w->rep vectors each, one after the other).
+// With a graph cache the sweeps (one
 // launch per group) are captured once per (factor, r, z) and replayed.
 // With dot (CG) the last move also leaves the partial sums of (z, z) and
 // (z, r) per kBlock rows there (see k_gather_at).
@@ -346,18 +353,19 @@ void ilu_apply(const CsrView<T>& A, const IluLevels& lv, const T* lu, const T* r
     throw std::invalid_argument("ILU(0) application without its sweep workspace");
   T* zl = static_cast<T*>(w->ilu_zl);
   T* zu = static_cast<T*>(w->ilu_zu);
-  const int n = lv.lptr.back();
-  const int gn = grid_for(n);
+  const int n = lv.lptr.back(), rep = w->rep;
+  const size_t n1 = n;
+  const dim3 gn(grid_for(n), rep);
   // r into the lower order, the lower sweep, its result into the upper
   // order, the upper sweep, z back into the natural order
-  hipLaunchKernelGGL((k_scatter<T, 0>), dim3(gn), dim3(kBlock), 0, s, n, lv.lpos, r, zl, st);
-  ilu_sweep<T>(lv.lower, static_cast<const T*>(w->ilu_lcoef), static_cast<const T*>(nullptr), zl, st, s);
-  hipLaunchKernelGGL((k_scatter<T, 1>), dim3(gn), dim3(kBlock), 0, s, n, lv.l2u, zl + n, zu, st);
-  ilu_sweep<T>(lv.upper, static_cast<const T*>(w->ilu_ucoef), static_cast<const T*>(w->ilu_own), zu, st, s);
+  hipLaunchKernelGGL((k_scatter<T, 0>), gn, dim3(kBlock), 0, s, n, lv.lpos, r, n1, zl, 2 * n1, st);
+  ilu_sweep<T>(lv.lower, static_cast<const T*>(w->ilu_lcoef), static_cast<const T*>(nullptr), zl, st, rep, s);
+  hipLaunchKernelGGL((k_scatter<T, 1>), gn, dim3(kBlock), 0, s, n, lv.l2u, zl + n, 2 * n1, zu, 2 * n1, st);
+  ilu_sweep<T>(lv.upper, static_cast<const T*>(w->ilu_ucoef), static_cast<const T*>(w->ilu_own), zu, st, rep, s);
   if (dot)
-    hipLaunchKernelGGL((k_gather_at<T, 2, true>), dim3(gn), dim3(kBlock), 0, s, n, lv.upos, zu + n, z, st, r, dot);
+    hipLaunchKernelGGL((k_gather_at<T, 2, true>), gn, dim3(kBlock), 0, s, n, lv.upos, zu + n, z, st, r, dot);
   else
-    hipLaunchKernelGGL((k_gather_at<T, 2>), dim3(gn), dim3(kBlock), 0, s, n, lv.upos, zu + n, z, st, nullptr, nullptr);
+    hipLaunchKernelGGL((k_gather_at<T, 2>), gn, dim3(kBlock), 0, s, n, lv.upos, zu + n, z, st, nullptr, nullptr);
   S355_LAUNCH_CHECK();
 }
 
@@ -414,6 +422,9 @@ __device__ __forceinline__ T row_dot(const CsrView<T>& A, const T* __restrict__ 
 template <class T, int L, bool NT>
 __global__ void __launch_bounds__(kBlock) k_spmv_pc(CsrView<T> A, Tiles t, const T* __restrict__ x,
                                                     const T* __restrict__ inv, T* __restrict__ y, const KState* st) {
+  x += blockIdx.y * static_cast<size_t>(A.n);  // right-hand side blockIdx.y of the same matrix
+  y += blockIdx.y * static_cast<size_t>(A.n);
+  st += blockIdx.y;
   const int g = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
   const int row = g / L, lane = g % L;
   // the lanes of one row share its case, so they leave together
@@ -534,6 +545,9 @@ __device__ __forceinline__ T sell_row_any(const SellView<T>& A, const Tiles& t, 
 template <class T, bool NT, bool PC, bool C16 = false>
 __global__ void __launch_bounds__(kBlock) k_spmv_sell(SellView<T> A, Tiles t, const T* __restrict__ x,
                                                       const T* __restrict__ inv, T* __restrict__ y, const KState* st) {
+  x += blockIdx.y * static_cast<size_t>(A.n);
+  y += blockIdx.y * static_cast<size_t>(A.n);
+  st += blockIdx.y;
   const int pos = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
   if (pos >= A.n) return;
   // a wave is one slice (64 consecutive positions), so the slice index and
@@ -599,6 +613,9 @@ template <class T, bool NT, bool PC, bool C16 = false>
 __global__ void __launch_bounds__(kBlock) k_spmv_sell2(SellView<T> A, Tiles t, const T* __restrict__ x,
                                                        const T* __restrict__ inv, T* __restrict__ y,
                                                        const KState* st) {
+  x += blockIdx.y * static_cast<size_t>(A.n);
+  y += blockIdx.y * static_cast<size_t>(A.n);
+  st += blockIdx.y;
   // wave w takes slices 2w and 2w + 1
   const int wv = xcd_block(blockIdx.x, gridDim.x) * (kBlock / kWave) + static_cast<int>(threadIdx.x) / kWave;
   const int sl = __builtin_amdgcn_readfirstlane(2 * wv), lane = threadIdx.x & (kWave - 1);
@@ -660,69 +677,69 @@ inline int spmv_variant(int lanes, int nt, int sell_v) {
 
 template <class T, int L>
 void launch_spmv_l(bool nt, const CsrView<T>& A, const Tiles& t, const T* x, const T* inv, T* y, const KState* st,
-                   hipStream_t s) {
+                   int rep, hipStream_t s) {
   const int g = grid_for(static_cast<long>(A.n) * L);
   if (nt)
-    hipLaunchKernelGGL((k_spmv_pc<T, L, true>), dim3(g), dim3(kBlock), 0, s, A, t, x, inv, y, st);
+    hipLaunchKernelGGL((k_spmv_pc<T, L, true>), dim3(g, rep), dim3(kBlock), 0, s, A, t, x, inv, y, st);
   else
-    hipLaunchKernelGGL((k_spmv_pc<T, L, false>), dim3(g), dim3(kBlock), 0, s, A, t, x, inv, y, st);
+    hipLaunchKernelGGL((k_spmv_pc<T, L, false>), dim3(g, rep), dim3(kBlock), 0, s, A, t, x, inv, y, st);
 }
 
 // the SELL-64 product: two slices per wave when the view says so (FP32, one
 // case), else one
 template <class T, bool NT, bool PC, bool C16>
-void launch_sell(const SellView<T>& sell, const Tiles& t, const T* x, const T* inv, T* y, const KState* st, hipStream_t s) {
+void launch_sell(const SellView<T>& sell, const Tiles& t, const T* x, const T* inv, T* y, const KState* st, int rep, hipStream_t s) {
   if constexpr (std::is_same<T, float>::value) {
     if (sell.two) {
       // two slices per wave: kBlock / kWave waves per block
       const int nsl = (sell.n + 63) / 64;
       const int g2 = grid_for((nsl + 1) / 2, kBlock / kWave);
-      hipLaunchKernelGGL((k_spmv_sell2<T, NT, PC, C16>), dim3(g2), dim3(kBlock), 0, s, sell, t, x, inv, y, st);
+      hipLaunchKernelGGL((k_spmv_sell2<T, NT, PC, C16>), dim3(g2, rep), dim3(kBlock), 0, s, sell, t, x, inv, y, st);
       return;
     }
   }
-  hipLaunchKernelGGL((k_spmv_sell<T, NT, PC, C16>), dim3(grid_for(sell.n)), dim3(kBlock), 0, s, sell, t, x, inv, y,
+  hipLaunchKernelGGL((k_spmv_sell<T, NT, PC, C16>), dim3(grid_for(sell.n), rep), dim3(kBlock), 0, s, sell, t, x, inv, y,
                      st);
 }
 
 template <class T, bool NT, bool PC>
 void launch_sell_c(const SellView<T>& sell, const Tiles& t, const T* x, const T* inv, T* y, const KState* st,
-                   hipStream_t s) {
+                   int rep, hipStream_t s) {
   if (sell.col16) {
     // 16-bit column offsets exist for the FP32 inner order only
     if constexpr (std::is_same<T, float>::value)
-      launch_sell<T, NT, PC, true>(sell, t, x, inv, y, st, s);
+      launch_sell<T, NT, PC, true>(sell, t, x, inv, y, st, rep, s);
     else
       throw std::logic_error("16-bit SELL columns in an FP64 product");
   } else {
-    launch_sell<T, NT, PC, false>(sell, t, x, inv, y, st, s);
+    launch_sell<T, NT, PC, false>(sell, t, x, inv, y, st, rep, s);
   }
 }
 
-// y = M^-1 A x with the CSR kernel at L lanes per row, or with the
+// y = M^-1 A x (rep vectors x and y, one after the other) with the CSR kernel at L lanes per row, or with the
 // SELL-64 copy for L = 0 (sell must then be set)
 template <class T>
 void launch_spmv(int L, int nt, const CsrView<T>& A, const SellView<T>& sell, const Tiles& t, const T* x, const T* inv,
-                 T* y, const KState* st, hipStream_t s) {
+                 T* y, const KState* st, hipStream_t s, int rep = 1) {
   switch (L) {
     case 0: {
       if (!sell.ptr) throw std::logic_error("SELL-64 SpMV without a SELL copy");
       if (sell.n != A.n) throw std::logic_error("SELL-64 copy of another size");
       if (nt && inv)
-        launch_sell_c<T, true, true>(sell, t, x, inv, y, st, s);
+        launch_sell_c<T, true, true>(sell, t, x, inv, y, st, rep, s);
       else if (nt)
-        launch_sell_c<T, true, false>(sell, t, x, inv, y, st, s);
+        launch_sell_c<T, true, false>(sell, t, x, inv, y, st, rep, s);
       else if (inv)
-        launch_sell_c<T, false, true>(sell, t, x, inv, y, st, s);
+        launch_sell_c<T, false, true>(sell, t, x, inv, y, st, rep, s);
       else
-        launch_sell_c<T, false, false>(sell, t, x, inv, y, st, s);
+        launch_sell_c<T, false, false>(sell, t, x, inv, y, st, rep, s);
       break;
     }
-    case 1: launch_spmv_l<T, 1>(nt != 0, A, t, x, inv, y, st, s); break;
-    case 2: launch_spmv_l<T, 2>(nt != 0, A, t, x, inv, y, st, s); break;
-    case 4: launch_spmv_l<T, 4>(nt != 0, A, t, x, inv, y, st, s); break;
-    case 16: launch_spmv_l<T, 16>(nt != 0, A, t, x, inv, y, st, s); break;
-    default: launch_spmv_l<T, 8>(nt != 0, A, t, x, inv, y, st, s); break;
+    case 1: launch_spmv_l<T, 1>(nt != 0, A, t, x, inv, y, st, rep, s); break;
+    case 2: launch_spmv_l<T, 2>(nt != 0, A, t, x, inv, y, st, rep, s); break;
+    case 4: launch_spmv_l<T, 4>(nt != 0, A, t, x, inv, y, st, rep, s); break;
+    case 16: launch_spmv_l<T, 16>(nt != 0, A, t, x, inv, y, st, rep, s); break;
+    default: launch_spmv_l<T, 8>(nt != 0, A, t, x, inv, y, st, rep, s); break;
   }
 }
 
@@ -1448,10 +1465,11 @@ __global__ void __launch_bounds__(kWave) k_build_y(KState* st, int m) {
 // (Batch as in k_maxpy_norm)
 template <class T, class X, int R, bool Batch>
 __global__ void __launch_bounds__(kBlock) k_update_x(const T* __restrict__ V, size_t ld, Tiles t, X* __restrict__ x,
-                                                     const KState* st, const int* __restrict__ xrow) {
+                                                     const KState* st, const int* __restrict__ xrow, int rhs_n) {
   using S = GsShape<T, R>;
   int a, e, c;
   t.range(blockIdx.x, a, e, c);
+  const size_t off = static_cast<size_t>(c) * rhs_n;  // as in k_residual_pc
   const KState* sc = st + c;
   const int nk = *reinterpret_cast<const int*>(&sc->pad);
   if (nk == 0) return;
@@ -1480,7 +1498,7 @@ __global__ void __launch_bounds__(kBlock) k_update_x(const T* __restrict__ V, si
 #pragma unroll
     for (int u = 0; u < S::VW; ++u)
       if (i0 + u < end) {
-        const size_t r = xrow ? static_cast<size_t>(xrow[i0 + u]) : i0 + u;
+        const size_t r = xrow ? off + static_cast<size_t>(xrow[i0 + u - off]) : i0 + u;
         x[r] = static_cast<X>(static_cast<double>(x[r]) + sacc[u]);
       }
   }
@@ -1496,10 +1514,17 @@ template <class T, class X>
 __global__ void __launch_bounds__(kBlock) k_residual_pc(CsrView<X> A, Tiles t, const X* __restrict__ b,
                                                         const X* __restrict__ x, const X* __restrict__ inv,
                                                         T* __restrict__ v0, double* partial, int zero_guess,
-                                                        const KState* st, const int* __restrict__ vpos) {
+                                                        const KState* st, const int* __restrict__ vpos, int rhs_n) {
   int a, e, c;
   t.range(blockIdx.x, a, e, c);
   if (st[c].done) return;
+  // several right-hand sides of one matrix: case c's vectors start at c rhs_n
+  const int off = c * rhs_n;
+  a -= off;
+  e -= off;
+  b += off;
+  x += off;
+  v0 += off;
   __shared__ double lds[kBlock / kWave];
   double nrm = 0.0;
   for (int i = a + threadIdx.x; i < e; i += kBlock) {
@@ -1535,10 +1560,14 @@ __global__ void __launch_bounds__(kBlock) k_jacobi_mixed(CsrView<double> A, doub
 // ---- partial ||M^-1 b||^2 per tile (reference norm for a nonzero guess)
 template <class T>
 __global__ void __launch_bounds__(kBlock) k_pc_norm(Tiles t, const T* __restrict__ b, const T* __restrict__ inv,
-                                                    double* partial, const KState* st) {
+                                                    double* partial, const KState* st, int rhs_n = 0) {
   int a, e, c;
   t.range(blockIdx.x, a, e, c);
   if (st[c].done) return;
+  const int off = c * rhs_n;
+  a -= off;
+  e -= off;
+  b += off;
   __shared__ double lds[kBlock / kWave];
   double nrm = 0.0;
   for (int i = a + threadIdx.x; i < e; i += kBlock) {
@@ -1847,11 +1876,11 @@ struct Dispatch {
   }
   template <int R, class X>
   static void update_r(const T* V, size_t ld, const Tiles& t, X* x, const KState* st, const int* xrow,
-                       hipStream_t s) {
+                       int rhs_n, hipStream_t s) {
     if (t.ntile < kBatchTiles)
-      hipLaunchKernelGGL((k_update_x<T, X, R, true>), dim3(t.ntile), dim3(kBlock), 0, s, V, ld, t, x, st, xrow);
+      hipLaunchKernelGGL((k_update_x<T, X, R, true>), dim3(t.ntile), dim3(kBlock), 0, s, V, ld, t, x, st, xrow, rhs_n);
     else
-      hipLaunchKernelGGL((k_update_x<T, X, R, false>), dim3(t.ntile), dim3(kBlock), 0, s, V, ld, t, x, st, xrow);
+      hipLaunchKernelGGL((k_update_x<T, X, R, false>), dim3(t.ntile), dim3(kBlock), 0, s, V, ld, t, x, st, xrow, rhs_n);
   }
   static void mdot(int R, const T* V, size_t ld, const Tiles& t, int it, double* partial, int pstride,
                    KState* st, hipStream_t s) {
@@ -1875,13 +1904,13 @@ struct Dispatch {
   }
   template <class X>
   static void update(int R, const T* V, size_t ld, const Tiles& t, X* x, const KState* st, const int* xrow,
-                     hipStream_t s) {
+                     int rhs_n, hipStream_t s) {
     switch (R) {
-      case 16: update_r<16>(V, ld, t, x, st, xrow, s); break;
-      case 8: update_r<8>(V, ld, t, x, st, xrow, s); break;
-      case 4: update_r<4>(V, ld, t, x, st, xrow, s); break;
-      case 2: update_r<2>(V, ld, t, x, st, xrow, s); break;
-      default: update_r<1>(V, ld, t, x, st, xrow, s); break;
+      case 16: update_r<16>(V, ld, t, x, st, xrow, rhs_n, s); break;
+      case 8: update_r<8>(V, ld, t, x, st, xrow, rhs_n, s); break;
+      case 4: update_r<4>(V, ld, t, x, st, xrow, rhs_n, s); break;
+      case 2: update_r<2>(V, ld, t, x, st, xrow, rhs_n, s); break;
+      default: update_r<1>(V, ld, t, x, st, xrow, rhs_n, s); break;
     }
   }
 };
@@ -1977,13 +2006,16 @@ KResult gmres(const CsrView<T>& A, const CsrView<X>& Ares, const X* b, X* x, con
   const int n = A.n;
   const int m = o.restart < 1 ? 1 : (o.restart > kMaxRestart ? kMaxRestart : o.restart);
   if (m > w.mmax) throw std::invalid_argument("gmres: restart above workspace size");
-  if (Ares.n != n || w.n != n) throw std::invalid_argument("gmres: operator sizes differ");
-  const size_t ld = w.ld ? w.ld : static_cast<size_t>(n);
+  // rep right-hand sides of one matrix: cases whose rows are n each
+  const int rep = w.rep, rhs_n = rep > 1 ? n : 0;
+  if (Ares.n != n || w.n != n * rep || (rep > 1 && w.ncase != rep))
+    throw std::invalid_argument("gmres: operator sizes differ");
+  const size_t ld = w.ld ? w.ld : static_cast<size_t>(w.n);
   const int R = w.rows ? w.rows : pick_r(n, sizeof(T));
   const SellView<T> sell = sell_of<T>(w, n);
   const int L = (w.lanes == 0 && !sell.ptr) ? 8 : w.lanes;
   const Tiles& tl = w.tiles[log2_r(R)];
-  if (tl.tile != kBlock * R || tl.n != n) throw std::runtime_error("gmres: tile table missing");
+  if (tl.tile != kBlock * R || tl.n != w.n) throw std::runtime_error("gmres: tile table missing");
   const int nc = w.ncase;
   // the inner order (mixed, no ILU): the FP32 basis, the matrix A and its
   // SELL copies are by position (each case of a batch keeps its own position
@@ -1992,8 +2024,8 @@ KResult gmres(const CsrView<T>& A, const CsrView<X>& Ares, const X* b, X* x, con
   const bool ordered = w.ord_pos != nullptr;
   if (ordered && (!mixed || o.pc == S355_PC_ILU0 || !w.ord_row))
     throw std::invalid_argument("gmres: the inner order serves mixed solves without ILU(0)");
-  // ILU sweeps skip their work only for a single system
-  const KState* ilu_st = nc == 1 ? w.st : nullptr;
+  // ILU sweeps skip finished work by right-hand side, in a batch never
+  const KState* ilu_st = nc == rep ? w.st : nullptr;
   T* V = static_cast<T*>(w.V);
   T* inv = nullptr;
   const X* invr = nullptr;
@@ -2003,17 +2035,18 @@ KResult gmres(const CsrView<T>& A, const CsrView<X>& Ares, const X* b, X* x, con
     inv = static_cast<T*>(w.pcinv);
     if constexpr (mixed) {
       if (!inv_x) throw std::invalid_argument("gmres: mixed Jacobi needs an FP64 inverse buffer");
-      hipLaunchKernelGGL(k_jacobi_mixed, dim3(grid_for(n)), dim3(kBlock), 0, s, Ares, inv_x, inv, w.ord_pos);
+      if (!w.prepared)
+        hipLaunchKernelGGL(k_jacobi_mixed, dim3(grid_for(n)), dim3(kBlock), 0, s, Ares, inv_x, inv, w.ord_pos);
       invr = inv_x;
       if (w.pc_folded) inv = nullptr;  // A is M^-1 A already
     } else {
-      hipLaunchKernelGGL((k_jacobi_setup<T>), dim3(grid_for(n)), dim3(kBlock), 0, s, A, inv);
+      if (!w.prepared) hipLaunchKernelGGL((k_jacobi_setup<T>), dim3(grid_for(n)), dim3(kBlock), 0, s, A, inv);
       invr = inv;
     }
   } else if (o.pc == S355_PC_ILU0) {
     if (!w.ilu || !w.lu || !w.r) throw std::invalid_argument("gmres: ILU(0) workspace missing");
     lu = static_cast<T*>(w.lu);
-    ilu_factor(A, A.nnz, *w.ilu, lu, s, &w);
+    if (!w.prepared) ilu_factor(A, A.nnz, *w.ilu, lu, s, &w);
   } else if (o.pc != S355_PC_NONE) {
     throw std::invalid_argument("gmres: unknown preconditioner");
   }
@@ -2032,9 +2065,9 @@ KResult gmres(const CsrView<T>& A, const CsrView<X>& Ares, const X* b, X* x, con
       }
       ilu_apply(A, *w.ilu, lu, bt, V, ilu_st, s, nullptr, &w);
       hipLaunchKernelGGL((k_pc_norm<T>), dim3(tl.ntile), dim3(kBlock), 0, s, tl, V, static_cast<const T*>(nullptr),
-                         w.partial, w.st);
+                         w.partial, w.st, rhs_n);
     } else {
-      hipLaunchKernelGGL((k_pc_norm<X>), dim3(tl.ntile), dim3(kBlock), 0, s, tl, b, invr, w.partial, w.st);
+      hipLaunchKernelGGL((k_pc_norm<X>), dim3(tl.ntile), dim3(kBlock), 0, s, tl, b, invr, w.partial, w.st, rhs_n);
     }
     hipLaunchKernelGGL(k_snorm_final, dim3(nc), dim3(kBlock), 0, s, w.partial, tl, w.st);
   } else {
@@ -2044,13 +2077,13 @@ KResult gmres(const CsrView<T>& A, const CsrView<X>& Ares, const X* b, X* x, con
     if (lu) {
       hipLaunchKernelGGL((k_residual_pc<T, X>), dim3(tl.ntile), dim3(kBlock), 0, s, Ares, tl, b, x,
                          static_cast<const X*>(nullptr), tmp, w.partial, gz_c ? 1 : 0, w.st,
-                         static_cast<const int*>(nullptr));
+                         static_cast<const int*>(nullptr), rhs_n);
       ilu_apply(A, *w.ilu, lu, tmp, V, ilu_st, s, w.graphs, &w);
       hipLaunchKernelGGL((k_pc_norm<T>), dim3(tl.ntile), dim3(kBlock), 0, s, tl, V, static_cast<const T*>(nullptr),
-                         w.partial, w.st);
+                         w.partial, w.st, rhs_n);
     } else {
       hipLaunchKernelGGL((k_residual_pc<T, X>), dim3(tl.ntile), dim3(kBlock), 0, s, Ares, tl, b, x, invr, V,
-                         w.partial, gz_c ? 1 : 0, w.st, w.ord_pos);
+                         w.partial, gz_c ? 1 : 0, w.st, w.ord_pos, rhs_n);
     }
     hipLaunchKernelGGL(k_restart_finalize, dim3(nc), dim3(kBlock), 0, s, w.partial, tl, w.st, first_c ? 1 : 0,
                        zero_guess ? 1 : 0, mixed ? 1 : 0);
@@ -2083,9 +2116,9 @@ KResult gmres(const CsrView<T>& A, const CsrView<X>& Ares, const X* b, X* x, con
     } else {
       if (rec) S355_HIP(hipEventRecord(e0, s));
       if (lu)
-        launch_spmv<T>(L, w.nt, A, sell, tl, V + it * ld, static_cast<const T*>(nullptr), tmp, w.st, s);
+        launch_spmv<T>(L, w.nt, A, sell, tl, V + it * ld, static_cast<const T*>(nullptr), tmp, w.st, s, rep);
       else
-        launch_spmv<T>(L, w.nt, A, sell, tl, V + it * ld, inv, V + (it + 1) * ld, w.st, s);
+        launch_spmv<T>(L, w.nt, A, sell, tl, V + it * ld, inv, V + (it + 1) * ld, w.st, s, rep);
       if (rec) S355_HIP(hipEventRecord(e1, s));
       if (lu) ilu_apply(A, *w.ilu, lu, tmp, V + (it + 1) * ld, ilu_st, s, w.graphs, &w);
       Dispatch<T>::mdot(R, V, ld, tl, it, w.partial, pstride, w.st, s);
@@ -2098,7 +2131,7 @@ KResult gmres(const CsrView<T>& A, const CsrView<X>& Ares, const X* b, X* x, con
   auto enqueue_end = [&] {
     flush_fin();
     hipLaunchKernelGGL(k_build_y, dim3(nc), dim3(kWave), 0, s, w.st, m);
-    Dispatch<T>::update(R, V, ld, tl, x, w.st, w.ord_row, s);
+    Dispatch<T>::update(R, V, ld, tl, x, w.st, w.ord_row, rhs_n, s);
     hipLaunchKernelGGL(k_cycle_end, dim3(grid_for(nc)), dim3(kBlock), 0, s, w.st, nc, mixed ? 1 : 0);
     S355_LAUNCH_CHECK();
   };
@@ -2124,7 +2157,8 @@ KResult gmres(const CsrView<T>& A, const CsrView<X>& Ares, const X* b, X* x, con
                                           static_cast<uintptr_t>(w.sell2 + 1), sizeof(T), sizeof(X),
                                           reinterpret_cast<uintptr_t>(w.ord_row),
                                           reinterpret_cast<uintptr_t>(sell.col16),
-                                          static_cast<uintptr_t>(first_c), static_cast<uintptr_t>(zero_guess), 0};
+                                          static_cast<uintptr_t>(rep), static_cast<uintptr_t>(first_c),
+                                          static_cast<uintptr_t>(zero_guess), 0};
       // segment: 0 a whole cycle, 1 the first ksplit steps, 2 the rest and
       // the end, 3 the end alone
       auto launch = [&](uintptr_t seg, const std::function<void()>& record) {

@@ -224,8 +224,13 @@ struct SpmvTimer {
 // type share one launch per kernel: their rows are consecutive, their states
 // are st[0..ncase), and tiles[k] splits the rows into tiles of kBlock * 2^k
 // rows that never straddle two cases.
+//
+// rep > 1: the cases are rep right-hand sides of one matrix of n / rep rows, the
+// vectors (basis, r, ilu_zl, ilu_zu) one after the other; the matrix, its copies
+// and the preconditioner exist once.
 struct KWork {
-  int n = 0, mmax = 0, ncase = 1;
+  int n = 0, mmax = 0, ncase = 1, rep = 1;
+  bool prepared = false;    // the preconditioner in the workspace is A's already
   size_t ld = 0;            // column stride of V (n rounded up to 8; 0 = n)
   Tiles tiles[5];
   void* V = nullptr;        // (mmax + 1) * ld elements of T
@@ -264,6 +269,14 @@ struct KWork {
   KHeader* host = nullptr;  // pinned, ncase headers
   std::vector<KResult>* per_case = nullptr;  // filled by a solve when set
 };
+
+// Up to this many rows the momentum components are solved together: the launches
+// and level groups of small systems are shared, larger ones are bound by the
+// vectors' bytes, and three bases of theirs would take gigabytes.  Momentum phase
+// one after the other and together: GMRES(30) + ILU(0), 331,776 tetrahedra, FP64
+// 8.4 -> 4.7 ms; GMRES(50) + Jacobi, 748,410 rows, mixed 6.6 -> 5.4 ms (2.5 ms of
+// both are the copies of the fields from and to the host).
+constexpr int kTripleRows = 1 << 20;
 
 // Buffers of the iterative-refinement solve (mixed precision).
 struct IrWork {
