@@ -717,6 +717,7 @@ void Context::ensure_ilu() {
     w.slots = p.col.size();
     w.len = upload(allocs_, p.len, stream);
     w.slot0 = upload(allocs_, p.slot0, stream);
+    w.lanes = upload(allocs_, p.lanes, stream);
     w.stride = upload(allocs_, p.stride, stream);
     w.col = upload(allocs_, p.col, stream);
     w.src = upload(allocs_, p.src, stream);

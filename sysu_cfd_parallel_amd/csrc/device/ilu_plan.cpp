@@ -153,6 +153,7 @@ IluPlan ilu_plan(int n, const int* rowptr, const int* col, const int* diag, bool
   out.group.assign(1, 0);
   out.len.resize(n);
   out.slot0.resize(n);
+  out.lanes.resize(n);
   out.stride.resize(n);
   out.depth.resize(n);
   for (int g = 0; g < ngroup; ++g) {
@@ -160,16 +161,18 @@ IluPlan ilu_plan(int n, const int* rowptr, const int* col, const int* diag, bool
       const long k = static_cast<long>(g) * kTermClasses + c;
       const int p0 = kptr[k], nr = kptr[k + 1] - p0;
       if (nr == 0) continue;
+      const int lanes = kTermLanes[c], batch = kTermBatch * lanes;
       if (c + 1 < kTermClasses)
         width[k] = kTermWidth[c];
       else
-        width[k] = (width[k] + kTermBatch - 1) / kTermBatch * kTermBatch;
+        width[k] = (width[k] + batch - 1) / batch * batch;
       out.subs.push_back(IluSub{slots, p0, nr, width[k], c});
       if (slots + static_cast<long>(width[k]) * nr > kMost)
         throw std::invalid_argument("ILU(0) sweep slots above 32-bit indices");
       for (int p = p0; p < p0 + nr; ++p) {
-        out.slot0[p] = static_cast<int>(slots + (p - p0));
-        out.stride[p] = nr;
+        out.slot0[p] = static_cast<int>(slots + static_cast<long>(p - p0) * lanes);
+        out.lanes[p] = lanes;
+        out.stride[p] = nr * lanes;
       }
       slots += static_cast<long>(width[k]) * nr;
     }
@@ -185,7 +188,7 @@ IluPlan ilu_plan(int n, const int* rowptr, const int* col, const int* diag, bool
           out.len[p] = count[i];
           out.depth[p] = dep[i];
           for (int u = 0; u < sub.width; ++u) {
-            const size_t at = static_cast<size_t>(sub.off) + static_cast<size_t>(u) * sub.nrows + k;
+            const int at = out.slot(p, u);
             if (u < count[i]) {
               const int c = code[start[i] + u];
               out.col[at] = c < n ? out.pos[c] : n + out.pos[c - n];
@@ -232,8 +235,8 @@ IluPlan ilu_plan(int n, const int* rowptr, const int* col, const int* diag, bool
           const int pj = out.pos[j];
           out.p[x0] = x;
           for (int y = -1; y < count[j]; ++y, ++at, ++from) {
-            out.r[at] = out.slot0[pi] + pr[from] * out.stride[pi];
-            out.q[at] = pq[from] < 0 ? -1 - pj : out.slot0[pj] + pq[from] * out.stride[pj];
+            out.r[at] = out.slot(pi, pr[from]);
+            out.q[at] = pq[from] < 0 ? -1 - pj : out.slot(pj, pq[from]);
           }
           out.uptr[++x0] = static_cast<int>(at);
         }

@@ -23,26 +23,27 @@ namespace s355 {
 // bytes, and merged rows read more of them) or where a row could pass
 // kMergeTerms terms (counted without looking for equal ones).  Pressure solves
 // (CG, 331,776 tetrahedra, FP64, 54 levels; mixed GMRES, 310,000 hexahedra, 134
-// levels) by levels, rows and terms: no merging 131.7 and 162.3 ms; 2, 49152,
-// 64: 98.7 and 112.1; 4, 49152, 64: 75.9 and 94.2; 4, 24576, 64: 82.5 and 94.3;
-// 6, 49152, 96: 72.3 and 84.7; 6, 131072, 160: 71.9 and 81.2; 8, 131072, 300:
-// 74.6 and 74.4.  With 6, 65536, 96 and the row's own input out of the terms:
-// 64.8 and 81.8.  Each case of a
-// batch is grouped by its own rows, so it sums the same terms in the same
-// order as alone.
-constexpr int kMergeLevels = 6;
-constexpr int kMergeTerms = 96;
+// levels), a k-epsilon step (98,304 tetrahedra) and a momentum phase (331,776, a
+// factorisation for 9 steps) by levels, rows and terms, in ms: no merging 131.7,
+// 162.3, 90.6, 13.2; 6, 65536, 96: 60.2, 62.3, 39.6, 4.68; 8, 65536, 160: 55.6,
+// 56.0, 38.0, 4.76; 8, 65536, 300: 55.2, 51.4, 38.9, 4.80; 12, 65536, 300: 52.8,
+// 50.4, 37.6, 5.30; 16, 65536, 1000: 51.9, 48.4, 40.2, 6.31.
+constexpr int kMergeLevels = 8;
+constexpr int kMergeTerms = 200;
 constexpr int kMergeRows = 65536;
 // Rows of a launch come in classes of term counts, each padded to a width the
-// kernel is compiled for; the last takes what is longer, padded to batches.
-constexpr int kTermWidth[] = {3, 6, 10, 15, 22, 32, 1 << 30};
+// kernel is compiled for.  A row of many terms is shared by 4 or 16 lanes, so
+// that no lane's chain of loads is longer than one batch; the last class takes
+// what is longer still, in batches of kTermBatch per lane.
+constexpr int kTermWidth[] = {3, 6, 10, 15, 32, 64, 1 << 30};
+constexpr int kTermLanes[] = {1, 1, 1, 1, 4, 4, 16};
 constexpr int kTermClasses = 7;
 constexpr int kNarrowClasses = 3;  // a launch without wider rows takes a kernel of fewer registers
 constexpr int kTermBatch = 16;
 
-// rows of one group and class of term counts
+// rows of one group and class of term counts, lanes = kTermLanes[cls] to a row
 struct IluSub {
-  long off;  // first slot; term u of the k-th row at off + u nrows + k
+  long off;  // first slot; term u of the k-th row at off + (u / lanes) lanes nrows + k lanes + u % lanes
   int p0, nrows, width, cls;
 };
 
@@ -54,7 +55,9 @@ struct IluPlan {
   std::vector<int> group;    // group g: subs group[g] .. group[g + 1] - 1
   std::vector<int> len;      // terms per position (the row's own input, o_i r_i, is not among them)
   std::vector<int> depth;    // per position: 0 where no entry refers to the row's own group
-  std::vector<int> slot0, stride;  // per position: its first slot, the distance of its terms
+  // per position: its first slot, its lanes, the distance of its terms of one lane
+  std::vector<int> slot0, lanes, stride;
+  int slot(int q, int u) const { return slot0[q] + u / lanes[q] * stride[q] + u % lanes[q]; }
   // per slot: buf index (padding: the row's own input), and where its
   // coefficient starts from: the CSR entry a_ij (coefficient -a_ij) or -1 (0)
   std::vector<int> col, src;

@@ -84,7 +84,7 @@ __global__ void __launch_bounds__(kBlock) k_ilu_factor(T* __restrict__ lu, IluSt
 // slots load before any is used and all its gathers before any is added: the
 // rows of a launch come in classes of term counts, each a run of workgroups
 // compiled for its padded width, its loads unconditional (guarded ones wait
-// for each other).  A longer row than the widest class takes batches.
+// for each other), a long row shared by several lanes.
 struct IluLaunch {
   // per class; blk0: its first workgroup (empty classes: nrows 0, where the
   // next class starts)
@@ -92,20 +92,21 @@ struct IluLaunch {
   int p0[kTermClasses], nrows[kTermClasses], width[kTermClasses], blk0[kTermClasses];
 };
 
-template <class T, int W>
-__device__ __forceinline__ T ilu_row(const int* __restrict__ col, const T* __restrict__ coef, const T* buf, size_t q0,
-                                     int nrows, int L, T s) {
+// the sum of a row's terms u = lane, lane + Lanes, ... (W of them, slots `step` apart)
+template <class T, int W, int Lanes>
+__device__ __forceinline__ T ilu_terms(const int* __restrict__ col, const T* __restrict__ coef, const T* buf, size_t q0,
+                                       int step, int lane, int L, T s) {
   T v[W], x[W];
   int c[W];
 #pragma unroll
   for (int u = 0; u < W; ++u) {
-    v[u] = coef[q0 + static_cast<size_t>(u) * nrows];
-    c[u] = col[q0 + static_cast<size_t>(u) * nrows];
+    v[u] = coef[q0 + static_cast<size_t>(u) * step];
+    c[u] = col[q0 + static_cast<size_t>(u) * step];
   }
 #pragma unroll
   for (int u = 0; u < W; ++u) x[u] = buf[c[u]];  // padding: the row's own input
 #pragma unroll
-  for (int u = 0; u < W; ++u) s = u < L ? s + v[u] * x[u] : s;
+  for (int u = 0; u < W; ++u) s = u * Lanes + lane < L ? s + v[u] * x[u] : s;
   return s;
 }
 
@@ -129,28 +130,44 @@ __global__ void __launch_bounds__(kBlock) k_ilu_group(IluLaunch g, const int* __
       blk0 = g.blk0[c];
       off = g.off[c];
     }
-  const int k = (blk - blk0) * static_cast<int>(blockDim.x) + threadIdx.x;
-  if (k >= nrows) return;
+  int lanes = 1;
+  if constexpr (Wide) lanes = cls < 4 ? 1 : cls < 6 ? 4 : 16;
+  const int i = (blk - blk0) * static_cast<int>(blockDim.x) + threadIdx.x;
+  const int k = i / lanes, lane = i % lanes;
+  if (k >= nrows) return;  // the lanes of a row together
   if (st && st[blockIdx.y].reason) return;
-  const int p = p0 + k, L = len[p];
-  const size_t q0 = static_cast<size_t>(off) + k;
-  T z = buf[p];
-  if (own) z *= own[p];
+  const int p = p0 + k, L = len[p], step = nrows * lanes;
+  const size_t q0 = static_cast<size_t>(off) + i;
+  T z = T(0);
+  if (lane == 0) {
+    z = buf[p];
+    if (own) z *= own[p];
+  }
   if (cls == 0) {
-    z = ilu_row<T, kTermWidth[0]>(col, coef, buf, q0, nrows, L, z);
+    z = ilu_terms<T, 3, 1>(col, coef, buf, q0, step, lane, L, z);
   } else if (cls == 1) {
-    z = ilu_row<T, kTermWidth[1]>(col, coef, buf, q0, nrows, L, z);
+    z = ilu_terms<T, 6, 1>(col, coef, buf, q0, step, lane, L, z);
   } else if (cls == 2) {
-    z = ilu_row<T, kTermWidth[2]>(col, coef, buf, q0, nrows, L, z);
+    z = ilu_terms<T, 10, 1>(col, coef, buf, q0, step, lane, L, z);
   } else if constexpr (Wide) {
     switch (cls) {
-      case 3: z = ilu_row<T, kTermWidth[3]>(col, coef, buf, q0, nrows, L, z); break;
-      case 4: z = ilu_row<T, kTermWidth[4]>(col, coef, buf, q0, nrows, L, z); break;
-      case 5: z = ilu_row<T, kTermWidth[5]>(col, coef, buf, q0, nrows, L, z); break;
+      case 3: z = ilu_terms<T, 15, 1>(col, coef, buf, q0, step, lane, L, z); break;
+      case 4: z = ilu_terms<T, 8, 4>(col, coef, buf, q0, step, lane, L, z); break;
+      case 5: z = ilu_terms<T, 16, 4>(col, coef, buf, q0, step, lane, L, z); break;
       default:
-        for (int j = 0; j < width; j += kTermBatch)
-          z = ilu_row<T, kTermBatch>(col, coef, buf, q0 + static_cast<size_t>(j) * nrows, nrows, L - j, z);
+        for (int j = 0; j < width; j += 16 * kTermBatch)
+          z = ilu_terms<T, kTermBatch, 16>(col, coef, buf, q0 + static_cast<size_t>(j / 16) * step, step, lane, L - j, z);
         break;
+    }
+    if (lanes > 1) {
+      // the lanes' sums, pairs first
+      z += __shfl_xor(z, 1, kWave);
+      z += __shfl_xor(z, 2, kWave);
+      if (lanes == 16) {
+        z += __shfl_xor(z, 4, kWave);
+        z += __shfl_xor(z, 8, kWave);
+      }
+      if (lane) return;
     }
   }
   buf[static_cast<size_t>(n) + p] = z;
@@ -161,20 +178,22 @@ __global__ void __launch_bounds__(kBlock) k_ilu_group(IluLaunch g, const int* __
 // (own: 1 / pivot in the upper sweep)
 template <class T, bool Upper>
 __global__ void __launch_bounds__(kBlock) k_ilu_coef(int n, const int* __restrict__ len, const int* __restrict__ slot0,
-                                                     const int* __restrict__ stride, const int* __restrict__ src,
-                                                     const int* __restrict__ dsrc, const T* __restrict__ lu,
-                                                     T* __restrict__ coef, T* __restrict__ own) {
+                                                     const int* __restrict__ lanes, const int* __restrict__ stride,
+                                                     const int* __restrict__ src, const int* __restrict__ dsrc,
+                                                     const T* __restrict__ lu, T* __restrict__ coef,
+                                                     T* __restrict__ own) {
   const int p = blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= n) return;
-  const int L = len[p];
-  const size_t q0 = slot0[p], step = stride[p];
+  const int L = len[p], nl = lanes[p], step = stride[p];
+  const size_t q0 = slot0[p];
   // dsrc < 0: a row below depth 0, divided by its pivot once its terms are complete
   const int dp = Upper ? dsrc[p] : -1;
   const T d = dp >= 0 ? lu[dp] : T(1);
   for (int u = 0; u < L; ++u) {
-    const int e = src[q0 + u * step];
+    const size_t at = q0 + static_cast<size_t>(u / nl) * step + u % nl;
+    const int e = src[at];
     const T c = e >= 0 ? -lu[e] : T(0);
-    coef[q0 + u * step] = dp >= 0 ? c / d : c;
+    coef[at] = dp >= 0 ? c / d : c;
   }
   if (dp >= 0) own[p] = T(1) / d;
 }
@@ -186,9 +205,9 @@ __global__ void __launch_bounds__(kBlock) k_ilu_merge(int k0, int nrows, const i
                                                       const int* __restrict__ sptr, const int* __restrict__ sp,
                                                       const int* __restrict__ uptr, const int* __restrict__ r,
                                                       const int* __restrict__ q, const int* __restrict__ len,
-                                                      const int* __restrict__ slot0, const int* __restrict__ stride,
-                                                      const int* __restrict__ dsrc, const T* __restrict__ lu, T* coef,
-                                                      T* own) {
+                                                      const int* __restrict__ slot0, const int* __restrict__ lanes,
+                                                      const int* __restrict__ stride, const int* __restrict__ dsrc,
+                                                      const T* __restrict__ lu, T* coef, T* own) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= nrows) return;
   const int k = k0 + t, p = later[k];
@@ -201,8 +220,9 @@ __global__ void __launch_bounds__(kBlock) k_ilu_merge(int k0, int nrows, const i
   }
   if constexpr (Upper) {
     const T d = lu[-1 - dsrc[p]];
-    const size_t q0 = slot0[p], step = stride[p];
-    for (int u = 0; u < len[p]; ++u) coef[q0 + u * step] /= d;
+    const int nl = lanes[p], step = stride[p];
+    const size_t q0 = slot0[p];
+    for (int u = 0; u < len[p]; ++u) coef[q0 + static_cast<size_t>(u / nl) * step + u % nl] /= d;
     own[p] = T(1) / d;
   }
 }
@@ -279,14 +299,14 @@ __global__ void __launch_bounds__(kBlock) k_gather(const int* __restrict__ src, 
 // the coefficients of one sweep from the factors lu
 template <class T, bool Upper>
 void ilu_coefficients(const IluSweep& w, const T* lu, T* coef, T* own, hipStream_t s) {
-  hipLaunchKernelGGL((k_ilu_coef<T, Upper>), dim3(grid_for(w.n)), dim3(kBlock), 0, s, w.n, w.len, w.slot0, w.stride,
-                     w.src, w.dsrc, lu, coef, own);
+  hipLaunchKernelGGL((k_ilu_coef<T, Upper>), dim3(grid_for(w.n)), dim3(kBlock), 0, s, w.n, w.len, w.slot0, w.lanes,
+                     w.stride, w.src, w.dsrc, lu, coef, own);
   for (size_t d = 0; d + 1 < w.dptr.size(); ++d) {
     const int nr = w.dptr[d + 1] - w.dptr[d];
     if (nr == 0) continue;
     const int b = level_block(nr);
     hipLaunchKernelGGL((k_ilu_merge<T, Upper>), dim3(grid_for(nr, b)), dim3(b), 0, s, w.dptr[d], nr, w.later, w.sptr,
-                       w.p, w.uptr, w.r, w.q, w.len, w.slot0, w.stride, w.dsrc, lu, coef, own);
+                       w.p, w.uptr, w.r, w.q, w.len, w.slot0, w.lanes, w.stride, w.dsrc, lu, coef, own);
   }
 }
 
@@ -313,7 +333,7 @@ void ilu_sweep(const IluSweep& w, const T* coef, const T* own, T* buf, const KSt
   for (size_t g = 0; g + 1 < w.group.size(); ++g) {
     IluLaunch a{};
     int rows = 0, blocks = 0, k = w.group[g];
-    for (int x = k; x < w.group[g + 1]; ++x) rows += w.subs[x].nrows;
+    for (int x = k; x < w.group[g + 1]; ++x) rows += w.subs[x].nrows * kTermLanes[w.subs[x].cls];
     const int b = level_block(rows);
     for (int c = 0; c < kTermClasses; ++c) {
       a.blk0[c] = blocks;
@@ -323,7 +343,7 @@ void ilu_sweep(const IluSweep& w, const T* coef, const T* own, T* buf, const KSt
       a.p0[c] = u.p0;
       a.nrows[c] = u.nrows;
       a.width[c] = u.width;
-      blocks += grid_for(u.nrows, b);
+      blocks += grid_for(static_cast<long>(u.nrows) * kTermLanes[c], b);
     }
     const bool wide = w.subs[w.group[g + 1] - 1].cls >= kNarrowClasses;
     hipLaunchKernelGGL((wide ? k_ilu_group<T, true> : k_ilu_group<T, false>), dim3(blocks, rep), dim3(b), 0, s, a, w.len,

@@ -137,7 +137,7 @@ struct IluSweep {
   std::vector<IluSub> subs;
   std::vector<int> group, dptr;
   size_t slots = 0;
-  const int *len = nullptr, *slot0 = nullptr, *stride = nullptr, *col = nullptr, *src = nullptr;
+  const int *len = nullptr, *slot0 = nullptr, *lanes = nullptr, *stride = nullptr, *col = nullptr, *src = nullptr;
   const int *later = nullptr, *sptr = nullptr, *p = nullptr, *uptr = nullptr, *r = nullptr, *q = nullptr;
   // upper sweep: CSR position of the pivot of the row at each position at
   // depth 0, and -1 minus it below

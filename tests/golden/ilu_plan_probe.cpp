@@ -16,7 +16,7 @@ extern "C" int probe_sweep(int n, const int* rowptr, const int* col, const int* 
   const IluPlan p = s355::ilu_plan(n, rowptr, col, diag, upper != 0, std::vector<int>(order, order + n),
                                    std::vector<int>(cases, cases + ncase + 1), levels, rows);
   std::vector<double> c(p.col.size(), 0.0), own(n, 1.0);
-  auto at = [&](int q, int u) { return static_cast<size_t>(p.slot0[q]) + static_cast<size_t>(u) * p.stride[q]; };
+  auto at = [&](int q, int u) { return static_cast<size_t>(p.slot(q, u)); };
   auto scale = [&](int q) {
     if (!upper) return;
     const double d = lu[diag[p.rows[q]]];
@@ -42,11 +42,16 @@ extern "C" int probe_sweep(int n, const int* rowptr, const int* col, const int* 
       const IluSub& sub = p.subs[s];
       widest = sub.width > widest ? sub.width : widest;
       if (s > p.group[g] && sub.cls <= p.subs[s - 1].cls) ++bad;
-      if (sub.cls + 1 < s355::kTermClasses ? sub.width != s355::kTermWidth[sub.cls] : sub.width % s355::kTermBatch)
+      const int lanes = s355::kTermLanes[sub.cls];
+      if (sub.cls + 1 < s355::kTermClasses ? sub.width != s355::kTermWidth[sub.cls]
+                                           : sub.width % (lanes * s355::kTermBatch))
         ++bad;
+      const bool even = sub.cls < 4 || sub.cls == 6 || sub.width % lanes == 0;
       for (int k = 0; k < sub.nrows; ++k) {
         const int q = sub.p0 + k;
-        if (p.slot0[q] != sub.off + k || p.stride[q] != sub.nrows || p.len[q] > sub.width) ++bad;
+        if (p.slot0[q] != sub.off + k * lanes || p.lanes[q] != lanes || p.stride[q] != sub.nrows * lanes ||
+            p.len[q] > sub.width || !even)
+          ++bad;
         double v = own[q] * buf[q];
         for (int u = 0; u < sub.width; ++u) {
           const int b = p.col[at(q, u)];

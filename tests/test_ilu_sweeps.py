@@ -67,7 +67,7 @@ def ip(a):
 
 
 @pytest.mark.parametrize("name", sorted(PATTERNS))
-@pytest.mark.parametrize("levels,rows", [(1, 65536), (2, 65536), (6, 65536), (6, 40), (4, 1)])
+@pytest.mark.parametrize("levels,rows", [(1, 65536), (2, 65536), (6, 65536), (8, 65536), (6, 40), (4, 1)])
 @pytest.mark.parametrize("upper", [0, 1])
 def test_sweep_plan_equals_the_triangular_solve(probe, name, levels, rows, upper):
     rng = np.random.default_rng(3)
