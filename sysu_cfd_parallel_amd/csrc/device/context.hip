@@ -8,8 +8,10 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <exception>
 #include <numeric>
 #include <stdexcept>
+#include <thread>
 
 #include "common.hpp"
 
@@ -697,18 +699,23 @@ void fill_info(const KResult& r, s355_solve_info* info) {
 
 void Context::ensure_ilu() {
   if (have_levels_) return;
-  {
-    std::vector<int> rows, sptr, sp, sd, su, sr, sq;
-    ilu_levels(dm.Nc, mesh.rowptr.data(), mesh.col.data(), mesh.diag.data(), rows, levels_.lptr);
-    ilu_steps(dm.Nc, mesh.rowptr.data(), mesh.col.data(), mesh.diag.data(), rows, sptr, sp, sd, su, sr, sq);
-    levels_.steps.ptr = upload(allocs_, sptr, stream);
-    levels_.steps.p = upload(allocs_, sp, stream);
-    levels_.steps.d = upload(allocs_, sd, stream);
-    levels_.steps.u = upload(allocs_, su, stream);
-    levels_.steps.r = upload(allocs_, sr, stream);
-    levels_.steps.q = upload(allocs_, sq, stream);
-    sync();  // host staging vectors go out of scope
-  }
+  // the factorisation's steps on a thread of their own, beside the sweeps' plans
+  std::vector<int> rows, sptr, sp, sd, su, sr, sq;
+  std::exception_ptr failed;
+  std::thread factor([&] {
+    try {
+      ilu_levels(dm.Nc, mesh.rowptr.data(), mesh.col.data(), mesh.diag.data(), rows, levels_.lptr);
+      ilu_steps(dm.Nc, mesh.rowptr.data(), mesh.col.data(), mesh.diag.data(), rows, sptr, sp, sd, su, sr, sq);
+    } catch (...) {
+      failed = std::current_exception();
+    }
+  });
+  struct Joined {
+    std::thread& t;
+    ~Joined() {
+      if (t.joinable()) t.join();
+    }
+  } joined{factor};
   auto put = [&](IluSweep& w, const IluPlan& p, bool up) {
     w.n = p.n;
     w.subs = p.subs;
@@ -751,6 +758,14 @@ void Context::ensure_ilu() {
     levels_.lpos = upload(allocs_, lower.pos, stream);
     levels_.l2u = upload(allocs_, l2u, stream);
     levels_.upos = upload(allocs_, upper.pos, stream);
+    factor.join();
+    if (failed) std::rethrow_exception(failed);
+    levels_.steps.ptr = upload(allocs_, sptr, stream);
+    levels_.steps.p = upload(allocs_, sp, stream);
+    levels_.steps.d = upload(allocs_, sd, stream);
+    levels_.steps.u = upload(allocs_, su, stream);
+    levels_.steps.r = upload(allocs_, sr, stream);
+    levels_.steps.q = upload(allocs_, sq, stream);
     sync();  // host staging vectors go out of scope
   }
   kwork_.lu = alloc<double>(dm.nnz);

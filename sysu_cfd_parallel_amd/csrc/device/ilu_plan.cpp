@@ -11,13 +11,6 @@ namespace {
 
 constexpr long kMost = 0x7fffffffL;
 
-// n ints without filling them
-struct Ints {
-  std::unique_ptr<int[]> p;
-  explicit Ints(size_t n) : p(new int[n ? n : 1]) {}
-  int& operator[](size_t i) { return p[i]; }
-};
-
 }  // namespace
 
 IluPlan ilu_plan(int n, const int* rowptr, const int* col, const int* diag, bool upper, const std::vector<int>& order,
@@ -32,7 +25,9 @@ IluPlan ilu_plan(int n, const int* rowptr, const int* col, const int* diag, bool
   auto first = [&](int i) { return upper ? diag[i] + 1 : rowptr[i]; };
   auto last = [&](int i) { return upper ? rowptr[i + 1] : diag[i]; };
 
-  std::vector<int> lev(n), grp(n), dep(n), most(n);  // most: terms of a row at most, its own input among them
+  IntArray lev, grp, dep, most, width_of;
+  for (IntArray* x : {&lev, &grp, &dep, &most, &width_of}) x->resize(n);
+  // most: terms of a row at most, its own input among them
   for (int k = 0; k < n; ++k) {
     const int i = upper ? n - 1 - k : k;
     int l = 0;
@@ -85,7 +80,8 @@ IluPlan ilu_plan(int n, const int* rowptr, const int* col, const int* diag, bool
   // referred to, -1 its own input), one run per reference in CSR order.
   std::vector<long> start(static_cast<size_t>(n) + 1, 0);
   for (int i = 0; i < n; ++i) start[i + 1] = start[i] + most[i];
-  Ints code(start[n]), src(start[n]), pr(start[n]), pq(start[n]);
+  IntArray code, src, pr, pq;
+  for (IntArray* x : {&code, &src, &pr, &pq}) x->resize(start[n]);
   std::vector<int> count(n), nstep(n, 0), npair(n, 0);
   for (int d = 0; d < merge_levels; ++d) {
     const std::vector<int>& list = dlist[d];
@@ -172,6 +168,7 @@ IluPlan ilu_plan(int n, const int* rowptr, const int* col, const int* diag, bool
       for (int p = p0; p < p0 + nr; ++p) {
         out.slot0[p] = static_cast<int>(slots + static_cast<long>(p - p0) * lanes);
         out.lanes[p] = lanes;
+        width_of[p] = width[k];
         out.stride[p] = nr * lanes;
       }
       slots += static_cast<long>(width[k]) * nr;
@@ -180,33 +177,35 @@ IluPlan ilu_plan(int n, const int* rowptr, const int* col, const int* diag, bool
   }
   out.col.resize(slots);
   out.src.resize(slots);
-  for (const IluSub& sub : out.subs)
-    parallel_for(
-        sub.nrows,
-        [&](long k) {
-          const int p = sub.p0 + static_cast<int>(k), i = out.rows[p];
-          out.len[p] = count[i];
-          out.depth[p] = dep[i];
-          for (int u = 0; u < sub.width; ++u) {
-            const int at = out.slot(p, u);
-            if (u < count[i]) {
-              const int c = code[start[i] + u];
-              out.col[at] = c < n ? out.pos[c] : n + out.pos[c - n];
-              out.src[at] = src[start[i] + u];
-            } else {
-              out.col[at] = p;
-              out.src[at] = -1;
-            }
+  parallel_for(
+      n,
+      [&](long k) {
+        const int p = static_cast<int>(k), i = out.rows[p];
+        out.len[p] = count[i];
+        out.depth[p] = dep[i];
+        for (int u = 0; u < width_of[p]; ++u) {
+          const int at = out.slot(p, u);
+          if (u < count[i]) {
+            const int c = code[start[i] + u];
+            out.col[at] = c < n ? out.pos[c] : n + out.pos[c - n];
+            out.src[at] = src[start[i] + u];
+          } else {
+            out.col[at] = p;
+            out.src[at] = -1;
           }
-        },
-        1 << 13);
+        }
+      },
+      1 << 13);
 
   // the steps of the rows below depth 0
   out.dptr.assign(1, 0);
-  for (int d = 1; d < merge_levels; ++d) {
+  for (int d = 1; d < merge_levels; ++d)
+    out.dptr.push_back(out.dptr.back() + static_cast<int>(dlist[d].size()));
+  out.later.resize(out.dptr.back());
+  {
+    std::vector<int> at(out.dptr);
     for (int p = 0; p < n; ++p)
-      if (out.depth[p] == d) out.later.push_back(p);
-    out.dptr.push_back(static_cast<int>(out.later.size()));
+      if (out.depth[p]) out.later[at[out.depth[p] - 1]++] = p;
   }
   const size_t nl = out.later.size();
   out.sptr.assign(nl + 1, 0);
@@ -220,7 +219,8 @@ IluPlan ilu_plan(int n, const int* rowptr, const int* col, const int* diag, bool
     out.sptr[k + 1] = static_cast<int>(steps);
   }
   out.p.resize(steps);
-  out.uptr.assign(static_cast<size_t>(steps) + 1, 0);
+  out.uptr.resize(static_cast<size_t>(steps) + 1);
+  out.uptr[0] = 0;
   out.r.resize(pairs[nl]);
   out.q.resize(pairs[nl]);
   parallel_for(

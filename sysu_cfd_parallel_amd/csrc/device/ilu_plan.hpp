@@ -1,6 +1,8 @@
 // Host plan of the ILU(0) sweeps: which rows go in one launch, and what each
 // of them sums.
 #pragma once
+#include <cstddef>
+#include <memory>
 #include <vector>
 
 namespace s355 {
@@ -47,6 +49,23 @@ struct IluSub {
   int p0, nrows, width, cls;
 };
 
+// n ints that are written before they are read (a vector would first fill them)
+struct IntArray {
+  using value_type = int;
+  std::unique_ptr<int[]> p;
+  size_t n = 0;
+  void resize(size_t m) {
+    p.reset(new int[m ? m : 1]);
+    n = m;
+  }
+  size_t size() const { return n; }
+  bool empty() const { return n == 0; }
+  int* data() { return p.get(); }
+  const int* data() const { return p.get(); }
+  int& operator[](size_t i) { return p[i]; }
+  int operator[](size_t i) const { return p[i]; }
+};
+
 struct IluPlan {
   int n = 0;
   std::vector<int> rows;     // sweep order: by group, class, then the order given
@@ -60,12 +79,13 @@ struct IluPlan {
   int slot(int q, int u) const { return slot0[q] + u / lanes[q] * stride[q] + u % lanes[q]; }
   // per slot: buf index (padding: the row's own input), and where its
   // coefficient starts from: the CSR entry a_ij (coefficient -a_ij) or -1 (0)
-  std::vector<int> col, src;
+  IntArray col, src;
   // rows below depth 0 by depth: positions later[dptr[d - 1]] .. dptr[d] - 1;
   // the k-th has steps sptr[k] .. : entry p of the matrix times the row
   // it refers to, c[r] -= a_p c[q] over pairs uptr[step] .. (q < 0: the own
   // coefficient of position -1 - q)
-  std::vector<int> dptr, later, sptr, p, uptr, r, q;
+  std::vector<int> dptr, later, sptr;
+  IntArray p, uptr, r, q;
 };
 
 // The plan of the lower (strictly lower entries) or upper sweep of a CSR
