@@ -138,11 +138,11 @@ void Context::free_all() {
   for (void* p : allocs_) hipFree(p);
   allocs_.clear();
   if (host_pinned_) hipHostFree(host_pinned_);
-  if (triple_.host) hipHostFree(triple_.host);
-  triple_.host = nullptr;
+  for (void*& p : mail_) {
+    if (p) hipHostFree(p);
+    p = nullptr;
+  }
   host_pinned_ = nullptr;
-  if (hdr_) hipHostFree(hdr_);
-  hdr_ = nullptr;
   if (stream) hipStreamDestroy(stream);
   stream = nullptr;
 }
@@ -390,8 +390,22 @@ void Context::allocate_fields() {
   kwork_.norms = alloc<double>(2 * tiles1);
   kwork_.st = alloc<KState>(ncase);
   S355_HIP(hipHostMalloc(&host_pinned_, 4096 + 10 * sizeof(double) * ncase, hipHostMallocDefault));
-  S355_HIP(hipHostMalloc(reinterpret_cast<void**>(&hdr_), sizeof(KHeader) * ncase, hipHostMallocDefault));
-  kwork_.host = hdr_;
+  open_mailbox(kwork_, ncase, 0);
+}
+
+// a mailbox for the headers of n cases
+void Context::open_mailbox(KWork& w, int n, int k) {
+  void* p = nullptr;
+  const size_t bytes = sizeof(KHeader) * n;
+  S355_HIP(hipHostMalloc(&p, bytes + 64, hipHostMallocMapped | hipHostMallocCoherent));
+  mail_[k] = p;
+  std::memset(p, 0, bytes + 64);
+  w.box.host = w.host = static_cast<KHeader*>(p);
+  w.box.arrived = reinterpret_cast<unsigned*>(static_cast<char*>(p) + bytes);
+  w.box.sent = alloc<unsigned>(1);
+  fill_zero(w.box.sent, sizeof(unsigned), stream);
+  sent_[k] = 0;
+  w.box_count = &sent_[k];
 }
 
 void Context::set_params(const s355_params& p) {
@@ -794,6 +808,8 @@ void Context::ensure_mixed() {
   kwork32_.norms = kwork_.norms;
   kwork32_.st = kwork_.st;
   kwork32_.host = kwork_.host;
+  kwork32_.box = kwork_.box;
+  kwork32_.box_count = kwork_.box_count;
   kwork32_.ncase = kwork_.ncase;
   for (int r = 0; r < 5; ++r) kwork32_.tiles[r] = kwork_.tiles[r];
   ir_.r64 = alloc<double>(Nc);
@@ -926,7 +942,7 @@ void Context::ensure_triple() {
   triple_.partial = alloc<double>(triple_.partial_len);
   triple_.norms = alloc<double>(2 * tiles1);
   triple_.st = alloc<KState>(3);
-  S355_HIP(hipHostMalloc(reinterpret_cast<void**>(&triple_.host), sizeof(KHeader) * 3, hipHostMallocDefault));
+  open_mailbox(triple_, 3, 1);
   // sized for FP64 vectors, which the mixed path's FP32 ones then fit
   const size_t elem = par.precision == S355_MIXED ? sizeof(float) : sizeof(double);
   triple_elem_ = elem;
@@ -956,6 +972,8 @@ KWork Context::triple_work(const KWork& w, bool fp32) {
   t.norms = triple_.norms;
   t.st = triple_.st;
   t.host = triple_.host;
+  t.box = triple_.box;
+  t.box_count = triple_.box_count;
   t.timer = nullptr;  // products of three vectors are not what it times
   if (w.ilu) {
     if (!triple_.ilu_zl) {

@@ -134,7 +134,10 @@ class Context {
   double* scalars_ = nullptr;  // [20..21] refinement norms
   double* res_ = nullptr;      // 10 residual slots per case
   double* rate_ = nullptr;     // outlet correction per case: mode, rate, m_in, m_out, a_out
-  KHeader* hdr_ = nullptr;     // pinned, one Krylov header per case
+  // mailboxes of the solver's headers: of the cases, and of the momentum components together
+  void open_mailbox(KWork& w, int n, int k);
+  void* mail_[2] = {nullptr, nullptr};  // pinned
+  unsigned sent_[2] = {0, 0};
   int* flags_ = nullptr;       // [0] bad boundary type, [1] inlet outflow in a scalar
   double *u0_ = nullptr, *v0_ = nullptr, *w0_ = nullptr;
   double *lim_vmax_ = nullptr, *lim_vmin_ = nullptr, *lim_tmp_ = nullptr;  // limiter scratch

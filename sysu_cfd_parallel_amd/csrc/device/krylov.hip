@@ -1643,6 +1643,38 @@ __global__ void __launch_bounds__(kBlock) k_restart_finalize(const double* parti
   if (reason) s_->done = 1;
 }
 
+// ---- the headers of all cases to the host: stores into coherent pinned memory,
+// then the count of such messages, which the host polls (one block)
+__device__ __forceinline__ void publish(const KState* st, int ncase, const Mailbox& box) {
+  for (int c = threadIdx.x; c < ncase; c += blockDim.x) {
+    KHeader h;
+    h.it = st[c].it;
+    h.its = st[c].its;
+    h.reason = st[c].reason;
+    h.maxit = st[c].maxit;
+    h.done = st[c].done;
+    h.cycles = st[c].cycles;
+    h.ended = st[c].ended;
+    h.pad0 = 0;
+    h.rnorm = st[c].rnorm;
+    h.rnorm0 = st[c].rnorm0;
+    h.ttol = st[c].ttol;
+    h.snorm = st[c].snorm;
+    box.host[c] = h;
+  }
+  __threadfence_system();
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const unsigned n = *box.sent + 1;
+    *box.sent = n;
+    __hip_atomic_store(box.arrived, n, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+
+__global__ void __launch_bounds__(kBlock) k_publish(const KState* st, int ncase, Mailbox box) {
+  publish(st, ncase, box);
+}
+
 // ---- end of a GMRES cycle, after the update of x (one thread per case).
 // Plain solve: a set reason ends the case, then the iteration cap.  Mixed
 // solve: a passed estimate, a breakdown of the FP32 cycle after which x was
@@ -1650,9 +1682,9 @@ __global__ void __launch_bounds__(kBlock) k_restart_finalize(const double* parti
 // the FP64 residual, which applies the cap after its own test; a divergence
 // ends the case, and so does a breakdown of the back substitution (no
 // update: the next cycle would start from the same residual and break down
-// the same way).
-__global__ void k_cycle_end(KState* st, int ncase, int mixed) {
-  for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < ncase; c += gridDim.x * blockDim.x) {
+// the same way).  One block, which then publishes the headers.
+__global__ void __launch_bounds__(kBlock) k_cycle_end(KState* st, int ncase, int mixed, Mailbox box) {
+  for (int c = threadIdx.x; c < ncase; c += blockDim.x) {
     KState* s = st + c;
     if (s->done) continue;
     const int r = s->reason;
@@ -1671,6 +1703,8 @@ __global__ void k_cycle_end(KState* st, int ncase, int mixed) {
         s->reason = 0;
     }
   }
+  // (a thread publishes the cases it has just ended)
+  publish(st, ncase, box);
 }
 
 // ---- solver state of every case at the start of a solve
@@ -1935,11 +1969,28 @@ struct Dispatch {
   }
 };
 
-// headers of every case: one strided copy out of the state array
+// Waits for the last message of w's mailbox launched on s.  A copy of the
+// headers and a stream synchronisation took 36-40 us between a cycle's last
+// kernel and the next one's first; the poll takes about half of that.  It ends
+// with the stream: a stream that is idle or in error without the message throws.
+void await_headers(KWork& w, hipStream_t s) {
+  const unsigned want = *w.box_count;
+  auto here = [&] { return __atomic_load_n(w.box.arrived, __ATOMIC_ACQUIRE) == want; };
+  for (int n = 0; !here(); ++n) {
+    if ((n & 4095) != 4095) continue;
+    const hipError_t e = hipStreamQuery(s);
+    if (e == hipErrorNotReady) continue;
+    S355_HIP(e);
+    if (!here()) throw HipError("solver state not received from the device");
+  }
+}
+
+// headers of every case
 void read_headers(KWork& w, hipStream_t s) {
-  S355_HIP(hipMemcpy2DAsync(w.host, sizeof(KHeader), w.st, sizeof(KState), sizeof(KHeader), w.ncase,
-                            hipMemcpyDeviceToHost, s));
-  S355_HIP(hipStreamSynchronize(s));
+  hipLaunchKernelGGL(k_publish, dim3(1), dim3(kBlock), 0, s, w.st, w.ncase, w.box);
+  S355_LAUNCH_CHECK();
+  ++*w.box_count;
+  await_headers(w, s);
 }
 
 bool all_done(const KWork& w) {
@@ -1964,6 +2015,11 @@ int running_its(const KWork& w) {
 }
 
 void init_states(KWork& w, const s355_ksp_opts& o, hipStream_t s) {
+  if (__atomic_load_n(w.box.arrived, __ATOMIC_ACQUIRE) != *w.box_count) {
+    // an earlier solve ended in an exception with a message under way or not sent
+    S355_HIP(hipStreamSynchronize(s));
+    *w.box_count = __atomic_load_n(w.box.arrived, __ATOMIC_ACQUIRE);
+  }
   hipLaunchKernelGGL(k_init_states, dim3(grid_for(w.ncase)), dim3(kBlock), 0, s, w.st, w.ncase, o.maxit, o.rtol,
                      o.abstol, o.dtol);
   S355_LAUNCH_CHECK();
@@ -2152,7 +2208,7 @@ KResult gmres(const CsrView<T>& A, const CsrView<X>& Ares, const X* b, X* x, con
     flush_fin();
     hipLaunchKernelGGL(k_build_y, dim3(nc), dim3(kWave), 0, s, w.st, m);
     Dispatch<T>::update(R, V, ld, tl, x, w.st, w.ord_row, rhs_n, s);
-    hipLaunchKernelGGL(k_cycle_end, dim3(grid_for(nc)), dim3(kBlock), 0, s, w.st, nc, mixed ? 1 : 0);
+    hipLaunchKernelGGL(k_cycle_end, dim3(1), dim3(kBlock), 0, s, w.st, nc, mixed ? 1 : 0, w.box);
     S355_LAUNCH_CHECK();
   };
 
@@ -2191,8 +2247,11 @@ KResult gmres(const CsrView<T>& A, const CsrView<X>& Ares, const X* b, X* x, con
           fin_pending = -1;
           for (int it = 0; it < ksplit; ++it) enqueue_iteration(it, false);
           flush_fin();
+          hipLaunchKernelGGL(k_publish, dim3(1), dim3(kBlock), 0, s, w.st, nc, w.box);
+          S355_LAUNCH_CHECK();
         });
-        read_headers(w, s);
+        ++*w.box_count;
+        await_headers(w, s);
         if (all_stopped(w)) {
           launch(3, [&] { enqueue_end(); });
         } else {
@@ -2208,7 +2267,8 @@ KResult gmres(const CsrView<T>& A, const CsrView<X>& Ares, const X* b, X* x, con
           enqueue_end();
         });
       }
-      read_headers(w, s);
+      ++*w.box_count;
+      await_headers(w, s);
       if (all_done(w)) break;
     }
     return collect(w, mixed);
@@ -2243,11 +2303,15 @@ KResult gmres(const CsrView<T>& A, const CsrView<X>& Ares, const X* b, X* x, con
       }
     }
     enqueue_end();
-    read_headers(w, s);
+    ++*w.box_count;
+    await_headers(w, s);
     if (all_done(w)) break;
     its = running_its(w);
   }
-  if (w.timer) w.timer->harvest();  // the header reads have synchronised the stream
+  if (w.timer) {
+    S355_HIP(hipStreamSynchronize(s));
+    w.timer->harvest();
+  }
   return collect(w, mixed);
 }
 

@@ -51,6 +51,15 @@ struct KHeader {
 };
 static_assert(offsetof(KState, rnorm) == offsetof(KHeader, rnorm), "KHeader mirrors the head of KState");
 
+// Where the solver kernels leave the headers for the host: coherent pinned memory
+// (host, arrived), the count of messages sent (device) and arrived.  One per set
+// of states; the solves of a context run one after the other on its stream.
+struct Mailbox {
+  KHeader* host = nullptr;
+  unsigned* arrived = nullptr;
+  unsigned* sent = nullptr;
+};
+
 template <class T>
 struct CsrView {
   int n = 0;
@@ -266,7 +275,9 @@ struct KWork {
   bool pc_folded = false;  // the FP32 matrix holds M^-1 A (Jacobi): the SpMV scales nothing
   SpmvTimer* timer = nullptr;    // set: time the Arnoldi SpMV launches
   KState* st = nullptr;     // device, ncase states
-  KHeader* host = nullptr;  // pinned, ncase headers
+  KHeader* host = nullptr;  // pinned, ncase headers (the mailbox's)
+  Mailbox box;
+  unsigned* box_count = nullptr;  // host: messages launched
   std::vector<KResult>* per_case = nullptr;  // filled by a solve when set
 };
 
