@@ -1190,7 +1190,7 @@ __device__ void arnoldi_finalize(const double* norms, const Tiles& t, int c, int
   arnoldi_close(s, it, m, s_, q, col, cc, ss);
 }
 
-// ... as a launch of its own (one block per case): the last step of a cycle
+// ... as a launch of its own (one block per case)
 __global__ void __launch_bounds__(kBlock) k_arnoldi_finalize(const double* norms, Tiles t, int it, int m, KState* st) {
   KState* s_ = st + blockIdx.x;
   if (s_->reason) return;
@@ -1212,28 +1212,41 @@ __global__ void __launch_bounds__(kBlock) k_arnoldi_finalize(const double* norms
 __global__ void __launch_bounds__(kBlock) k_orth(const double* dots, const double* norms, Tiles t, int it, int m,
                                                  int fin, KState* st) {
   KState* s = st + blockIdx.y;
-  if (s->ended) return;
-  const int k = blockIdx.x;
+  const int ended = s->ended, k = blockIdx.x;
   if (k > it) {
-    arnoldi_finalize(norms, t, blockIdx.y, it - 1, m, s);
+    if (!ended) arnoldi_finalize(norms, t, blockIdx.y, it - 1, m, s);
     return;
   }
-  __shared__ double lds[kBlock / kWave], lds2[kBlock / kWave];
+  __shared__ double lds[2 * kBlock / kWave];
   int t0, t1;
   t.tiles_of(blockIdx.y, t0, t1);
-  double v = strided_sum(dots + static_cast<size_t>(k) * t.ntile, t0, t1);  // column k: contiguous over tiles
+  // (column k: contiguous over tiles; everything loads before the state is tested)
+  double v = strided_sum(dots + static_cast<size_t>(k) * t.ntile, t0, t1);
   double n2 = fin ? strided_sum(norms, t0, t1) : 0.0;
-  v = block_sum(v, lds);
-  if (fin) n2 = block_sum(n2, lds2);
+  const double sk = s->scale[k], sit = fin ? 0.0 : s->scale[it];
+  if (ended) return;
+  // both block sums behind one barrier, in block_sum's order
+  v = wave_sum(v);
+  if (fin) n2 = wave_sum(n2);
+  const int wid = threadIdx.x / kWave;
+  if ((threadIdx.x & (kWave - 1)) == 0) {
+    lds[wid] = v;
+    lds[kBlock / kWave + wid] = n2;
+  }
+  __syncthreads();
   if (threadIdx.x == 0) {
-    double sw;
-    if (fin) {
-      const double tt = sqrt(n2);
-      sw = tt != 0.0 ? 1.0 / tt : 1.0;
-    } else {
-      sw = s->scale[it];
+    double a = 0.0, b = 0.0;
+#pragma unroll
+    for (int w = 0; w < kBlock / kWave; ++w) {
+      a += lds[w];
+      b += lds[kBlock / kWave + w];
     }
-    s->hcol[it & 1][k] = v * (k == it ? sw : s->scale[k]) * sw;
+    double sw = sit;
+    if (fin) {
+      const double tt = sqrt(b);
+      sw = tt != 0.0 ? 1.0 / tt : 1.0;
+    }
+    s->hcol[it & 1][k] = a * (k == it ? sw : sk) * sw;
   }
 }
 
@@ -1443,32 +1456,45 @@ void launch_spmv_dots(int nt, const SellView<T>& sell, const Tiles& t, T* V, siz
     launch_spmv_dots_c<T, false, false>(sell, t, V, ld, inv, st, it, dots, s);
 }
 
-// ---- back substitution R y = g on the completed columns of each case, y_j
-// scaled by scale_j; one wavefront per case, column-oriented: lane i keeps
-// t_i, and once y_r is known every lane i < r subtracts H(i,r) y_r.  The
+// ---- the end of a cycle, one block per case: the finalisation of its last step
+// it (fin), then the back substitution R y = g on the completed columns, y_j
+// scaled by scale_j.  One wavefront solves it, column-oriented: lane i keeps
+// t_i, and once y_r is known every lane i < r subtracts H(i,r) y_r; the columns
+// are staged in LDS, so its chain is a division and an exchange per column and
+// no global load (50 columns: 30 us with the loads in it, 6 without).  The
 // number of terms of the update goes to the state's pad word.
-__global__ void __launch_bounds__(kWave) k_build_y(KState* st, int m) {
+__global__ void __launch_bounds__(kBlock) k_build_y(const double* norms, Tiles t, int it, int m, int fin, KState* st) {
   KState* s = st + blockIdx.x;
+  constexpr int kCol = kMaxRestart + 1;
+  __shared__ double hs[kMaxRestart * kCol], g[kMaxRestart];
+  if (fin && !s->reason) arnoldi_finalize(norms, t, blockIdx.x, it, m, s);
+  __syncthreads();  // the block's own writes to the state
   int* nupd = reinterpret_cast<int*>(&s->pad);
   const int lane = threadIdx.x;
-  const int ld = m + 1;
   const int k = s->it - 1;
   if (k < 0) {
     if (lane == 0) *nupd = 0;
     return;
   }
-  double t = lane <= k ? s->grs[lane] : 0.0;
+  for (int j = threadIdx.x; j < (k + 1) * (k + 1); j += kBlock) {
+    const int c = j / (k + 1), r = j - c * (k + 1);
+    if (r <= c) hs[c * kCol + r] = Hm(s, m + 1, r, c);
+  }
+  if (lane <= k) g[lane] = s->grs[lane];
+  __syncthreads();
+  if (lane >= kWave) return;
+  double tl = lane <= k ? g[lane] : 0.0;
   double y = 0.0;
   bool broke = false;
   for (int r = k; r >= 0; --r) {
-    const double hrr = Hm(s, ld, r, r);
+    const double hrr = hs[r * kCol + r], hir = lane < r ? hs[r * kCol + lane] : 0.0;
     if (hrr == 0.0) {
       broke = true;
       break;
     }
-    const double yr = __shfl(t, r, kWave) / hrr;
+    const double yr = __shfl(tl, r, kWave) / hrr;
     if (lane == r) y = yr;
-    if (lane < r) t -= Hm(s, ld, lane, r) * yr;
+    if (lane < r) tl -= hir * yr;
   }
   if (broke) {
     if (lane == 0) {
@@ -2205,8 +2231,9 @@ KResult gmres(const CsrView<T>& A, const CsrView<X>& Ares, const X* b, X* x, con
     S355_LAUNCH_CHECK();
   };
   auto enqueue_end = [&] {
-    flush_fin();
-    hipLaunchKernelGGL(k_build_y, dim3(nc), dim3(kWave), 0, s, w.st, m);
+    hipLaunchKernelGGL(k_build_y, dim3(nc), dim3(kBlock), 0, s, norms[fin_pending & 1], tl, fin_pending, m,
+                       fin_pending >= 0 ? 1 : 0, w.st);
+    fin_pending = -1;
     Dispatch<T>::update(R, V, ld, tl, x, w.st, w.ord_row, rhs_n, s);
     hipLaunchKernelGGL(k_cycle_end, dim3(1), dim3(kBlock), 0, s, w.st, nc, mixed ? 1 : 0, w.box);
     S355_LAUNCH_CHECK();
