@@ -138,10 +138,6 @@ void Context::free_all() {
   for (void* p : allocs_) hipFree(p);
   allocs_.clear();
   if (host_pinned_) hipHostFree(host_pinned_);
-  for (void*& p : mail_) {
-    if (p) hipHostFree(p);
-    p = nullptr;
-  }
   host_pinned_ = nullptr;
   if (stream) hipStreamDestroy(stream);
   stream = nullptr;
@@ -389,19 +385,20 @@ void Context::allocate_fields() {
   kwork_.partial_len = partial_len_;
   kwork_.norms = alloc<double>(2 * tiles1);
   kwork_.st = alloc<KState>(ncase);
-  S355_HIP(hipHostMalloc(&host_pinned_, 4096 + 10 * sizeof(double) * ncase, hipHostMallocDefault));
+  // 4 KiB of fixed slots, the residuals, the mailboxes of the cases' and of the
+  // momentum components' headers
+  const size_t mail0 = 4096 + (10 * sizeof(double) * ncase + 63) / 64 * 64, mail1 = mail0 + mail_bytes(ncase);
+  S355_HIP(hipHostMalloc(&host_pinned_, mail1 + mail_bytes(3), hipHostMallocMapped | hipHostMallocCoherent));
+  mail_[0] = static_cast<char*>(host_pinned_) + mail0;
+  mail_[1] = static_cast<char*>(host_pinned_) + mail1;
   open_mailbox(kwork_, ncase, 0);
 }
 
-// a mailbox for the headers of n cases
+// the mailbox for the headers of n cases at mail_[k] (see mail_bytes)
 void Context::open_mailbox(KWork& w, int n, int k) {
-  void* p = nullptr;
-  const size_t bytes = sizeof(KHeader) * n;
-  S355_HIP(hipHostMalloc(&p, bytes + 64, hipHostMallocMapped | hipHostMallocCoherent));
-  mail_[k] = p;
-  std::memset(p, 0, bytes + 64);
-  w.box.host = w.host = static_cast<KHeader*>(p);
-  w.box.arrived = reinterpret_cast<unsigned*>(static_cast<char*>(p) + bytes);
+  std::memset(mail_[k], 0, mail_bytes(n));
+  w.box.host = w.host = reinterpret_cast<KHeader*>(mail_[k]);
+  w.box.arrived = reinterpret_cast<unsigned*>(mail_[k] + sizeof(KHeader) * n);
   w.box.sent = alloc<unsigned>(1);
   fill_zero(w.box.sent, sizeof(unsigned), stream);
   sent_[k] = 0;

@@ -136,7 +136,8 @@ class Context {
   double* rate_ = nullptr;     // outlet correction per case: mode, rate, m_in, m_out, a_out
   // mailboxes of the solver's headers: of the cases, and of the momentum components together
   void open_mailbox(KWork& w, int n, int k);
-  void* mail_[2] = {nullptr, nullptr};  // pinned
+  static size_t mail_bytes(int n) { return (sizeof(KHeader) * n + sizeof(unsigned) + 63) / 64 * 64; }
+  char* mail_[2] = {nullptr, nullptr};  // in host_pinned_
   unsigned sent_[2] = {0, 0};
   int* flags_ = nullptr;       // [0] bad boundary type, [1] inlet outflow in a scalar
   double *u0_ = nullptr, *v0_ = nullptr, *w0_ = nullptr;

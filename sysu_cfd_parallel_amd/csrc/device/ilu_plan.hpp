@@ -29,7 +29,8 @@ namespace s355 {
 // factorisation for 9 steps) by levels, rows and terms, in ms: no merging 131.7,
 // 162.3, 90.6, 13.2; 6, 65536, 96: 60.2, 62.3, 39.6, 4.68; 8, 65536, 160: 55.6,
 // 56.0, 38.0, 4.76; 8, 65536, 300: 55.2, 51.4, 38.9, 4.80; 12, 65536, 300: 52.8,
-// 50.4, 37.6, 5.30; 16, 65536, 1000: 51.9, 48.4, 40.2, 6.31.
+// 50.4, 37.6, 5.30; 16, 65536, 1000: 51.9, 48.4, 40.2, 6.31.  Taken: 8, 65536, 200
+// (55.7, 56.7, 39.1, 4.82); more terms save little and lengthen the plan.
 constexpr int kMergeLevels = 8;
 constexpr int kMergeTerms = 200;
 constexpr int kMergeRows = 65536;
