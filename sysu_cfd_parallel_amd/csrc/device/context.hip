@@ -940,30 +940,22 @@ void Context::ensure_triple() {
   triple_.norms = alloc<double>(2 * tiles1);
   triple_.st = alloc<KState>(3);
   open_mailbox(triple_, 3, 1);
-  // sized for FP64 vectors, which the mixed path's FP32 ones then fit
-  const size_t elem = par.precision == S355_MIXED ? sizeof(float) : sizeof(double);
-  triple_elem_ = elem;
-  triple_.V = alloc<char>((static_cast<size_t>(max_restart_) + 1) * ld * elem);
-  triple_.r = alloc<char>(ld * elem);
 }
 
 // The workspace of the three momentum components' solve: the shapes, matrix
 // copies and preconditioner of w, the vectors and states of three cases.
 KWork Context::triple_work(const KWork& w, bool fp32) {
-  const size_t n = dm.Nc, elem = fp32 ? sizeof(float) : sizeof(double);
-  if (elem > triple_elem_) {  // the precision was changed
-    triple_.V = alloc<char>((static_cast<size_t>(max_restart_) + 1) * ((3 * n + 7) / 8 * 8) * elem);
-    triple_.r = alloc<char>((3 * n + 7) / 8 * 8 * elem);
-    triple_.ilu_zl = nullptr;
-    triple_elem_ = elem;
-  }
+  const size_t n = dm.Nc, ld = (3 * n + 7) / 8 * 8, elem = fp32 ? sizeof(float) : sizeof(double);
+  TripleVectors& own = triple_vec_[fp32];
+  if (!own.V) own.V = alloc<char>((static_cast<size_t>(max_restart_) + 1) * ld * elem);
+  if (!own.r) own.r = alloc<char>(ld * elem);
   KWork t = w;
   t.n = 3 * dm.Nc;
   t.ncase = t.rep = 3;
-  t.ld = (3 * n + 7) / 8 * 8;
+  t.ld = ld;
   for (int r = 0; r < 5; ++r) t.tiles[r] = triple_.tiles[r];
-  t.V = triple_.V;
-  t.r = triple_.r;
+  t.V = own.V;
+  t.r = own.r;
   t.partial = triple_.partial;
   t.partial_len = triple_.partial_len;
   t.norms = triple_.norms;
@@ -973,12 +965,10 @@ KWork Context::triple_work(const KWork& w, bool fp32) {
   t.box_count = triple_.box_count;
   t.timer = nullptr;  // products of three vectors are not what it times
   if (w.ilu) {
-    if (!triple_.ilu_zl) {
-      triple_.ilu_zl = alloc<char>(6 * n * triple_elem_);
-      triple_.ilu_zu = alloc<char>(6 * n * triple_elem_);
-    }
-    t.ilu_zl = triple_.ilu_zl;
-    t.ilu_zu = triple_.ilu_zu;
+    if (!own.ilu_zl) own.ilu_zl = alloc<char>(6 * n * elem);
+    if (!own.ilu_zu) own.ilu_zu = alloc<char>(6 * n * elem);
+    t.ilu_zl = own.ilu_zl;
+    t.ilu_zu = own.ilu_zu;
   }
   return t;
 }

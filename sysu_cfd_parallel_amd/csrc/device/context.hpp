@@ -149,10 +149,14 @@ class Context {
   float* a32_ = nullptr;
   KWork kwork32_{};
   IrWork ir_{};
-  // the three momentum components solved together: vectors and states, sized by
-  // triple_elem_ bytes an element
+  // the three momentum components solved together: states and sums, and the
+  // vectors of each precision (FP64, FP32).  None is ever replaced: captured
+  // cycles hold their addresses.
   KWork triple_{};
-  size_t triple_elem_ = 0;
+  struct TripleVectors {
+    void *V = nullptr, *r = nullptr, *ilu_zl = nullptr, *ilu_zu = nullptr;
+  };
+  TripleVectors triple_vec_[2];
   double *x3_ = nullptr, *b3_ = nullptr;
   // inner order of mixed GMRES: rows in reverse Cuthill-McKee order
   bool have_order_ = false, order_ok_ = false;

@@ -364,6 +364,7 @@ void ilu_apply(const CsrView<T>& A, const IluLevels& lv, const T* lu, const T* r
                                         reinterpret_cast<uintptr_t>(z), reinterpret_cast<uintptr_t>(st),
                                         reinterpret_cast<uintptr_t>(lv.lpos), sizeof(T),
                                         reinterpret_cast<uintptr_t>(w ? w->ilu_lcoef : nullptr),
+                                        reinterpret_cast<uintptr_t>(w ? w->ilu_zl : nullptr),
                                         reinterpret_cast<uintptr_t>(dot)};
     hipGraphExec_t g = graphs->get(key, s, [&] { ilu_apply(A, lv, lu, r, z, st, s, nullptr, w, dot); });
     S355_HIP(hipGraphLaunch(g, s));
@@ -2254,6 +2255,8 @@ KResult gmres(const CsrView<T>& A, const CsrView<X>& Ares, const X* b, X* x, con
       std::vector<uintptr_t> key = {reinterpret_cast<uintptr_t>(A.val), reinterpret_cast<uintptr_t>(Ares.val),
                                           reinterpret_cast<uintptr_t>(b), reinterpret_cast<uintptr_t>(x),
                                           reinterpret_cast<uintptr_t>(inv), reinterpret_cast<uintptr_t>(invr),
+                                          reinterpret_cast<uintptr_t>(V), reinterpret_cast<uintptr_t>(w.st),
+                                          reinterpret_cast<uintptr_t>(w.partial),
                                           static_cast<uintptr_t>(m), static_cast<uintptr_t>(R),
                                           static_cast<uintptr_t>(L), static_cast<uintptr_t>(w.nt),
                                           static_cast<uintptr_t>(w.sell_v),
