@@ -2161,7 +2161,7 @@ KResult gmres(const CsrView<T>& A, const CsrView<X>& Ares, const X* b, X* x, con
     if (lu) {
       const T* bt;
       if constexpr (mixed) {
-        convert_to_float(b, tmp, ld, s);
+        convert_to_float(b, tmp, w.n, s);
         bt = tmp;
       } else {
         bt = b;
@@ -2174,7 +2174,7 @@ KResult gmres(const CsrView<T>& A, const CsrView<X>& Ares, const X* b, X* x, con
     }
     hipLaunchKernelGGL(k_snorm_final, dim3(nc), dim3(kBlock), 0, s, w.partial, tl, w.st);
   } else {
-    fill_zero(x, sizeof(X) * ld, s);
+    fill_zero(x, sizeof(X) * static_cast<size_t>(w.n), s);
   }
   auto enqueue_restart = [&](bool first_c, bool gz_c) {
     if (lu) {

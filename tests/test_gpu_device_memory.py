@@ -1,0 +1,77 @@
+"""Device allocations under guard: no solve writes behind a vector of its own
+(row counts that are no multiple of the basis' padding).  Each test runs in a
+process of its own, in which the probe's hipMalloc is the library's."""
+import subprocess
+import sys
+from pathlib import Path
+
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+ROOT = Path(__file__).resolve().parents[1]
+
+HEAD = """
+import ctypes as C, sys
+probe = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
+probe.probe_fail_from.argtypes = [C.c_size_t]
+for f in ("probe_count", "probe_live", "probe_damaged"):
+    getattr(probe, f).restype = C.c_long
+probe.probe_fail.argtypes = [C.c_long]
+sys.path[:0] = [sys.argv[2], sys.argv[2] + "/tests"]
+import numpy as np
+import sysu_cfd_parallel_amd as s
+from helpers import params, push, random_state
+"""
+
+
+@pytest.fixture(scope="module")
+def probe(tmp_path_factory):
+    so = tmp_path_factory.mktemp("alloc") / "probe.so"
+    subprocess.run(["g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-o", str(so),
+                    str(ROOT / "tests/golden/device_alloc_probe.cpp"), "-ldl"], check=True)
+
+    def run(body):
+        r = subprocess.run([sys.executable, "-c", HEAD + body, str(so), str(ROOT)], capture_output=True, text=True,
+                           timeout=100)
+        assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-4000:]
+        return r.stdout
+
+    return run
+
+
+def test_solves_stay_inside_their_vectors(probe):
+    out = probe("""
+CASES = [s.channel(9, 1, 1), s.channel(5, 2, 1), s.cavity(3), s.channel(3, 2, 2), s.cavity(5, jitter=0.1),
+         s.cavity(5, tets=True, jitter=0.1), s.cavity(7), s.channel(11, 7, 3, jitter=0.1, split=0.3, seed=2)]
+rest = set()
+for case in CASES:
+    for precision, order in ((s.FP64, 0), (s.MIXED, 0), (s.MIXED, 2)):
+        for pc in (s.PC_JACOBI, s.PC_ILU0):
+            for graphs in (0, 1):
+                p = params(restart=7, pc=pc)
+                p.precision, p.graphs, p.inner_order = precision, graphs, order
+                d = s.Solver(case, p)
+                n = d.sizes.n_cell
+                rest.add(n % 8)
+                push(d, {k: v for k, v in random_state(n, d.sizes.n_bnd, d.sizes.n_face, 5).items()
+                         if k in ("U", "V", "W", "P", "R", "APR", "DPDX", "RUFACE", "VISLAM")})
+                d.call("build_velocity_matrix")
+                d.solve_velocity(1e-8, 500)
+                for k in ("bc_velocity", "cal_ru_face", "build_pressure_matrix"):
+                    d.call(k)
+                try:
+                    d.solve_pressure(1e-6, 20)
+                except s.NotConverged:
+                    pass
+                try:
+                    d.update_energy()
+                except s.NotConverged:
+                    pass
+                bad = probe.probe_damaged()
+                assert bad == 0, (n, precision, order, pc, graphs, bad)
+                d.close()
+assert rest == set(range(1, 8)), rest
+print("guards whole", probe.probe_count(), sorted(rest))
+""")
+    assert "guards whole" in out and int(out.split()[2]) > 1000
