@@ -13,6 +13,11 @@ struct HipError : std::runtime_error {
   using std::runtime_error::runtime_error;
 };
 
+// the device has no room for an allocation
+struct DeviceMemoryError : HipError {
+  using HipError::HipError;
+};
+
 #define S355_HIP(call)                                                                              \
   do {                                                                                              \
     hipError_t e_ = (call);                                                                         \

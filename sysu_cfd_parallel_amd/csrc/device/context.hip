@@ -20,28 +20,35 @@ namespace s355 {
 namespace {
 constexpr double kSmallInit = 1.e-16;
 constexpr double kCmuInit = 0.09;
+constexpr int kNoRoom = -1;  // of run_solve, never returned to a caller
 }  // namespace
+
+void* Context::device_bytes(size_t bytes) {
+  void* p = nullptr;
+  hipError_t e = hipMalloc(&p, bytes);
+  if (e == hipErrorOutOfMemory) {
+    (void)hipGetLastError();  // reported here, not by the next launch's check
+    if (drop_triple() && (e = hipMalloc(&p, bytes)) == hipErrorOutOfMemory) (void)hipGetLastError();
+  }
+  if (e == hipErrorOutOfMemory)
+    throw DeviceMemoryError("hipMalloc: out of memory (" + std::to_string(bytes) + " bytes)");
+  S355_HIP(e);
+  allocs_.push_back(p);
+  return p;
+}
 
 template <class T>
 T* Context::alloc(size_t n) {
-  void* p = nullptr;
-  size_t bytes = std::max<size_t>(n, 1) * sizeof(T);
-  S355_HIP(hipMalloc(&p, bytes));
-  allocs_.push_back(p);
-  return static_cast<T*>(p);
+  return static_cast<T*>(device_bytes(std::max<size_t>(n, 1) * sizeof(T)));
 }
 
-namespace {
 template <class Vec>
-auto upload(std::vector<void*>& allocs, const Vec& v, hipStream_t s) {
+auto Context::upload(const Vec& v) {
   using T = typename Vec::value_type;
-  void* p = nullptr;
-  S355_HIP(hipMalloc(&p, std::max<size_t>(v.size(), 1) * sizeof(T)));
-  allocs.push_back(p);
-  if (!v.empty()) S355_HIP(hipMemcpyAsync(p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice, s));
+  T* p = alloc<T>(v.size());
+  if (!v.empty()) S355_HIP(hipMemcpyAsync(p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice, stream));
   return static_cast<const T*>(p);
 }
-}  // namespace
 
 Context::Context(const s355_mesh_desc* descs, int n_case, const s355_params& params) : par(params), ncase(n_case) {
   if (par.density_model != 0) throw std::invalid_argument("only DensityModel 0 (constant density) is supported");
@@ -115,10 +122,10 @@ Tiles Context::make_tiles(const std::vector<int>& case_row, int tile) {
   ct[nc] = static_cast<int>(lo.size());
   t.ntile = static_cast<int>(lo.size());
   lo.push_back(t.n);
-  t.lo = upload(allocs_, lo, stream);
-  t.tcase = upload(allocs_, tc, stream);
-  t.case_tile = upload(allocs_, ct, stream);
-  t.case_row = upload(allocs_, case_row, stream);
+  t.lo = upload(lo);
+  t.tcase = upload(tc);
+  t.case_tile = upload(ct);
+  t.case_row = upload(case_row);
   S355_HIP(hipStreamSynchronize(stream));  // host staging vectors go out of scope
   if (t.ntile < 1) throw std::invalid_argument("empty batch");
   return t;
@@ -151,8 +158,8 @@ void Context::compute_geometry() {
   Mesh& m = mesh;
   const size_t Nc = m.n_cell, Nf = m.n_face, Nb = m.n_bnd;
   dm.Nv = m.n_vert;
-  dm.vert = upload(allocs_, m.vert, stream);
-  dm.c_vert = upload(allocs_, m.c_vert, stream);
+  dm.vert = upload(m.vert);
+  dm.c_vert = upload(m.c_vert);
   // topology used by the geometry only: freed once it is done
   uint8_t *poly = nullptr, *warped = nullptr;
   int* fv = nullptr;
@@ -236,20 +243,20 @@ void Context::upload_mesh() {
   dm.Nf = m.n_face;
   dm.Nb = m.n_bnd;
   dm.nnz = m.nnz();
-  dm.f_c1 = upload(allocs_, m.f_c1, stream);
-  dm.f_c2 = upload(allocs_, m.f_c2, stream);
-  dm.cf_ptr = upload(allocs_, m.cf_ptr, stream);
-  dm.cf_pat = upload(allocs_, m.cf_pat, stream);
-  dm.rowptr = upload(allocs_, m.rowptr, stream);
-  dm.col = upload(allocs_, m.col, stream);
-  dm.diag = upload(allocs_, m.diag, stream);
+  dm.f_c1 = upload(m.f_c1);
+  dm.f_c2 = upload(m.f_c2);
+  dm.cf_ptr = upload(m.cf_ptr);
+  dm.cf_pat = upload(m.cf_pat);
+  dm.rowptr = upload(m.rowptr);
+  dm.col = upload(m.col);
+  dm.diag = upload(m.diag);
   compute_geometry();
   std::vector<int> btype(m.n_bnd);
   for (int b = 0; b < m.n_bnd; ++b) {
     btype[b] = m.type1_of_rid(m.b_rid[b]);
     if (btype[b] == kOutlet) has_outlet_ = true;
   }
-  dm.b_type = upload(allocs_, btype, stream);
+  dm.b_type = upload(btype);
   // wall-adjacent cells with their wall faces in ascending order
   std::vector<int> wcell, wptr(1, 0), wface;
   {
@@ -275,8 +282,8 @@ void Context::upload_mesh() {
       const int a1 = cpos[m.f_c1[a]], b1 = cpos[m.f_c1[b]];
       return a1 < b1 || (a1 == b1 && cpos[m.f_c2[a]] < cpos[m.f_c2[b]]);
     });
-    dm.c_order = upload(allocs_, cord, stream);
-    dm.f_order = upload(allocs_, ford, stream);
+    dm.c_order = upload(cord);
+    dm.f_order = upload(ford);
     // the half-face streams in that order, packed into blocks of whole cells
     auto stream_of = [&](const hvec<int>& faces, const hvec<int>* slots, const int*& blk, int& nblk) {
       std::vector<int4> rec;
@@ -299,8 +306,8 @@ void Context::upload_mesh() {
       }
       b.push_back(static_cast<int>(rec.size()));
       nblk = static_cast<int>(b.size()) - 1;
-      blk = upload(allocs_, b, stream);
-      return upload(allocs_, rec, stream);
+      blk = upload(b);
+      return upload(rec);
     };
     dm.hf = stream_of(m.cf_pat, &m.cf_slot, dm.hf_blk, dm.hf_nblk);
     S355_HIP(hipStreamSynchronize(stream));
@@ -310,9 +317,9 @@ void Context::upload_mesh() {
   dm.ctile = make_tiles(lay.cell, kBlock);
   dm.btile = make_tiles(lay.bnd, kBlock);
   dm.n_wcell = static_cast<int>(wcell.size());
-  dm.wc_cell = upload(allocs_, wcell, stream);
-  dm.wc_ptr = upload(allocs_, wptr, stream);
-  dm.wc_face = upload(allocs_, wface, stream);
+  dm.wc_cell = upload(wcell);
+  dm.wc_ptr = upload(wptr);
+  dm.wc_face = upload(wface);
   S355_HIP(hipStreamSynchronize(stream));  // host staging vectors go out of scope
 }
 
@@ -663,8 +670,8 @@ void Context::ensure_vertices() {
   for (int i = 0; i < nc; ++i)
     for (int j = 0; j < 8; ++j)
       if (distinct(i, j)) v2c[fill[mesh.c_vert[8 * static_cast<size_t>(i) + j]]++] = i;
-  dm.v2c_ptr = upload(allocs_, ptr, stream);
-  dm.v2c = upload(allocs_, v2c, stream);
+  dm.v2c_ptr = upload(ptr);
+  dm.v2c = upload(v2c);
   lim_vmax_ = alloc<double>(std::max(nv, 1));
   lim_vmin_ = alloc<double>(std::max(nv, 1));
   lim_tmp_ = alloc<double>(3 * static_cast<size_t>(dm.Nc));
@@ -733,25 +740,25 @@ void Context::ensure_ilu() {
     w.group = p.group;
     w.dptr = p.dptr;
     w.slots = p.col.size();
-    w.len = upload(allocs_, p.len, stream);
-    w.slot0 = upload(allocs_, p.slot0, stream);
-    w.lanes = upload(allocs_, p.lanes, stream);
-    w.stride = upload(allocs_, p.stride, stream);
-    w.col = upload(allocs_, p.col, stream);
-    w.src = upload(allocs_, p.src, stream);
-    w.later = upload(allocs_, p.later, stream);
-    w.sptr = upload(allocs_, p.sptr, stream);
-    w.p = upload(allocs_, p.p, stream);
-    w.uptr = upload(allocs_, p.uptr, stream);
-    w.r = upload(allocs_, p.r, stream);
-    w.q = upload(allocs_, p.q, stream);
+    w.len = upload(p.len);
+    w.slot0 = upload(p.slot0);
+    w.lanes = upload(p.lanes);
+    w.stride = upload(p.stride);
+    w.col = upload(p.col);
+    w.src = upload(p.src);
+    w.later = upload(p.later);
+    w.sptr = upload(p.sptr);
+    w.p = upload(p.p);
+    w.uptr = upload(p.uptr);
+    w.r = upload(p.r);
+    w.q = upload(p.q);
     if (up) {
       std::vector<int> dsrc(p.n);
       for (int k = 0; k < p.n; ++k) {
         const int d = mesh.diag[p.rows[k]];
         dsrc[k] = p.depth[k] ? -1 - d : d;
       }
-      w.dsrc = upload(allocs_, dsrc, stream);
+      w.dsrc = upload(dsrc);
       sync();
     }
   };
@@ -766,17 +773,17 @@ void Context::ensure_ilu() {
     put(levels_.upper, upper, true);
     std::vector<int> l2u(dm.Nc);
     for (int q = 0; q < dm.Nc; ++q) l2u[q] = upper.pos[lower.rows[q]];
-    levels_.lpos = upload(allocs_, lower.pos, stream);
-    levels_.l2u = upload(allocs_, l2u, stream);
-    levels_.upos = upload(allocs_, upper.pos, stream);
+    levels_.lpos = upload(lower.pos);
+    levels_.l2u = upload(l2u);
+    levels_.upos = upload(upper.pos);
     factor.join();
     if (failed) std::rethrow_exception(failed);
-    levels_.steps.ptr = upload(allocs_, sptr, stream);
-    levels_.steps.p = upload(allocs_, sp, stream);
-    levels_.steps.d = upload(allocs_, sd, stream);
-    levels_.steps.u = upload(allocs_, su, stream);
-    levels_.steps.r = upload(allocs_, sr, stream);
-    levels_.steps.q = upload(allocs_, sq, stream);
+    levels_.steps.ptr = upload(sptr);
+    levels_.steps.p = upload(sp);
+    levels_.steps.d = upload(sd);
+    levels_.steps.u = upload(su);
+    levels_.steps.r = upload(sr);
+    levels_.steps.q = upload(sq);
     sync();  // host staging vectors go out of scope
   }
   kwork_.lu = alloc<double>(dm.nnz);
@@ -820,8 +827,9 @@ void Context::ensure_mixed() {
 }
 
 // same: the matrix is the previous call's, unchanged, and so are its copies and
-// its preconditioner; rep = 3: b and x hold the three momentum components'
-// right-hand sides and solutions, solved together, records in slots 0..2
+// its preconditioner; rep = 3: the three momentum components solved together
+// (b and x unused: gathered into b3_ and x3_), records in slots 0..2; kNoRoom
+// where the device has no memory for that, before anything was solved
 int Context::run_solve(int which, const double* b, double* x, const s355_ksp_opts& o, bool zero_guess,
                        s355_solve_info* info, int slot, bool same, int rep) {
   const double* val = which == 0 ? df.Au : (which == 1 ? df.Ap : df.As);
@@ -835,6 +843,17 @@ int Context::run_solve(int which, const double* b, double* x, const s355_ksp_opt
   kwork_.prepared = kwork32_.prepared = same;
   if (rep == 1) case_info[slot].assign(ncase, KResult{});
   if (o.pc == S355_PC_ILU0) ensure_ilu();
+  // after everything else the solve allocates
+  auto gathered = [&](bool fp32) {
+    if (rep == 1) return true;
+    if (!ensure_triple(fp32, o.pc == S355_PC_ILU0)) return false;
+    const size_t n = dm.Nc;
+    launch_copy3(dm.Nc, df.bu, df.bv, df.bw, b3_, b3_ + n, b3_ + 2 * n, stream);
+    launch_copy3(dm.Nc, df.U, df.V, df.W, x3_, x3_ + n, x3_ + 2 * n, stream);
+    b = b3_;
+    x = x3_;
+    return true;
+  };
   if (par.precision == S355_MIXED) {
     // FP32 inner solves on the rounded matrix inside FP64 refinement
     ensure_mixed();
@@ -857,11 +876,13 @@ int Context::run_solve(int which, const double* b, double* x, const s355_ksp_opt
       CsrView<float> Ao{dm.Nc, ord_rowptr_, ord_col_, ord_diag_, a32o_, dm.nnz};
       if (tune) tune_ordered(Ao, std::min(o.restart, kMaxRestart));
       KWork w = ordered_work(false, same);
+      if (!gathered(true)) return kNoRoom;
       if (rep > 1) w = triple_work(w, true);
       r = ir_solve(A64, Ao, b, x, o, zero_guess, par.ir_max, par.ir_inner_rtol, w, ir_, stream);
     } else {
       if (o.type == S355_KSP_GMRES && !same && (tune || kwork32_.lanes == 0)) prepare_sell(val, true, tune);
       if (tune) autotune<float>(A, kwork32_, std::min(o.restart, kMaxRestart), stream);
+      if (!gathered(true)) return kNoRoom;
       KWork w3;
       if (rep > 1) w3 = triple_work(kwork32_, true);
       r = ir_solve(A64, A, b, x, o, zero_guess, par.ir_max, par.ir_inner_rtol, rep > 1 ? w3 : kwork32_, ir_, stream);
@@ -871,6 +892,7 @@ int Context::run_solve(int which, const double* b, double* x, const s355_ksp_opt
     const bool tune = par.autotune && o.type == S355_KSP_GMRES && !kwork_.tuned;
     if (o.type == S355_KSP_GMRES && !same && (tune || kwork_.lanes == 0)) prepare_sell(val, false, tune);
     if (tune) autotune<double>(A, kwork_, std::min(o.restart, kMaxRestart), stream);
+    if (!gathered(false)) return kNoRoom;
     KWork w3;
     if (rep > 1) w3 = triple_work(kwork_, false);
     r = krylov_solve<double>(A, b, x, o, zero_guess, rep > 1 ? w3 : kwork_, stream);
@@ -898,11 +920,8 @@ int Context::solve_velocity(double rtol, int maxit, s355_solve_info info[3]) {
     // every launch (see triple_work), each with its own state and the bits of
     // its own solve
     const size_t n = dm.Nc;
-    ensure_triple();
-    launch_copy3(dm.Nc, df.bu, df.bv, df.bw, b3_, b3_ + n, b3_ + 2 * n, stream);
-    launch_copy3(dm.Nc, df.U, df.V, df.W, x3_, x3_ + n, x3_ + 2 * n, stream);
-    rc = run_solve(0, b3_, x3_, o, false, info, 0, false, 3);
-    for (int k = 0; k < 3; ++k) {
+    rc = run_solve(0, nullptr, nullptr, o, false, info, 0, false, 3);
+    for (int k = 0; k < 3 && rc != kNoRoom; ++k) {
       S355_HIP(hipMemcpyAsync(x[k], x3_ + k * n, n * sizeof(double), hipMemcpyDeviceToDevice, stream));
       KResult r;
       r.iters = info[k].iters;
@@ -915,7 +934,7 @@ int Context::solve_velocity(double rtol, int maxit, s355_solve_info info[3]) {
       for (int j = k + 1; j < 3; ++j) info[j] = s355_solve_info{0, 0, 0.0, 0.0, 0, 0};  // left as they were
       break;
     }
-    return rc;
+    if (rc != kNoRoom) return rc;
   }
   for (int k = 0; k < 3; ++k) {
     rc = run_solve(0, b[k], x[k], o, false, &info[k], k, k > 0);
@@ -927,32 +946,87 @@ int Context::solve_velocity(double rtol, int maxit, s355_solve_info info[3]) {
   return rc;
 }
 
-void Context::ensure_triple() {
-  if (x3_) return;
-  const size_t n = dm.Nc, ld = (3 * n + 7) / 8 * 8;
-  x3_ = alloc<double>(ld);
-  b3_ = alloc<double>(ld);
-  const std::vector<int> rows = {0, dm.Nc, 2 * dm.Nc, 3 * dm.Nc};
-  for (int r = 0; r < 5; ++r) triple_.tiles[r] = make_tiles(rows, kBlock << r);
-  const size_t tiles1 = triple_.tiles[0].ntile;
-  triple_.partial_len = tiles1 * (max_restart_ + 1);
-  triple_.partial = alloc<double>(triple_.partial_len);
-  triple_.norms = alloc<double>(2 * tiles1);
-  triple_.st = alloc<KState>(3);
-  open_mailbox(triple_, 3, 1);
+// What the three components' solve needs beyond the single solve's workspace,
+// whole or not at all; false where the device has no room for it.
+bool Context::ensure_triple(bool fp32, bool ilu) {
+  TripleVectors& own = triple_vec_[fp32];
+  if (own.refused) return false;
+  if (have_triple_ && own.r && (!ilu || own.ilu_zu)) return true;
+  const size_t n = dm.Nc, ld = (3 * n + 7) / 8 * 8, elem = fp32 ? sizeof(float) : sizeof(double);
+  const size_t kept = allocs_.size();
+  KWork t = triple_;
+  TripleVectors v = own;
+  double *x3 = x3_, *b3 = b3_;
+  struct Building {  // its own allocations drop nothing
+    bool& on;
+    ~Building() { on = false; }
+  } building{building_triple_ = true};
+  try {
+    if (!have_triple_) {
+      x3 = alloc<double>(ld);
+      b3 = alloc<double>(ld);
+      const std::vector<int> rows = {0, dm.Nc, 2 * dm.Nc, 3 * dm.Nc};
+      for (int r = 0; r < 5; ++r) t.tiles[r] = make_tiles(rows, kBlock << r);
+      const size_t tiles1 = t.tiles[0].ntile;
+      t.partial_len = tiles1 * (max_restart_ + 1);
+      t.partial = alloc<double>(t.partial_len);
+      t.norms = alloc<double>(2 * tiles1);
+      t.st = alloc<KState>(3);
+      open_mailbox(t, 3, 1);
+    }
+    if (!v.r) {
+      v.V = alloc<char>((static_cast<size_t>(max_restart_) + 1) * ld * elem);
+      v.r = alloc<char>(ld * elem);
+    }
+    if (ilu && !v.ilu_zu) {
+      v.ilu_zl = alloc<char>(6 * n * elem);
+      v.ilu_zu = alloc<char>(6 * n * elem);
+    }
+  } catch (const DeviceMemoryError&) {
+    own.refused = true;
+    sync();
+    while (allocs_.size() > kept) {
+      hipFree(allocs_.back());
+      allocs_.pop_back();
+    }
+    return false;
+  }
+  triple_ = t;
+  own = v;
+  x3_ = x3;
+  b3_ = b3;
+  have_triple_ = true;
+  return true;
+}
+
+// Gives the vectors of the three components' solve back (the components are
+// solved one after the other from then on); false where there are none.
+bool Context::drop_triple() {
+  if (building_triple_) return false;
+  bool any = false;
+  for (TripleVectors& v : triple_vec_) {
+    if (!v.r) continue;
+    any = true;
+    hipStreamSynchronize(stream);
+    for (void* p : {v.V, v.r, v.ilu_zl, v.ilu_zu}) {
+      if (!p) continue;
+      allocs_.erase(std::find(allocs_.begin(), allocs_.end(), p));
+      hipFree(p);
+    }
+    v = TripleVectors{};
+    v.refused = true;
+  }
+  return any;
 }
 
 // The workspace of the three momentum components' solve: the shapes, matrix
 // copies and preconditioner of w, the vectors and states of three cases.
 KWork Context::triple_work(const KWork& w, bool fp32) {
-  const size_t n = dm.Nc, ld = (3 * n + 7) / 8 * 8, elem = fp32 ? sizeof(float) : sizeof(double);
-  TripleVectors& own = triple_vec_[fp32];
-  if (!own.V) own.V = alloc<char>((static_cast<size_t>(max_restart_) + 1) * ld * elem);
-  if (!own.r) own.r = alloc<char>(ld * elem);
+  const TripleVectors& own = triple_vec_[fp32];
   KWork t = w;
   t.n = 3 * dm.Nc;
   t.ncase = t.rep = 3;
-  t.ld = ld;
+  t.ld = (3 * static_cast<size_t>(dm.Nc) + 7) / 8 * 8;
   for (int r = 0; r < 5; ++r) t.tiles[r] = triple_.tiles[r];
   t.V = own.V;
   t.r = own.r;
@@ -965,8 +1039,6 @@ KWork Context::triple_work(const KWork& w, bool fp32) {
   t.box_count = triple_.box_count;
   t.timer = nullptr;  // products of three vectors are not what it times
   if (w.ilu) {
-    if (!own.ilu_zl) own.ilu_zl = alloc<char>(6 * n * elem);
-    if (!own.ilu_zu) own.ilu_zu = alloc<char>(6 * n * elem);
     t.ilu_zl = own.ilu_zl;
     t.ilu_zu = own.ilu_zu;
   }
@@ -1174,14 +1246,14 @@ void Context::ensure_sell() {
     sell_pattern(dm.Nc, mesh.rowptr.data(), mesh.col.data(), kSellSigma[v], ptr, row, col, src);
     SellPat pt;
     pt.slots = src.size();
-    pt.ptr = upload(allocs_, ptr, stream);
-    pt.row = upload(allocs_, row, stream);
-    pt.col = upload(allocs_, col, stream);
-    pt.src = upload(allocs_, src, stream);
+    pt.ptr = upload(ptr);
+    pt.row = upload(row);
+    pt.col = upload(col);
+    pt.src = upload(src);
     std::vector<int> scase;
     if (ncase > 1) {
       scase = slice_cases(ptr, row);
-      pt.scase = upload(allocs_, scase, stream);
+      pt.scase = upload(scase);
     }
     sync();  // host staging vectors go out of scope
     kwork_.sell[v] = kwork32_.sell[v] = pt;
@@ -1262,21 +1334,21 @@ void Context::ensure_order() {
     ident[v] = true;
     for (int p = 0; p < n && ident[v]; ++p) ident[v] = srow[v][p] == p;
   }
-  ord_pos_ = upload(allocs_, pos, stream);
-  ord_row_ = upload(allocs_, row, stream);
-  ord_rowptr_ = upload(allocs_, rp, stream);
-  ord_col_ = upload(allocs_, col, stream);
-  ord_diag_ = upload(allocs_, dg, stream);
-  ord_src_ = upload(allocs_, src, stream);
+  ord_pos_ = upload(pos);
+  ord_row_ = upload(row);
+  ord_rowptr_ = upload(rp);
+  ord_col_ = upload(col);
+  ord_diag_ = upload(dg);
+  ord_src_ = upload(src);
   a32o_ = alloc<float>(nnz);
   for (int v = 0; v < kSellVariants; ++v) {
     SellPat pt;
     pt.slots = ssrc[v].size();
-    pt.ptr = upload(allocs_, ptr[v], stream);
-    pt.row = ident[v] ? nullptr : upload(allocs_, srow[v], stream);
-    pt.col16 = upload(allocs_, off[v], stream);
-    pt.src = upload(allocs_, ssrc[v], stream);  // positions in the ordered CSR
-    if (ncase > 1) pt.scase = upload(allocs_, slice_cases(ptr[v], srow[v]), stream);
+    pt.ptr = upload(ptr[v]);
+    pt.row = ident[v] ? nullptr : upload(srow[v]);
+    pt.col16 = upload(off[v]);
+    pt.src = upload(ssrc[v]);  // positions in the ordered CSR
+    if (ncase > 1) pt.scase = upload(slice_cases(ptr[v], srow[v]));
     osell_[v] = pt;
   }
   sync();  // host staging vectors go out of scope

@@ -98,8 +98,13 @@ class Context {
   const TuneReport& tune_report(int precision) const { return precision ? kwork32_.report : kwork_.report; }
 
  private:
+  // device memory of the context; where there is none left, the three momentum
+  // components' vectors are given back first, then DeviceMemoryError is thrown
+  void* device_bytes(size_t bytes);
   template <class T>
   T* alloc(size_t n);
+  template <class Vec>
+  auto upload(const Vec& v);
   void upload_mesh();
   std::vector<int> slice_cases(const std::vector<int>& ptr, const std::vector<int>& srow) const;
   void compute_geometry();
@@ -107,7 +112,8 @@ class Context {
   void free_all();
   int run_solve(int which_matrix, const double* b, double* x, const s355_ksp_opts& o, bool zero_guess,
                 s355_solve_info* info, int slot, bool same = false, int rep = 1);
-  void ensure_triple();
+  bool ensure_triple(bool fp32, bool ilu);
+  bool drop_triple();
   KWork triple_work(const KWork& w, bool fp32);
   Tiles make_tiles(const std::vector<int>& case_row, int tile);
   void ensure_mixed();
@@ -150,12 +156,14 @@ class Context {
   KWork kwork32_{};
   IrWork ir_{};
   // the three momentum components solved together: states and sums, and the
-  // vectors of each precision (FP64, FP32).  None is ever replaced: captured
-  // cycles hold their addresses.
+  // vectors of each precision (FP64, FP32).  None is ever replaced, and a set
+  // given back is not built again: captured cycles hold their addresses.
   KWork triple_{};
   struct TripleVectors {
     void *V = nullptr, *r = nullptr, *ilu_zl = nullptr, *ilu_zu = nullptr;
+    bool refused = false;  // no room on the device: one component after the other
   };
+  bool have_triple_ = false, building_triple_ = false;
   TripleVectors triple_vec_[2];
   double *x3_ = nullptr, *b3_ = nullptr;
   // inner order of mixed GMRES: rows in reverse Cuthill-McKee order

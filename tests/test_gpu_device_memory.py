@@ -75,3 +75,104 @@ assert rest == set(range(1, 8)), rest
 print("guards whole", probe.probe_count(), sorted(rest))
 """)
     assert "guards whole" in out and int(out.split()[2]) > 1000
+
+
+MOMENTUM = """
+case = s.cavity(12, jitter=0.1, seed=3)
+
+def context(precision, pc):
+    p = params(restart=30, pc=pc)
+    p.precision = precision
+    d = s.Solver(case, p)
+    global st
+    st = random_state(d.sizes.n_cell, d.sizes.n_bnd, d.sizes.n_face, 5)
+    push(d, {k: st[k] for k in ("U", "V", "W", "P", "R", "RUFACE")})
+    d.call("build_velocity_matrix")
+    return d
+
+def solve(d):
+    push(d, {k: st[k] for k in "UVW"})
+    its = [i["iters"] for i in d.solve_velocity(1e-8, 500)]
+    return its, [d.get(k) for k in "UVW"]
+
+def same(a, b):
+    return a[0] == b[0] and all(np.array_equal(x, y) for x, y in zip(a[1], b[1]))
+
+FORMS = [(s.FP64, s.PC_JACOBI), (s.FP64, s.PC_ILU0), (s.MIXED, s.PC_JACOBI), (s.MIXED, s.PC_ILU0)]
+"""
+
+
+def test_an_allocation_that_fails_in_the_momentum_solve(probe):
+    """Each allocation of the first solve in turn: the solve answers as ever or
+    reports the error, and the next one answers as ever."""
+    out = probe(MOMENTUM + """
+tried = 0
+for form in FORMS[:2]:
+    d = context(*form)
+    c0 = probe.probe_count()
+    want = solve(d)
+    count = probe.probe_count() - c0
+    d.close()
+    refused = 0
+    for k in range(count):
+        d = context(*form)
+        probe.probe_fail(k)
+        try:
+            assert same(solve(d), want), (form, k)
+        except s.S355Error as e:
+            assert not isinstance(e, s.NotConverged) and "memory" in str(e), (form, k, e)
+            refused += 1
+        probe.probe_fail(-1)
+        assert same(solve(d), want), (form, k)
+        assert probe.probe_damaged() == 0
+        d.close()
+        tried += 1
+    # the tables that every solve needs are missed, the common solve's are not
+    assert refused <= count - 12, (form, refused, count)
+print("allocations tried", tried)
+""")
+    assert "allocations tried" in out
+
+
+def test_no_room_for_the_common_basis(probe):
+    out = probe(MOMENTUM + """
+rows = 12 ** 3
+for precision, pc in FORMS:
+    d = context(precision, pc)
+    want = solve(d)
+    d.close()
+    d = context(precision, pc)
+    live = probe.probe_live()
+    # the basis of three components has 31 vectors of three times the rows
+    probe.probe_fail_from(31 * 3 * rows * (8 if precision == s.FP64 else 4))
+    assert same(solve(d), want)
+    probe.probe_fail_from(0)
+    assert same(solve(d), want)
+    assert probe.probe_damaged() == 0
+    d.close()
+# an allocation that finds no room while the common solve holds some: given back
+for precision in (s.FP64, s.MIXED):
+    want = {}
+    for pc in (s.PC_JACOBI, s.PC_ILU0):
+        d = context(precision, pc)
+        want[pc] = solve(d)
+        d.close()
+    d = context(precision, s.PC_JACOBI)
+    assert same(solve(d), want[s.PC_JACOBI])
+    live = probe.probe_live()
+    p = params(restart=30, pc=s.PC_ILU0)
+    p.precision = precision
+    d.set_params(p)
+    probe.probe_fail(0)
+    assert same(solve(d), want[s.PC_ILU0])
+    probe.probe_fail(-1)
+    for pc in (s.PC_JACOBI, s.PC_ILU0):
+        p = params(restart=30, pc=pc)
+        p.precision = precision
+        d.set_params(p)
+        assert same(solve(d), want[pc])
+    assert probe.probe_damaged() == 0
+    d.close()
+print("one after the other")
+""")
+    assert "one after the other" in out
