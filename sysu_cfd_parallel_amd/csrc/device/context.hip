@@ -670,11 +670,11 @@ void Context::ensure_vertices() {
   for (int i = 0; i < nc; ++i)
     for (int j = 0; j < 8; ++j)
       if (distinct(i, j)) v2c[fill[mesh.c_vert[8 * static_cast<size_t>(i) + j]]++] = i;
-  dm.v2c_ptr = upload(ptr);
-  dm.v2c = upload(v2c);
   lim_vmax_ = alloc<double>(std::max(nv, 1));
   lim_vmin_ = alloc<double>(std::max(nv, 1));
   lim_tmp_ = alloc<double>(3 * static_cast<size_t>(dm.Nc));
+  dm.v2c_ptr = upload(ptr);
+  dm.v2c = upload(v2c);  // the last: says that all of it is there
   sync();  // host staging vectors go out of scope
 }
 
@@ -682,8 +682,9 @@ void Context::ensure_vertices() {
 void Context::ensure_transient() {
   if (df.Unp) return;
   const size_t Nc = dm.Nc;
-  double** old[] = {&df.Unp, &df.Vnp, &df.Wnp, &df.Tnp, &df.TEp, &df.EDp,
-                    &df.Unp2, &df.Vnp2, &df.Wnp2, &df.Tnp2, &df.TEp2, &df.EDp2, &kw_.esrc, &kw_.ape};
+  // Unp is the last: it says that all of them are there
+  double** old[] = {&df.Vnp, &df.Wnp, &df.Tnp, &df.TEp, &df.EDp, &df.Unp2, &df.Vnp2,
+                    &df.Wnp2, &df.Tnp2, &df.TEp2, &df.EDp2, &kw_.esrc, &kw_.ape, &df.Unp};
   for (double** p : old) {
     *p = alloc<double>(Nc);
     fill_zero(*p, Nc * sizeof(double), stream);
@@ -799,7 +800,6 @@ void Context::ensure_ilu() {
 void Context::ensure_mixed() {
   if (a32_) return;
   const size_t Nc = dm.Nc;
-  a32_ = alloc<float>(dm.nnz);
   kwork32_.r = alloc<float>(Nc);
   kwork32_.lu = alloc<float>(dm.nnz);
   kwork32_.n = dm.Nc;
@@ -824,6 +824,7 @@ void Context::ensure_mixed() {
   ir_.partial_len = partial_len_;
   ir_.scal = scalars_ + 20;
   ir_.host = reinterpret_cast<double*>(static_cast<char*>(host_pinned_) + 3584);
+  a32_ = alloc<float>(dm.nnz);  // the last: says that all of it is there
 }
 
 // same: the matrix is the previous call's, unchanged, and so are its copies and
@@ -859,11 +860,11 @@ int Context::run_solve(int which, const double* b, double* x, const s355_ksp_opt
     ensure_mixed();
     kwork32_.ilu = kwork_.ilu;
     if (kwork32_.ilu && !kwork32_.ilu_lcoef) {
-      kwork32_.ilu_lcoef = alloc<float>(levels_.lower.slots);
       kwork32_.ilu_ucoef = alloc<float>(levels_.upper.slots);
       kwork32_.ilu_own = alloc<float>(dm.Nc);
       kwork32_.ilu_zl = alloc<float>(2 * static_cast<size_t>(dm.Nc));
       kwork32_.ilu_zu = alloc<float>(2 * static_cast<size_t>(dm.Nc));
+      kwork32_.ilu_lcoef = alloc<float>(levels_.lower.slots);  // the last: says that all of it is there
     }
     CsrView<float> A{dm.Nc, dm.rowptr, dm.col, dm.diag, a32_, dm.nnz};
     CsrView<double> A64{dm.Nc, dm.rowptr, dm.col, dm.diag, val, dm.nnz};
@@ -1283,8 +1284,12 @@ bool Context::use_order(const s355_ksp_opts& o) {
 // refinement, checked against the FP64 residual).
 void Context::ensure_order() {
   if (have_order_) return;
-  have_order_ = true;
   order_kind_ = par.inner_order;
+  build_order();
+  have_order_ = true;
+}
+
+void Context::build_order() {
   const int n = dm.Nc;
   std::vector<int> row;
   if (par.inner_order == 2) {

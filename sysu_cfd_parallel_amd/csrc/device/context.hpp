@@ -130,6 +130,7 @@ class Context {
   // the mixed path's FP32 assembly option
   bool fp32_assembly() const { return par.precision == S355_MIXED && par.assembly_fp32 == 1; }
   void ensure_order();
+  void build_order();
   void fill_order(const double* csr_val, bool jacobi);
   KWork ordered_work(bool all, bool filled = false);
   void tune_ordered(const CsrView<float>& Ao, int m);

@@ -107,7 +107,7 @@ def test_an_allocation_that_fails_in_the_momentum_solve(probe):
     reports the error, and the next one answers as ever."""
     out = probe(MOMENTUM + """
 tried = 0
-for form in FORMS[:2]:
+for form in FORMS:
     d = context(*form)
     c0 = probe.probe_count()
     want = solve(d)
@@ -176,3 +176,49 @@ for precision in (s.FP64, s.MIXED):
 print("one after the other")
 """)
     assert "one after the other" in out
+
+
+def test_an_allocation_that_fails_in_a_run(probe):
+    """... in the first iteration of a run that builds what the unsteady terms,
+    the limiter and the inner order need: refused with the error, and the next
+    run answers as ever."""
+    out = probe("""
+case = s.cavity(8, jitter=0.1, seed=3)
+
+def made(order):
+    p = params(restart=20, maxit=500)
+    p.precision, p.inner_order = s.MIXED, order
+    return s.Solver(case, p), p
+
+def run(d, p):
+    q = type(p).from_buffer_copy(p)
+    q.steady, q.time_scheme, q.dt, q.total_time, q.max_outer_step, q.limiter = 0, 2, 0.05, 1e6, 2, 1
+    d.set_params(q)
+    d.call("init_flow_field")
+    d.iterate(1)
+    return [d.get(k) for k in "UVWP"]
+
+for order in (1, 2):
+    d, p = made(order)
+    c0 = probe.probe_count()
+    want = run(d, p)
+    count = probe.probe_count() - c0
+    d.close()
+    for k in range(count):
+        d, p = made(order)
+        probe.probe_fail(k)
+        try:
+            got = run(d, p)
+            assert all(np.array_equal(a, b) for a, b in zip(got, want)), (order, k)
+        except s.S355Error as e:
+            assert "memory" in str(e), (order, k, e)
+        probe.probe_fail(-1)
+        got = run(d, p)
+        # (a second run starts its time step count where the first stopped)
+        assert all(np.isfinite(a).all() for a in got), (order, k)
+        if k % 4 == 0:
+            assert probe.probe_damaged() == 0
+        d.close()
+print("allocations of a run", count)
+""")
+    assert "allocations of a run" in out
