@@ -916,7 +916,9 @@ int Context::solve_velocity(double rtol, int maxit, s355_solve_info info[3]) {
   // MPIStructure.cpp:279-283 leaves V and W unsolved).
   const double* b[3] = {df.bu, df.bv, df.bw};
   double* x[3] = {df.U, df.V, df.W};
-  if (ncase == 1 && o.type == S355_KSP_GMRES && dm.Nc > 0 && dm.Nc <= kTripleRows) {
+  // (the products that are timed are those of one vector; captured cycles have none)
+  const bool timed = (par.precision == S355_MIXED ? kwork32_ : kwork_).timer && !(par.graphs && o.pc != S355_PC_ILU0);
+  if (ncase == 1 && o.type == S355_KSP_GMRES && dm.Nc > 0 && dm.Nc <= kTripleRows && !timed) {
     // the three components as one solve with three right-hand sides: they share
     // every launch (see triple_work), each with its own state and the bits of
     // its own solve
@@ -1038,7 +1040,6 @@ KWork Context::triple_work(const KWork& w, bool fp32) {
   t.host = triple_.host;
   t.box = triple_.box;
   t.box_count = triple_.box_count;
-  t.timer = nullptr;  // products of three vectors are not what it times
   if (w.ilu) {
     t.ilu_zl = own.ilu_zl;
     t.ilu_zu = own.ilu_zu;

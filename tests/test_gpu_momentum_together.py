@@ -83,3 +83,24 @@ def test_a_failed_component_leaves_the_later_ones(precision, pc):
                 assert info["iters"] == 0 and info["reason"] == 0
                 assert np.array_equal(d.get(k), st[k])
     d.close()
+
+
+@pytest.mark.parametrize("precision,order", [(s.FP64, 0), (s.MIXED, 0), (s.MIXED, 2)])
+def test_momentum_products_are_timed(precision, order):
+    """The in-solve SpMV timing sees the momentum solves, the results unchanged."""
+    p = form(precision, s.PC_JACOBI, order, 0, restart=30)
+    fields = []
+    for on in (False, True):
+        d, st = prepared(CASES["odd"], p)
+        k = 1 if precision == s.MIXED else 0
+        if on:
+            d.spmv_profile(k, 1)
+        its = [i["iters"] for i in d.solve_velocity(1e-8, 500)]
+        if on:
+            ms, n = d.spmv_profile(k, -1)
+            assert 0 < n <= sum(its) + 3 * 8 and 0 < ms < 1
+        fields.append((its, [d.get(x) for x in "UVW"]))
+        d.close()
+    assert fields[0][0] == fields[1][0]
+    for a, b in zip(fields[0][1], fields[1][1]):
+        assert np.array_equal(a, b)
