@@ -838,9 +838,8 @@ int Context::run_solve(int which, const double* b, double* x, const s355_ksp_opt
   if (par.graphs && !graphs_) graphs_ = std::make_unique<GraphCache>();
   kwork_.graphs = par.graphs ? graphs_.get() : nullptr;
   kwork32_.graphs = kwork_.graphs;
-  std::vector<KResult> together;
-  kwork_.per_case = rep > 1 ? &together : &case_info[slot];
-  kwork32_.per_case = kwork_.per_case;
+  std::vector<KResult> together;  // known to the components' own workspace alone
+  kwork_.per_case = kwork32_.per_case = rep > 1 ? nullptr : &case_info[slot];
   kwork_.prepared = kwork32_.prepared = same;
   if (rep == 1) case_info[slot].assign(ncase, KResult{});
   if (o.pc == S355_PC_ILU0) ensure_ilu();
@@ -878,14 +877,14 @@ int Context::run_solve(int which, const double* b, double* x, const s355_ksp_opt
       if (tune) tune_ordered(Ao, std::min(o.restart, kMaxRestart));
       KWork w = ordered_work(false, same);
       if (!gathered(true)) return kNoRoom;
-      if (rep > 1) w = triple_work(w, true);
+      if (rep > 1) w = triple_work(w, true, &together);
       r = ir_solve(A64, Ao, b, x, o, zero_guess, par.ir_max, par.ir_inner_rtol, w, ir_, stream);
     } else {
       if (o.type == S355_KSP_GMRES && !same && (tune || kwork32_.lanes == 0)) prepare_sell(val, true, tune);
       if (tune) autotune<float>(A, kwork32_, std::min(o.restart, kMaxRestart), stream);
       if (!gathered(true)) return kNoRoom;
       KWork w3;
-      if (rep > 1) w3 = triple_work(kwork32_, true);
+      if (rep > 1) w3 = triple_work(kwork32_, true, &together);
       r = ir_solve(A64, A, b, x, o, zero_guess, par.ir_max, par.ir_inner_rtol, rep > 1 ? w3 : kwork32_, ir_, stream);
     }
   } else {
@@ -895,7 +894,7 @@ int Context::run_solve(int which, const double* b, double* x, const s355_ksp_opt
     if (tune) autotune<double>(A, kwork_, std::min(o.restart, kMaxRestart), stream);
     if (!gathered(false)) return kNoRoom;
     KWork w3;
-    if (rep > 1) w3 = triple_work(kwork_, false);
+    if (rep > 1) w3 = triple_work(kwork_, false, &together);
     r = krylov_solve<double>(A, b, x, o, zero_guess, rep > 1 ? w3 : kwork_, stream);
   }
   if (rep > 1) {
@@ -1024,7 +1023,7 @@ bool Context::drop_triple() {
 
 // The workspace of the three momentum components' solve: the shapes, matrix
 // copies and preconditioner of w, the vectors and states of three cases.
-KWork Context::triple_work(const KWork& w, bool fp32) {
+KWork Context::triple_work(const KWork& w, bool fp32, std::vector<KResult>* records) {
   const TripleVectors& own = triple_vec_[fp32];
   KWork t = w;
   t.n = 3 * dm.Nc;
@@ -1040,6 +1039,7 @@ KWork Context::triple_work(const KWork& w, bool fp32) {
   t.host = triple_.host;
   t.box = triple_.box;
   t.box_count = triple_.box_count;
+  t.per_case = records;
   if (w.ilu) {
     t.ilu_zl = own.ilu_zl;
     t.ilu_zu = own.ilu_zu;

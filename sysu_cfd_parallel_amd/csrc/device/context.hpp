@@ -114,7 +114,7 @@ class Context {
                 s355_solve_info* info, int slot, bool same = false, int rep = 1);
   bool ensure_triple(bool fp32, bool ilu);
   bool drop_triple();
-  KWork triple_work(const KWork& w, bool fp32);
+  KWork triple_work(const KWork& w, bool fp32, std::vector<KResult>* records);
   Tiles make_tiles(const std::vector<int>& case_row, int tile);
   void ensure_mixed();
   void ensure_ilu();
