@@ -762,6 +762,13 @@ void Context::ensure_ilu() {
       w.dsrc = upload(dsrc);
       sync();
     }
+    if (ncase > 1) {
+      std::vector<int> rcase(p.n);
+      for (int c = 0; c < ncase; ++c)
+        for (int i = lay.cell[c]; i < lay.cell[c + 1]; ++i) rcase[p.pos[i]] = c;
+      w.rcase = upload(rcase);
+      sync();
+    }
   };
   {
     std::vector<int> natural(dm.Nc);

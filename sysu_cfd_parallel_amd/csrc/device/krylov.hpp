@@ -151,6 +151,7 @@ struct IluSweep {
   // upper sweep: CSR position of the pivot of the row at each position at
   // depth 0, and -1 minus it below
   const int* dsrc = nullptr;
+  const int* rcase = nullptr;  // batches: the case of the row at each position
 };
 
 // The elimination steps of ILU(0) per row, rows by level: row
