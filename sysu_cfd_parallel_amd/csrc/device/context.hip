@@ -9,6 +9,7 @@
 #include <cmath>
 #include <cstring>
 #include <exception>
+#include <future>
 #include <numeric>
 #include <stdexcept>
 #include <thread>
@@ -773,11 +774,41 @@ void Context::ensure_ilu() {
   {
     std::vector<int> natural(dm.Nc);
     std::iota(natural.begin(), natural.end(), 0);
-    const IluPlan lower = ilu_plan(dm.Nc, mesh.rowptr.data(), mesh.col.data(), mesh.diag.data(), false, natural,
-                                   lay.cell);
+    // both plans at once; the upper one waits for the lower one's rows where it
+    // orders its own.  (Above 4 M rows one after the other: their tables would
+    // take tens of gigabytes together.)
+    std::promise<void> lower_done;
+    const std::shared_future<void> lower_rows(lower_done.get_future());
+    IluPlan lower, upper;
+    std::exception_ptr upper_failed;
+    const bool at_once = dm.Nc <= (1 << 22);
+    std::thread upper_plan([&] {
+      try {
+        if (!at_once) lower_rows.wait();
+        upper = ilu_plan(
+            dm.Nc, mesh.rowptr.data(), mesh.col.data(), mesh.diag.data(), true,
+            [&]() -> const std::vector<int>& {
+              lower_rows.get();
+              return lower.rows;
+            },
+            lay.cell);
+      } catch (...) {
+        upper_failed = std::current_exception();
+      }
+    });
+    Joined upper_joined{upper_plan};
+    try {
+      lower = ilu_plan(
+          dm.Nc, mesh.rowptr.data(), mesh.col.data(), mesh.diag.data(), false,
+          [&]() -> const std::vector<int>& { return natural; }, lay.cell);
+      lower_done.set_value();
+    } catch (...) {
+      lower_done.set_exception(std::current_exception());
+      throw;
+    }
     put(levels_.lower, lower, false);
-    const IluPlan upper = ilu_plan(dm.Nc, mesh.rowptr.data(), mesh.col.data(), mesh.diag.data(), true, lower.rows,
-                                   lay.cell);
+    upper_plan.join();
+    if (upper_failed) std::rethrow_exception(upper_failed);
     put(levels_.upper, upper, true);
     std::vector<int> l2u(dm.Nc);
     for (int q = 0; q < dm.Nc; ++q) l2u[q] = upper.pos[lower.rows[q]];

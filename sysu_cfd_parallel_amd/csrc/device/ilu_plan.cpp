@@ -13,8 +13,9 @@ constexpr long kMost = 0x7fffffffL;
 
 }  // namespace
 
-IluPlan ilu_plan(int n, const int* rowptr, const int* col, const int* diag, bool upper, const std::vector<int>& order,
-                 const std::vector<int>& cases, int merge_levels, int merge_rows) {
+IluPlan ilu_plan(int n, const int* rowptr, const int* col, const int* diag, bool upper,
+                 const std::function<const std::vector<int>&()>& order, const std::vector<int>& cases, int merge_levels,
+                 int merge_rows) {
   if (n > kMost / 2) throw std::invalid_argument("ILU(0) sweeps above 32-bit indices");
   if (merge_levels < 1 || merge_levels > kMergeLevels) throw std::invalid_argument("ilu_plan: merge_levels");
   // the merged rows' terms fit 32-bit indices below this many rows on any mesh
@@ -139,7 +140,7 @@ IluPlan ilu_plan(int n, const int* rowptr, const int* col, const int* diag, bool
   out.pos.resize(n);
   {
     std::vector<int> at(kptr.begin(), kptr.end() - 1);
-    for (int i : order) {
+    for (int i : order()) {
       const int p = at[key(i)]++;
       out.rows[p] = i;
       out.pos[i] = p;

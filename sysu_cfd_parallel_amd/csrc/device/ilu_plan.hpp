@@ -2,6 +2,7 @@
 // of them sums.
 #pragma once
 #include <cstddef>
+#include <functional>
 #include <memory>
 #include <vector>
 
@@ -91,9 +92,18 @@ struct IluPlan {
 
 // The plan of the lower (strictly lower entries) or upper sweep of a CSR
 // pattern with sorted columns; order is the order rows keep inside a group
-// and class, cases the first row of each case and n.  Throws
-// std::invalid_argument where a table passes 32-bit indices.
-IluPlan ilu_plan(int n, const int* rowptr, const int* col, const int* diag, bool upper, const std::vector<int>& order,
-                 const std::vector<int>& cases, int merge_levels = kMergeLevels, int merge_rows = kMergeRows);
+// and class (as a function: asked for once the terms are known, so that the upper
+// sweep's, the lower plan's rows, can be built at the same time), cases the
+// first row of each case and n.  Throws std::invalid_argument where a table
+// passes 32-bit indices.
+IluPlan ilu_plan(int n, const int* rowptr, const int* col, const int* diag, bool upper,
+                 const std::function<const std::vector<int>&()>& order, const std::vector<int>& cases,
+                 int merge_levels = kMergeLevels, int merge_rows = kMergeRows);
+inline IluPlan ilu_plan(int n, const int* rowptr, const int* col, const int* diag, bool upper,
+                        const std::vector<int>& order, const std::vector<int>& cases,
+                        int merge_levels = kMergeLevels, int merge_rows = kMergeRows) {
+  return ilu_plan(
+      n, rowptr, col, diag, upper, [&]() -> const std::vector<int>& { return order; }, cases, merge_levels, merge_rows);
+}
 
 }  // namespace s355
