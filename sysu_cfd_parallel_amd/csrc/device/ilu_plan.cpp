@@ -1,7 +1,10 @@
 #include "ilu_plan.hpp"
 
+#include <sys/mman.h>
+
 #include <algorithm>
 #include <memory>
+#include <new>
 #include <stdexcept>
 
 #include "../mesh/parallel.hpp"
@@ -10,8 +13,19 @@ namespace s355 {
 namespace {
 
 constexpr long kMost = 0x7fffffffL;
+constexpr size_t kHuge = size_t(1) << 21;
 
 }  // namespace
+
+void IntArray::resize(size_t m) {
+  const size_t bytes = std::max<size_t>(m, 1) * sizeof(int);
+  const bool huge = bytes >= 2 * kHuge;
+  int* q = static_cast<int*>(huge ? std::aligned_alloc(kHuge, (bytes + kHuge - 1) / kHuge * kHuge) : std::malloc(bytes));
+  if (!q) throw std::bad_alloc();
+  if (huge) madvise(q, bytes, MADV_HUGEPAGE);
+  p.reset(q);
+  n = m;
+}
 
 IluPlan ilu_plan(int n, const int* rowptr, const int* col, const int* diag, bool upper,
                  const std::function<const std::vector<int>&()>& order, const std::vector<int>& cases, int merge_levels,
@@ -92,25 +106,27 @@ IluPlan ilu_plan(int n, const int* rowptr, const int* col, const int* diag, bool
           const int i = list[k];
           const long s = start[i];
           int m = 0, pairs = 0, steps = 0;
-          auto term = [&](int c) {
-            int u = 0;
-            while (u < m && code[s + u] != c) ++u;
-            if (u == m) {
-              code[s + m] = c;
-              src[s + m] = -1;
-              ++m;
-            }
-            return u;
+          int* const codes = code.data() + s;
+          // the term of code c, looked for among the first `before` (the codes of
+          // one reference differ from each other)
+          auto term = [&](int c, int before) {
+            int u = -1;
+            for (int v = 0; v < before; ++v) u = std::max(u, codes[v] == c ? v : -1);
+            if (u >= 0) return u;
+            codes[m] = c;
+            src[s + m] = -1;
+            return m++;
           };
           for (int x = first(i); x < last(i); ++x) {
             const int j = col[x];
             if (grp[j] != grp[i]) {
-              src[s + term(n + j)] = x;
+              src[s + term(n + j, m)] = x;
               continue;
             }
             ++steps;
+            const int before = m;
             for (int y = -1; y < count[j]; ++y) {  // -1: row j's own input
-              pr[s + pairs] = term(y < 0 ? j : code[start[j] + y]);
+              pr[s + pairs] = term(y < 0 ? j : code[start[j] + y], before);
               pq[s + pairs] = y;
               ++pairs;
             }
@@ -233,9 +249,9 @@ IluPlan ilu_plan(int n, const int* rowptr, const int* col, const int* diag, bool
         for (int x = first(i); x < last(i); ++x) {
           const int j = col[x];
           if (grp[j] != grp[i]) continue;
-          const int pj = out.pos[j];
+          const int pj = out.pos[j], most_terms = count[j];
           out.p[x0] = x;
-          for (int y = -1; y < count[j]; ++y, ++at, ++from) {
+          for (int y = -1; y < most_terms; ++y, ++at, ++from) {
             out.r[at] = out.slot(pi, pr[from]);
             out.q[at] = pq[from] < 0 ? -1 - pj : out.slot(pj, pq[from]);
           }

@@ -2,6 +2,7 @@
 // of them sums.
 #pragma once
 #include <cstddef>
+#include <cstdlib>
 #include <functional>
 #include <memory>
 #include <vector>
@@ -51,15 +52,17 @@ struct IluSub {
   int p0, nrows, width, cls;
 };
 
-// n ints that are written before they are read (a vector would first fill them)
+// n ints that are written before they are read (a vector would first fill them).
+// Large ones ask for 2 MiB pages: the plan of 331,776 tetrahedra touches some 80 MB
+// for the first time, by 4 KiB pages from many threads at once.
 struct IntArray {
   using value_type = int;
-  std::unique_ptr<int[]> p;
+  struct Free {
+    void operator()(int* q) const { std::free(q); }
+  };
+  std::unique_ptr<int[], Free> p;
   size_t n = 0;
-  void resize(size_t m) {
-    p.reset(new int[m ? m : 1]);
-    n = m;
-  }
+  void resize(size_t m);
   size_t size() const { return n; }
   bool empty() const { return n == 0; }
   int* data() { return p.get(); }
@@ -78,7 +81,10 @@ struct IluPlan {
   std::vector<int> depth;    // per position: 0 where no entry refers to the row's own group
   // per position: its first slot, its lanes, the distance of its terms of one lane
   std::vector<int> slot0, lanes, stride;
-  int slot(int q, int u) const { return slot0[q] + u / lanes[q] * stride[q] + u % lanes[q]; }
+  int slot(int q, int u) const {  // (lanes: 1, 4 or 16)
+    const int shift = lanes[q] == 1 ? 0 : lanes[q] == 4 ? 2 : 4;
+    return slot0[q] + (u >> shift) * stride[q] + (u & (lanes[q] - 1));
+  }
   // per slot: buf index (padding: the row's own input), and where its
   // coefficient starts from: the CSR entry a_ij (coefficient -a_ij) or -1 (0)
   IntArray col, src;
