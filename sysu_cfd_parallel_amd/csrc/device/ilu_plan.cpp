@@ -27,14 +27,18 @@ void IntArray::resize(size_t m) {
   n = m;
 }
 
-IluPlan ilu_plan(int n, const int* rowptr, const int* col, const int* diag, bool upper,
-                 const std::function<const std::vector<int>&()>& order, const std::vector<int>& cases, int merge_levels,
-                 int merge_rows) {
+namespace {
+
+// a table of the plan would pass its bound
+struct TooLarge : std::invalid_argument {
+  using std::invalid_argument::invalid_argument;
+};
+
+IluPlan build(int n, const int* rowptr, const int* col, const int* diag, bool upper,
+              const std::function<const std::vector<int>&()>& order, const std::vector<int>& cases, int merge_levels,
+              int merge_rows, long most_entries) {
   if (n > kMost / 2) throw std::invalid_argument("ILU(0) sweeps above 32-bit indices");
   if (merge_levels < 1 || merge_levels > kMergeLevels) throw std::invalid_argument("ilu_plan: merge_levels");
-  // the merged rows' terms fit 32-bit indices below this many rows on any mesh
-  // of hexahedra and tetrahedra; above it the levels are large anyway
-  if (n > (1 << 26)) merge_levels = 1;
   IluPlan out;
   out.n = n;
   auto first = [&](int i) { return upper ? diag[i] + 1 : rowptr[i]; };
@@ -95,6 +99,7 @@ IluPlan ilu_plan(int n, const int* rowptr, const int* col, const int* diag, bool
   // referred to, -1 its own input), one run per reference in CSR order.
   std::vector<long> start(static_cast<size_t>(n) + 1, 0);
   for (int i = 0; i < n; ++i) start[i + 1] = start[i] + most[i];
+  if (merge_levels > 1 && start[n] > most_entries) throw TooLarge("ILU(0) merged rows");
   IntArray code, src, pr, pq;
   for (IntArray* x : {&code, &src, &pr, &pq}) x->resize(start[n]);
   std::vector<int> count(n), nstep(n, 0), npair(n, 0);
@@ -180,8 +185,7 @@ IluPlan ilu_plan(int n, const int* rowptr, const int* col, const int* diag, bool
       else
         width[k] = (width[k] + batch - 1) / batch * batch;
       out.subs.push_back(IluSub{slots, p0, nr, width[k], c});
-      if (slots + static_cast<long>(width[k]) * nr > kMost)
-        throw std::invalid_argument("ILU(0) sweep slots above 32-bit indices");
+      if (slots + static_cast<long>(width[k]) * nr > kMost) throw TooLarge("ILU(0) sweep slots above 32-bit indices");
       for (int p = p0; p < p0 + nr; ++p) {
         out.slot0[p] = static_cast<int>(slots + static_cast<long>(p - p0) * lanes);
         out.lanes[p] = lanes;
@@ -232,7 +236,7 @@ IluPlan ilu_plan(int n, const int* rowptr, const int* col, const int* diag, bool
     const int i = out.rows[out.later[k]];
     steps += nstep[i];
     pairs[k + 1] = pairs[k] + npair[i];
-    if (steps > kMost || pairs[k + 1] > kMost) throw std::invalid_argument("ILU(0) sweep steps above 32-bit indices");
+    if (steps > kMost || pairs[k + 1] > kMost) throw TooLarge("ILU(0) sweep steps above 32-bit indices");
     out.sptr[k + 1] = static_cast<int>(steps);
   }
   out.p.resize(steps);
@@ -260,6 +264,19 @@ IluPlan ilu_plan(int n, const int* rowptr, const int* col, const int* diag, bool
       },
       1 << 12);
   return out;
+}
+
+}  // namespace
+
+IluPlan ilu_plan(int n, const int* rowptr, const int* col, const int* diag, bool upper,
+                 const std::function<const std::vector<int>&()>& order, const std::vector<int>& cases, int merge_levels,
+                 int merge_rows, long most_entries) {
+  try {
+    return build(n, rowptr, col, diag, upper, order, cases, merge_levels, merge_rows, most_entries);
+  } catch (const TooLarge&) {
+    if (merge_levels == 1) throw;
+    return build(n, rowptr, col, diag, upper, order, cases, 1, merge_rows, most_entries);
+  }
 }
 
 }  // namespace s355

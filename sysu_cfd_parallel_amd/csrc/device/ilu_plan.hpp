@@ -36,6 +36,11 @@ namespace s355 {
 constexpr int kMergeLevels = 8;
 constexpr int kMergeTerms = 200;
 constexpr int kMergeRows = 65536;
+// Entries that the merged rows of one plan may have, counted without looking for
+// equal ones: 16 bytes each while the plan is built, so 16 GB, and 32-bit indices
+// hold the tables.  Long thin meshes, whose levels are small however many
+// rows they have, come there (a duct of 4000 x 32 x 32 hexahedra has 35 entries a row).
+constexpr long kMergeEntries = 1L << 30;
 // Rows of a launch come in classes of term counts, each padded to a width the
 // kernel is compiled for.  A row of many terms is shared by 4 or 16 lanes, so
 // that no lane's chain of loads is longer than one batch; the last class takes
@@ -100,16 +105,19 @@ struct IluPlan {
 // pattern with sorted columns; order is the order rows keep inside a group
 // and class (as a function: asked for once the terms are known, so that the upper
 // sweep's, the lower plan's rows, can be built at the same time), cases the
-// first row of each case and n.  Throws std::invalid_argument where a table
-// passes 32-bit indices.
+// first row of each case and n.  Where merged rows would take more than
+// most_entries entries, or a table passes 32-bit indices, nothing is merged; throws
+// std::invalid_argument where a table passes them all the same.
 IluPlan ilu_plan(int n, const int* rowptr, const int* col, const int* diag, bool upper,
                  const std::function<const std::vector<int>&()>& order, const std::vector<int>& cases,
-                 int merge_levels = kMergeLevels, int merge_rows = kMergeRows);
+                 int merge_levels = kMergeLevels, int merge_rows = kMergeRows, long most_entries = kMergeEntries);
 inline IluPlan ilu_plan(int n, const int* rowptr, const int* col, const int* diag, bool upper,
                         const std::vector<int>& order, const std::vector<int>& cases,
-                        int merge_levels = kMergeLevels, int merge_rows = kMergeRows) {
+                        int merge_levels = kMergeLevels, int merge_rows = kMergeRows,
+                        long most_entries = kMergeEntries) {
   return ilu_plan(
-      n, rowptr, col, diag, upper, [&]() -> const std::vector<int>& { return order; }, cases, merge_levels, merge_rows);
+      n, rowptr, col, diag, upper, [&]() -> const std::vector<int>& { return order; }, cases, merge_levels, merge_rows,
+      most_entries);
 }
 
 }  // namespace s355
