@@ -825,21 +825,27 @@ void Context::ensure_ilu() {
     levels_.steps.q = upload(sq);
     sync();  // host staging vectors go out of scope
   }
-  kwork_.lu = alloc<double>(dm.nnz);
-  kwork_.ilu_lcoef = alloc<double>(levels_.lower.slots);
-  kwork_.ilu_ucoef = alloc<double>(levels_.upper.slots);
-  kwork_.ilu_own = alloc<double>(dm.Nc);
-  kwork_.ilu_zl = alloc<double>(2 * static_cast<size_t>(dm.Nc));
-  kwork_.ilu_zu = alloc<double>(2 * static_cast<size_t>(dm.Nc));
-  kwork_.ilu = &levels_;
   have_levels_ = true;
+}
+
+// the factors, coefficients and sweep buffers of one precision
+template <class T>
+void Context::ensure_ilu_work(KWork& w) {
+  ensure_ilu();
+  w.ilu = &levels_;
+  if (w.ilu_lcoef) return;
+  w.lu = alloc<T>(dm.nnz);
+  w.ilu_ucoef = alloc<T>(levels_.upper.slots);
+  w.ilu_own = alloc<T>(dm.Nc);
+  w.ilu_zl = alloc<T>(2 * static_cast<size_t>(dm.Nc));
+  w.ilu_zu = alloc<T>(2 * static_cast<size_t>(dm.Nc));
+  w.ilu_lcoef = alloc<T>(levels_.lower.slots);  // the last: says that all of it is there
 }
 
 void Context::ensure_mixed() {
   if (a32_) return;
   const size_t Nc = dm.Nc;
   kwork32_.r = alloc<float>(Nc);
-  kwork32_.lu = alloc<float>(dm.nnz);
   kwork32_.n = dm.Nc;
   kwork32_.mmax = max_restart_;
   kwork32_.ld = kwork_.ld;
@@ -880,7 +886,6 @@ int Context::run_solve(int which, const double* b, double* x, const s355_ksp_opt
   kwork_.per_case = kwork32_.per_case = rep > 1 ? nullptr : &case_info[slot];
   kwork_.prepared = kwork32_.prepared = same;
   if (rep == 1) case_info[slot].assign(ncase, KResult{});
-  if (o.pc == S355_PC_ILU0) ensure_ilu();
   // after everything else the solve allocates
   auto gathered = [&](bool fp32) {
     if (rep == 1) return true;
@@ -895,14 +900,7 @@ int Context::run_solve(int which, const double* b, double* x, const s355_ksp_opt
   if (par.precision == S355_MIXED) {
     // FP32 inner solves on the rounded matrix inside FP64 refinement
     ensure_mixed();
-    kwork32_.ilu = kwork_.ilu;
-    if (kwork32_.ilu && !kwork32_.ilu_lcoef) {
-      kwork32_.ilu_ucoef = alloc<float>(levels_.upper.slots);
-      kwork32_.ilu_own = alloc<float>(dm.Nc);
-      kwork32_.ilu_zl = alloc<float>(2 * static_cast<size_t>(dm.Nc));
-      kwork32_.ilu_zu = alloc<float>(2 * static_cast<size_t>(dm.Nc));
-      kwork32_.ilu_lcoef = alloc<float>(levels_.lower.slots);  // the last: says that all of it is there
-    }
+    if (o.pc == S355_PC_ILU0) ensure_ilu_work<float>(kwork32_);
     CsrView<float> A{dm.Nc, dm.rowptr, dm.col, dm.diag, a32_, dm.nnz};
     CsrView<double> A64{dm.Nc, dm.rowptr, dm.col, dm.diag, val, dm.nnz};
     const bool tune = par.autotune && o.type == S355_KSP_GMRES && !kwork32_.tuned;
@@ -926,6 +924,7 @@ int Context::run_solve(int which, const double* b, double* x, const s355_ksp_opt
       r = ir_solve(A64, A, b, x, o, zero_guess, par.ir_max, par.ir_inner_rtol, rep > 1 ? w3 : kwork32_, ir_, stream);
     }
   } else {
+    if (o.pc == S355_PC_ILU0) ensure_ilu_work<double>(kwork_);
     CsrView<double> A{dm.Nc, dm.rowptr, dm.col, dm.diag, val, dm.nnz};
     const bool tune = par.autotune && o.type == S355_KSP_GMRES && !kwork_.tuned;
     if (o.type == S355_KSP_GMRES && !same && (tune || kwork_.lanes == 0)) prepare_sell(val, false, tune);

@@ -118,6 +118,8 @@ class Context {
   Tiles make_tiles(const std::vector<int>& case_row, int tile);
   void ensure_mixed();
   void ensure_ilu();
+  template <class T>
+  void ensure_ilu_work(KWork& w);
   void ensure_sell();
   void prepare_sell(const double* csr_val, bool fp32, bool all);
   void grad(int nf, const double* const* phi, const double* const* bphi, double* const* out);

@@ -51,6 +51,11 @@ int hipFree(void* p) {
 // allocations asked for so far
 long probe_count() { return count; }
 long probe_live() { return static_cast<long>(live.size()); }
+long probe_bytes() {
+  long n = 0;
+  for (const auto& a : live) n += static_cast<long>(a.second);
+  return n;
+}
 // the k-th allocation from now fails (-1: none)
 void probe_fail(long k) { fail_at = k < 0 ? -1 : count + k; }
 // every allocation of at least this many bytes fails (0: none)

@@ -15,7 +15,7 @@ HEAD = """
 import ctypes as C, sys
 probe = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
 probe.probe_fail_from.argtypes = [C.c_size_t]
-for f in ("probe_count", "probe_live", "probe_damaged"):
+for f in ("probe_count", "probe_live", "probe_damaged", "probe_bytes"):
     getattr(probe, f).restype = C.c_long
 probe.probe_fail.argtypes = [C.c_long]
 sys.path[:0] = [sys.argv[2], sys.argv[2] + "/tests"]
@@ -222,3 +222,23 @@ for order in (1, 2):
 print("allocations of a run", count)
 """)
     assert "allocations of a run" in out
+
+
+def test_mixed_ilu_holds_its_own_precision_only(probe):
+    """What ILU(0) adds to a mixed context is less than what it adds to an FP64
+    one: the tables and FP32 coefficients, no FP64 ones."""
+    out = probe(MOMENTUM + """
+added = {}
+for precision in (s.FP64, s.MIXED):
+    held = {}
+    for pc in (s.PC_JACOBI, s.PC_ILU0):
+        b0 = probe.probe_bytes()
+        d = context(precision, pc)
+        solve(d)
+        held[pc] = probe.probe_bytes() - b0
+        d.close()
+    added[precision] = held[s.PC_ILU0] - held[s.PC_JACOBI]
+assert 0 < added[s.MIXED] < added[s.FP64], added
+print("added", added)
+""")
+    assert "added" in out
