@@ -11,7 +11,8 @@ pytestmark = pytest.mark.gpu
 
 CASES = {
     "one": lambda: s.cavity(1),
-    "odd": lambda: s.channel(11, 7, 5, jitter=0.1, split=0.35, seed=3, re=600.0),  # 1040 rows
+    "odd": lambda: s.channel(11, 7, 5, jitter=0.1, split=0.35, seed=3, re=600.0),  # 1040 rows, the last tile short
+    "unaligned": lambda: s.channel(9, 7, 5, jitter=0.1, re=400.0),  # 315 rows: V and W start off 16 bytes
     "hex": lambda: s.channel(11, 7, 5, jitter=0.1, re=400.0),
     "tets": lambda: s.step(2, downstream=6.0, tets=True, turbulent=False, re=400.0),
 }

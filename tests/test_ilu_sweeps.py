@@ -113,14 +113,34 @@ def test_sweep_plan_equals_the_triangular_solve(probe, name, levels, rows, upper
             assert np.array_equal(z1, z[a:e])
 
 
+def shuffled(case, seed):
+    """The same mesh, its cells numbered at random: few levels of many rows."""
+    perm = np.arange(len(case.etype))
+    vol = np.flatnonzero(case.etype >= 4)
+    perm[vol] = np.random.default_rng(seed).permutation(vol)
+    verts = [case.vidx[case.vptr[e]:case.vptr[e + 1]] for e in perm]
+    ptr = np.concatenate([[0], np.cumsum([len(v) for v in verts])]).astype(np.int32)
+    return s.CaseData(case.xyz, case.etype[perm].copy(), case.tag[perm].copy(), ptr,
+                      np.concatenate(verts).astype(np.int32), case.regions, dict(case.meta))
+
+
+def widest_level(ptr, col, diag):
+    lev = [0] * len(diag)
+    ptr, col, diag = ptr.tolist(), col.tolist(), diag.tolist()
+    for i in range(len(lev)):
+        lev[i] = max((lev[j] + 1 for j in col[ptr[i]:diag[i]]), default=0)
+    return int(np.bincount(lev).max())
+
+
 GPU_CASES = {
     "one_cell": lambda: s.cavity(1),
     "cavity3": lambda: s.cavity(3),
     "cavity17": lambda: s.cavity(17, jitter=0.1, seed=2),
     "tets": lambda: s.cavity(6, tets=True, jitter=0.1, seed=3),
     "split": lambda: s.channel(20, 9, 11, jitter=0.12, split=0.25, seed=6, re=400.0),
-    # levels of more rows than a launch merges
     "large": lambda: s.channel(120, 60, 60, jitter=0.1),
+    # levels of more rows than a launch merges (and workgroups of 256 threads)
+    "wide": lambda: shuffled(s.cavity(40, tets=True, jitter=0.1, seed=5), 1),
 }
 
 
@@ -128,7 +148,8 @@ GPU_CASES = {
 @pytest.mark.parametrize("precision", [s.FP64, s.MIXED])
 @pytest.mark.parametrize("name", sorted(GPU_CASES))
 def test_first_preconditioned_step_matches_the_oracle(name, precision):
-    """One GMRES iteration from a zero guess: x is a multiple of (LU)^-1 b."""
+    """One GMRES iteration from a zero guess: x is a multiple of (LU)^-1 b, for
+    each of the three momentum components."""
     from oracle.pyoracle import pc_apply
 
     case = GPU_CASES[name]()
@@ -140,13 +161,16 @@ def test_first_preconditioned_step_matches_the_oracle(name, precision):
     push(d, {k: st[k] for k in ("U", "V", "W", "P", "R", "APR", "DPDX", "RUFACE")})
     d.call("build_velocity_matrix")  # momentum: no null space, three right-hand sides
     push(d, {k: np.zeros(d.sizes.n_cell) for k in ("U", "V", "W")})
-    try:
-        d.solve_velocity(1e-30, 1)
-    except s.NotConverged:
-        pass
-    z = pc_apply(d.ints("CSR_ROWPTR"), d.ints("CSR_COL"), d.get("AU"), s.PC_ILU0, d.get("BU_RHS"))
-    x = d.get("U")
-    scale = (x @ z) / (z @ z)
-    # FP32 factors and sweeps: a few roundings per row, condition below 1e2
-    assert rel_err(x, scale * z) <= (1e-11 if precision == s.FP64 else 3e-5)
+    # a preconditioned step takes more than a hundredth off the residual
+    info = d.solve_velocity(0.99, 1)
+    assert [i["iters"] for i in info] == [1, 1, 1]
+    pattern = d.ints("CSR_ROWPTR"), d.ints("CSR_COL"), d.ints("CSR_DIAG")
+    if name == "wide":
+        assert widest_level(*pattern) > 65536
+    for k in "UVW":
+        z = pc_apply(pattern[0], pattern[1], d.get("AU"), s.PC_ILU0, d.get("B%s_RHS" % k))
+        x = d.get(k)
+        scale = (x @ z) / (z @ z)
+        # FP32 factors and sweeps: a few roundings per row, condition below 1e2
+        assert rel_err(x, scale * z) <= (1e-11 if precision == s.FP64 else 3e-5), k
     d.close()
