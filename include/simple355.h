@@ -98,7 +98,9 @@ typedef struct s355_params {
   int autotune;         /* 1: on the first GMRES solve of each precision, time
                            the SpMV lanes per row and the rows per thread of the
                            Gram-Schmidt kernels and keep the fastest (cached per
-                           process and system shape); 0: fixed heuristics */
+                           process and system shape; one case of up to 65,536
+                           rows takes SELL-64 and one row per thread, only its
+                           matrix loads are timed); 0: fixed heuristics */
   int graphs;           /* 1: capture each GMRES restart cycle as a hipGraph
                            and replay it; 0: launch kernel by kernel */
   int solve_energy;     /* SolveEnergy: 1 = UpdateEnergy after the k-epsilon step */
@@ -424,7 +426,9 @@ int s355_kernel_shapes(s355_ctx* ctx, int lanes[2], int nt[2], int rows[2], int 
  * events on the context stream, without added synchronisation.  mode 1
  * starts (and resets), 0 reads, -1 reads and stops; *avg_ms is the mean
  * launch time, *count the launches timed.  Solves replayed from captured
- * graphs are not timed.  No reference counterpart. */
+ * graphs are not timed.  While products are timed, the momentum components
+ * of a case are solved one after the other (the same bits), so that each
+ * launch is one product.  No reference counterpart. */
 int s355_spmv_profile(s355_ctx* ctx, int precision, int mode, double* avg_ms, int* count);
 
 /* Sets the kernel shapes of one precision's GMRES solves explicitly (the
@@ -441,7 +445,11 @@ int s355_set_kernel_shapes(s355_ctx* ctx, int precision, int lanes, int nt, int 
  * for SELL-64 sorted in windows of 64, 512, 4096 rows; gs_ms[r] for 2^r rows
  * per thread (multi-dot, its final reduction and the Gram-Schmidt update,
  * averaged over the Arnoldi steps a quarter, half and three quarters into the
- * restart cycle; *gs_it is the middle one); -1 where not timed.  No reference
+ * restart cycle; *gs_it is the middle one); -1 where not timed.  One case of
+ * up to 65,536 rows is timed in the one form it takes (SELL-64, windows of 64
+ * rows or the inner order's, one row per thread): spmv_ms then holds the
+ * product with its dots, at the step half into the cycle, gs_ms[0] the rest
+ * of the Arnoldi step (sums and update) at the three steps.  No reference
  * counterpart. */
 int s355_tune_report(s355_ctx* ctx, int precision, double spmv_ms[16], double gs_ms[5], int* gs_it);
 

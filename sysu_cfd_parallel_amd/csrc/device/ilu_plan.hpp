@@ -25,14 +25,29 @@ namespace s355 {
 //
 // A group ends where it would pass kMergeRows rows (such launches are bound by
 // bytes, and merged rows read more of them) or where a row could pass
-// kMergeTerms terms (counted without looking for equal ones).  Pressure solves
-// (CG, 331,776 tetrahedra, FP64, 54 levels; mixed GMRES, 310,000 hexahedra, 134
-// levels), a k-epsilon step (98,304 tetrahedra) and a momentum phase (331,776, a
-// factorisation for 9 steps) by levels, rows and terms, in ms: no merging 131.7,
-// 162.3, 90.6, 13.2; 6, 65536, 96: 60.2, 62.3, 39.6, 4.68; 8, 65536, 160: 55.6,
-// 56.0, 38.0, 4.76; 8, 65536, 300: 55.2, 51.4, 38.9, 4.80; 12, 65536, 300: 52.8,
-// 50.4, 37.6, 5.30; 16, 65536, 1000: 51.9, 48.4, 40.2, 6.31.  Taken: 8, 65536, 200
-// (55.7, 56.7, 39.1, 4.82); more terms save little and lengthen the plan.
+// kMergeTerms terms (counted without looking for equal ones).  One build, four
+// repeated passes: pressure solves by CG on 331,776 tetrahedra in FP64 (54 levels)
+// and mixed GMRES(50) on 310,000 hexahedra (134 levels), a momentum phase with its
+// factorisation on the tetrahedra, a pressure solve of 512 cavities of 16^3 as a
+// batch in FP64, ms:
+//   levels, terms   CG     GMRES  momentum  batch
+//    1              154.6  139.1  7.7       22.2
+//    4,  200         73.6   45.4  4.4       21.1
+//    6,  100         62.1   43.1  4.1       21.2
+//    8,   60         64.3   52.9  4.1       20.7
+//    8,  100         59.7   42.6  4.0       21.2
+//    8,  200         56.8   38.1  3.9       22.1
+//    8,  300         56.8   35.4  3.9       22.7
+//   12,  300         54.0   34.6  3.9       22.7
+//   16, 1000         51.7   32.3  4.0       25.1
+// (65,536 rows).  Taken: 8, 200; what more terms give a single case a batch loses,
+// whose launches are bound by the gathers, and the plan grows (first GMRES solve
+// 136 ms at 8, 200, 183 at 16, 1000).  By rows at 8, 200, the same two solves and
+// those of 1,119,744 tetrahedra and 1,008,000 hexahedra: 8,192 84.9, 67.1, 191.5,
+// 248.0; 16,384 78.3, 43.4, 188.8, 216.4; 32,768 70.1, 38.1, 179.4, 145.0; 65,536
+// 56.8, 38.1, 168.6, 127.5; 131,072 56.7, 38.1, 170.7, 127.9; 262,144 54.9, 38.1, 158.3,
+// 127.6.  Nothing is gained on hexahedra above 65,536, and the plan of the large
+// tetrahedra costs 110 ms more for 10 a solve.
 constexpr int kMergeLevels = 8;
 constexpr int kMergeTerms = 200;
 constexpr int kMergeRows = 65536;

@@ -1311,8 +1311,11 @@ __global__ void __launch_bounds__(kBlock) k_orth(const double* dots, const doubl
 // returns, so what sets the time is the number of launches and the chain of
 // loads in each (32,768 rows, FP64, step 15 of 30: product 5.0 with the
 // finalisation, dots 3.8, sums 3.0, update 3.9 us as four launches; 4.5 and 5.9
-// as two, and four SIMPLE steps of the cavity 40.3 -> 29.9 ms).  Above kBlock
-// tiles every block's own sums of all tiles cost more than the launch.
+// as two, and four SIMPLE steps of the cavity 40.3 -> 29.9 ms).  An iteration of
+// captured GMRES(30), two launches against four, us: 4,096 rows FP64 10.9 and 13.9,
+// mixed 11.6 and 15.0; 32,768 11.0 and 14.2, 11.0 and 14.0; 65,536 12.5 and 15.5, 12.0 and
+// 14.9.  kBlock tiles are what the sums below are written for (four 64-tile
+// pieces a wave); every block reads all tiles' sums, so the gain ends not far above.
 
 // The product w = M^-1 A V_it, and its dots with V_0..V_it: a block's rows are
 // one tile, so each thread still holds its w.  The first 8 basis vectors load

@@ -284,10 +284,13 @@ struct KWork {
 
 // Up to this many rows the momentum components are solved together: the launches
 // and level groups of small systems are shared, larger ones are bound by the
-// vectors' bytes, and three bases of theirs would take gigabytes.  Momentum phase
-// one after the other and together: GMRES(30) + ILU(0), 331,776 tetrahedra, FP64
-// 8.4 -> 4.7 ms; GMRES(50) + Jacobi, 748,410 rows, mixed 6.6 -> 5.4 ms (2.5 ms of
-// both are the copies of the fields from and to the host).
+// vectors' bytes, and three bases of theirs would take gigabytes.  solve_velocity
+// one after the other and together, ms: GMRES(50) + Jacobi, mixed and FP64,
+// 99,550 rows 1.54 -> 0.80 and 1.27 -> 0.68; 340,215 1.91 -> 1.31 and 1.75 -> 1.38;
+// 808,240 3.11 -> 2.18 and 2.63 -> 2.25; 1,566,245 3.71 -> 3.68 and 4.16 -> 4.09.
+// GMRES(30) + ILU(0), FP64 and mixed, 331,776 rows 4.26 -> 2.50 and 6.54 -> 3.51;
+// 786,432 6.51 -> 3.86 and 9.68 -> 4.96 (1,536,000: 9.25 -> 6.09, 10.6 -> 6.34, left
+// out for the memory).
 constexpr int kTripleRows = 1 << 20;
 
 // Buffers of the iterative-refinement solve (mixed precision).
