@@ -839,7 +839,11 @@ void Context::ensure_ilu_work(KWork& w) {
   w.ilu_own = alloc<T>(dm.Nc);
   w.ilu_zl = alloc<T>(2 * static_cast<size_t>(dm.Nc));
   w.ilu_zu = alloc<T>(2 * static_cast<size_t>(dm.Nc));
-  w.ilu_lcoef = alloc<T>(levels_.lower.slots);  // the last: says that all of it is there
+  // the padding's coefficients stay 0, the others are set per factorisation
+  fill_zero(w.ilu_ucoef, levels_.upper.slots * sizeof(T), stream);
+  T* lower = alloc<T>(levels_.lower.slots);
+  fill_zero(lower, levels_.lower.slots * sizeof(T), stream);
+  w.ilu_lcoef = lower;  // the last: says that all of it is there
 }
 
 void Context::ensure_mixed() {

@@ -106,7 +106,8 @@ struct RowSum;
 template <>
 struct RowSum<float> {
   double s = 0.0;
-  __device__ __forceinline__ void add(float c, float x) { s += static_cast<double>(c) * static_cast<double>(x); }
+  // (the product is exact, so the fused sum rounds as the separate one would)
+  __device__ __forceinline__ void add(float c, float x) { s = fma(static_cast<double>(c), static_cast<double>(x), s); }
   __device__ __forceinline__ void join(int mask) { s += __shfl_xor(s, mask, kWave); }
   __device__ __forceinline__ float value() const { return static_cast<float>(s); }
 };
@@ -136,10 +137,11 @@ struct RowSum<double> {
   }
 };
 
-// adds a row's terms u = lane, lane + Lanes, ... (W of them, slots `step` apart)
-template <class T, int W, int Lanes>
+// adds a row's terms u = lane, lane + Lanes, ... (W of them, slots `step` apart;
+// padding: coefficient 0 times the row's own input)
+template <class T, int W>
 __device__ __forceinline__ void ilu_terms(const int* __restrict__ col, const T* __restrict__ coef, const T* buf,
-                                          size_t q0, int step, int lane, int L, RowSum<T>& s) {
+                                          size_t q0, int step, RowSum<T>& s) {
   T v[W], x[W];
   int c[W];
 #pragma unroll
@@ -148,19 +150,16 @@ __device__ __forceinline__ void ilu_terms(const int* __restrict__ col, const T* 
     c[u] = col[q0 + static_cast<size_t>(u) * step];
   }
 #pragma unroll
-  for (int u = 0; u < W; ++u) x[u] = buf[c[u]];  // padding: the row's own input
+  for (int u = 0; u < W; ++u) x[u] = buf[c[u]];
 #pragma unroll
-  for (int u = 0; u < W; ++u) {
-    const bool in = u * Lanes + lane < L;
-    s.add(in ? v[u] : T(0), in ? x[u] : T(0));
-  }
+  for (int u = 0; u < W; ++u) s.add(v[u], x[u]);
 }
 
 // (own: the coefficient of each row's own input, null: 1; rcase: the case of
 // each row of a batch, whose finished cases' rows are left out)
 template <class T, bool Wide>
-__global__ void __launch_bounds__(kBlock) k_ilu_group(IluLaunch g, const int* __restrict__ len,
-                                                      const int* __restrict__ col, const T* __restrict__ coef,
+__global__ void __launch_bounds__(kBlock) k_ilu_group(IluLaunch g, const int* __restrict__ col,
+                                                      const T* __restrict__ coef,
                                                       const T* __restrict__ own, T* buf, int n, const KState* st,
                                                       const int* __restrict__ rcase) {
   buf += blockIdx.y * 2 * static_cast<size_t>(n);  // right-hand side blockIdx.y
@@ -185,24 +184,24 @@ __global__ void __launch_bounds__(kBlock) k_ilu_group(IluLaunch g, const int* __
   if (k >= nrows) return;  // the lanes of a row together
   const int p = p0 + k;
   if (st && st[rcase ? rcase[p] : blockIdx.y].reason) return;
-  const int L = len[p], step = nrows * lanes;
+  const int step = nrows * lanes;
   const size_t q0 = static_cast<size_t>(off) + i;
   RowSum<T> z;
   if (lane == 0) z.add(own ? own[p] : T(1), buf[p]);
   if (cls == 0) {
-    ilu_terms<T, 3, 1>(col, coef, buf, q0, step, lane, L, z);
+    ilu_terms<T, 3>(col, coef, buf, q0, step, z);
   } else if (cls == 1) {
-    ilu_terms<T, 6, 1>(col, coef, buf, q0, step, lane, L, z);
+    ilu_terms<T, 6>(col, coef, buf, q0, step, z);
   } else if (cls == 2) {
-    ilu_terms<T, 10, 1>(col, coef, buf, q0, step, lane, L, z);
+    ilu_terms<T, 10>(col, coef, buf, q0, step, z);
   } else if constexpr (Wide) {
     switch (cls) {
-      case 3: ilu_terms<T, 15, 1>(col, coef, buf, q0, step, lane, L, z); break;
-      case 4: ilu_terms<T, 8, 4>(col, coef, buf, q0, step, lane, L, z); break;
-      case 5: ilu_terms<T, 16, 4>(col, coef, buf, q0, step, lane, L, z); break;
+      case 3: ilu_terms<T, 15>(col, coef, buf, q0, step, z); break;
+      case 4: ilu_terms<T, 8>(col, coef, buf, q0, step, z); break;
+      case 5: ilu_terms<T, 16>(col, coef, buf, q0, step, z); break;
       default:
         for (int j = 0; j < width; j += 16 * kTermBatch)
-          ilu_terms<T, kTermBatch, 16>(col, coef, buf, q0 + static_cast<size_t>(j / 16) * step, step, lane, L - j, z);
+          ilu_terms<T, kTermBatch>(col, coef, buf, q0 + static_cast<size_t>(j / 16) * step, step, z);
         break;
     }
     if (lanes > 1) {
@@ -399,7 +398,7 @@ void ilu_sweep(const IluSweep& w, const T* coef, const T* own, T* buf, const KSt
       blocks += grid_for(static_cast<long>(u.nrows) * kTermLanes[c], b);
     }
     const bool wide = w.subs[w.group[g + 1] - 1].cls >= kNarrowClasses;
-    hipLaunchKernelGGL((wide ? k_ilu_group<T, true> : k_ilu_group<T, false>), dim3(blocks, rep), dim3(b), 0, s, a, w.len,
+    hipLaunchKernelGGL((wide ? k_ilu_group<T, true> : k_ilu_group<T, false>), dim3(blocks, rep), dim3(b), 0, s, a,
                        w.col, coef, own, buf, w.n, st, w.rcase);
   }
 }
