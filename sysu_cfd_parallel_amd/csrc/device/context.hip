@@ -777,35 +777,37 @@ void Context::ensure_ilu() {
     // both plans at once; the upper one waits for the lower one's rows where it
     // orders its own.  (Above 4 M rows one after the other: their tables would
     // take tens of gigabytes together.)
-    std::promise<void> lower_done;
-    const std::shared_future<void> lower_rows(lower_done.get_future());
+    std::promise<std::vector<int>> lower_known;
+    const std::shared_future<std::vector<int>> lower_rows(lower_known.get_future());
+    bool known = false;  // (a plan made again without merging: any order of its rows will do)
     IluPlan lower, upper;
     std::exception_ptr upper_failed;
     const bool at_once = dm.Nc <= (1 << 22);
-    std::thread upper_plan([&] {
+    auto make_upper = [&] {
       try {
-        if (!at_once) lower_rows.wait();
         upper = ilu_plan(
             dm.Nc, mesh.rowptr.data(), mesh.col.data(), mesh.diag.data(), true,
-            [&]() -> const std::vector<int>& {
-              lower_rows.get();
-              return lower.rows;
-            },
-            lay.cell);
+            [&]() -> const std::vector<int>& { return lower_rows.get(); }, lay.cell);
       } catch (...) {
         upper_failed = std::current_exception();
       }
-    });
+    };
+    std::thread upper_plan;
     Joined upper_joined{upper_plan};
+    if (at_once) upper_plan = std::thread(make_upper);
     try {
       lower = ilu_plan(
           dm.Nc, mesh.rowptr.data(), mesh.col.data(), mesh.diag.data(), false,
-          [&]() -> const std::vector<int>& { return natural; }, lay.cell);
-      lower_done.set_value();
+          [&]() -> const std::vector<int>& { return natural; }, lay.cell, kMergeLevels, kMergeRows, kMergeEntries,
+          [&](const std::vector<int>& rows) {
+            if (!known) lower_known.set_value(rows);
+            known = true;
+          });
     } catch (...) {
-      lower_done.set_exception(std::current_exception());
+      if (!known) lower_known.set_exception(std::current_exception());
       throw;
     }
+    if (!at_once) upper_plan = std::thread(make_upper);
     put(levels_.lower, lower, false);
     upper_plan.join();
     if (upper_failed) std::rethrow_exception(upper_failed);

@@ -36,7 +36,7 @@ struct TooLarge : std::invalid_argument {
 
 IluPlan build(int n, const int* rowptr, const int* col, const int* diag, bool upper,
               const std::function<const std::vector<int>&()>& order, const std::vector<int>& cases, int merge_levels,
-              int merge_rows, long most_entries) {
+              int merge_rows, long most_entries, const std::function<void(const std::vector<int>&)>& known) {
   if (n > kMost / 2) throw std::invalid_argument("ILU(0) sweeps above 32-bit indices");
   if (merge_levels < 1 || merge_levels > kMergeLevels) throw std::invalid_argument("ilu_plan: merge_levels");
   IluPlan out;
@@ -94,22 +94,33 @@ IluPlan build(int n, const int* rowptr, const int* col, const int* diag, bool up
   }
 
   // the terms of every row, depth by depth.  Code j: the input of row j, n + j:
-  // the result of row j.  Row i's terms are at start[i], count[i] of them; so
+  // the result of row j.  Row i's terms are at its start, count of them; so
   // are, for a row below depth 0, its pairs (term of the row, term of the row
   // referred to, -1 its own input), one run per reference in CSR order.
-  std::vector<long> start(static_cast<size_t>(n) + 1, 0);
-  for (int i = 0; i < n; ++i) start[i + 1] = start[i] + most[i];
-  if (merge_levels > 1 && start[n] > most_entries) throw TooLarge("ILU(0) merged rows");
+  // (what another row reads of a row stands together: the loops wait for memory)
+  struct Row {
+    long start;
+    int grp, count;
+  };
+  std::vector<Row> row(n);
+  long entries = 0;
+  for (int i = 0; i < n; ++i) {
+    row[i] = Row{entries, grp[i], 0};
+    entries += most[i];
+  }
+  if (merge_levels > 1 && entries > most_entries) throw TooLarge("ILU(0) merged rows");
   IntArray code, src, pr, pq;
-  for (IntArray* x : {&code, &src, &pr, &pq}) x->resize(start[n]);
-  std::vector<int> count(n), nstep(n, 0), npair(n, 0);
+  for (IntArray* x : {&code, &src, &pr, &pq}) x->resize(entries);
+  IntArray nstep, npair, key;  // key: group and class of terms
+  for (IntArray* x : {&nstep, &npair, &key}) x->resize(n);
   for (int d = 0; d < merge_levels; ++d) {
     const std::vector<int>& list = dlist[d];
     parallel_for(
         static_cast<long>(list.size()),
         [&](long k) {
           const int i = list[k];
-          const long s = start[i];
+          const long s = row[i].start;
+          const int g = row[i].grp;
           int m = 0, pairs = 0, steps = 0;
           int* const codes = code.data() + s;
           // the term of code c, looked for among the first `before` (the codes of
@@ -124,37 +135,36 @@ IluPlan build(int n, const int* rowptr, const int* col, const int* diag, bool up
           };
           for (int x = first(i); x < last(i); ++x) {
             const int j = col[x];
-            if (grp[j] != grp[i]) {
+            const Row from = row[j];
+            if (from.grp != g) {
               src[s + term(n + j, m)] = x;
               continue;
             }
             ++steps;
             const int before = m;
-            for (int y = -1; y < count[j]; ++y) {  // -1: row j's own input
-              pr[s + pairs] = term(y < 0 ? j : code[start[j] + y], before);
+            for (int y = -1; y < from.count; ++y) {  // -1: row j's own input
+              pr[s + pairs] = term(y < 0 ? j : code[from.start + y], before);
               pq[s + pairs] = y;
               ++pairs;
             }
           }
-          count[i] = m;
+          row[i].count = m;
           nstep[i] = steps;
           npair[i] = pairs;
+          int c = 0;
+          while (m > kTermWidth[c]) ++c;
+          key[i] = g * kTermClasses + c;
         },
         1 << 12);
   }
 
   // sweep order: by (group, class), keeping the order given
-  auto key = [&](int i) {
-    int c = 0;
-    while (count[i] > kTermWidth[c]) ++c;
-    return static_cast<long>(grp[i]) * kTermClasses + c;
-  };
   const long nkey = static_cast<long>(ngroup) * kTermClasses;
   std::vector<int> kptr(nkey + 1, 0), width(nkey, 0);
   for (int i = 0; i < n; ++i) {
-    const long k = key(i);
+    const int k = key[i];
     ++kptr[k + 1];
-    width[k] = std::max(width[k], count[i]);
+    width[k] = std::max(width[k], row[i].count);
   }
   for (long k = 0; k < nkey; ++k) kptr[k + 1] += kptr[k];
   out.rows.resize(n);
@@ -162,11 +172,12 @@ IluPlan build(int n, const int* rowptr, const int* col, const int* diag, bool up
   {
     std::vector<int> at(kptr.begin(), kptr.end() - 1);
     for (int i : order()) {
-      const int p = at[key(i)]++;
+      const int p = at[key[i]]++;
       out.rows[p] = i;
       out.pos[i] = p;
     }
   }
+  if (known) known(out.rows);
   long slots = 0;
   out.group.assign(1, 0);
   out.len.resize(n);
@@ -198,18 +209,27 @@ IluPlan build(int n, const int* rowptr, const int* col, const int* diag, bool up
   }
   out.col.resize(slots);
   out.src.resize(slots);
+  struct Place {
+    int pos, slot0, stride, shift;  // (lanes: 1 << shift)
+    int slot(int u) const { return slot0 + (u >> shift) * stride + (u & ((1 << shift) - 1)); }
+  };
+  std::vector<Place> place(n);
   parallel_for(
       n,
       [&](long k) {
         const int p = static_cast<int>(k), i = out.rows[p];
-        out.len[p] = count[i];
+        const Row own = row[i];
+        const int lanes = out.lanes[p];
+        const Place at_p{p, out.slot0[p], out.stride[p], lanes == 1 ? 0 : lanes == 4 ? 2 : 4};
+        place[i] = at_p;
+        out.len[p] = own.count;
         out.depth[p] = dep[i];
         for (int u = 0; u < width_of[p]; ++u) {
-          const int at = out.slot(p, u);
-          if (u < count[i]) {
-            const int c = code[start[i] + u];
+          const int at = at_p.slot(u);
+          if (u < own.count) {
+            const int c = code[own.start + u];
             out.col[at] = c < n ? out.pos[c] : n + out.pos[c - n];
-            out.src[at] = src[start[i] + u];
+            out.src[at] = src[own.start + u];
           } else {
             out.col[at] = p;
             out.src[at] = -1;
@@ -247,17 +267,19 @@ IluPlan build(int n, const int* rowptr, const int* col, const int* diag, bool up
   parallel_for(
       static_cast<long>(nl),
       [&](long k) {
-        const int pi = out.later[k], i = out.rows[pi];
+        const int i = out.rows[out.later[k]];
+        const Place to = place[i];
+        const int g = row[i].grp;
         int x0 = out.sptr[k];
-        long at = pairs[k], from = start[i];
+        long at = pairs[k], from = row[i].start;
         for (int x = first(i); x < last(i); ++x) {
           const int j = col[x];
-          if (grp[j] != grp[i]) continue;
-          const int pj = out.pos[j], most_terms = count[j];
+          if (row[j].grp != g) continue;
+          const Place by = place[j];
           out.p[x0] = x;
-          for (int y = -1; y < most_terms; ++y, ++at, ++from) {
-            out.r[at] = out.slot(pi, pr[from]);
-            out.q[at] = pq[from] < 0 ? -1 - pj : out.slot(pj, pq[from]);
+          for (int y = -1; y < row[j].count; ++y, ++at, ++from) {
+            out.r[at] = to.slot(pr[from]);
+            out.q[at] = pq[from] < 0 ? -1 - by.pos : by.slot(pq[from]);
           }
           out.uptr[++x0] = static_cast<int>(at);
         }
@@ -270,12 +292,12 @@ IluPlan build(int n, const int* rowptr, const int* col, const int* diag, bool up
 
 IluPlan ilu_plan(int n, const int* rowptr, const int* col, const int* diag, bool upper,
                  const std::function<const std::vector<int>&()>& order, const std::vector<int>& cases, int merge_levels,
-                 int merge_rows, long most_entries) {
+                 int merge_rows, long most_entries, const std::function<void(const std::vector<int>&)>& known) {
   try {
-    return build(n, rowptr, col, diag, upper, order, cases, merge_levels, merge_rows, most_entries);
+    return build(n, rowptr, col, diag, upper, order, cases, merge_levels, merge_rows, most_entries, known);
   } catch (const TooLarge&) {
     if (merge_levels == 1) throw;
-    return build(n, rowptr, col, diag, upper, order, cases, 1, merge_rows, most_entries);
+    return build(n, rowptr, col, diag, upper, order, cases, 1, merge_rows, most_entries, known);
   }
 }
 

@@ -119,13 +119,15 @@ struct IluPlan {
 // The plan of the lower (strictly lower entries) or upper sweep of a CSR
 // pattern with sorted columns; order is the order rows keep inside a group
 // and class (as a function: asked for once the terms are known, so that the upper
-// sweep's, the lower plan's rows, can be built at the same time), cases the
-// first row of each case and n.  Where merged rows would take more than
+// sweep's, the lower plan's rows, can be built at the same time; known is called
+// with a plan's rows as soon as they are ordered), cases the first row of each
+// case and n.  Where merged rows would take more than
 // most_entries entries, or a table passes 32-bit indices, nothing is merged; throws
 // std::invalid_argument where a table passes them all the same.
 IluPlan ilu_plan(int n, const int* rowptr, const int* col, const int* diag, bool upper,
                  const std::function<const std::vector<int>&()>& order, const std::vector<int>& cases,
-                 int merge_levels = kMergeLevels, int merge_rows = kMergeRows, long most_entries = kMergeEntries);
+                 int merge_levels = kMergeLevels, int merge_rows = kMergeRows, long most_entries = kMergeEntries,
+                 const std::function<void(const std::vector<int>&)>& known = {});
 inline IluPlan ilu_plan(int n, const int* rowptr, const int* col, const int* diag, bool upper,
                         const std::vector<int>& order, const std::vector<int>& cases,
                         int merge_levels = kMergeLevels, int merge_rows = kMergeRows,
