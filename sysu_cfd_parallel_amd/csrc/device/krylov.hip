@@ -99,10 +99,11 @@ struct IluLaunch {
 // times that of plain solves in T (hexahedra, tetrahedra, both mixed, FP64 and
 // FP32), summed so it is 0.7-0.8 of theirs.  The coefficients stay rounded to T; they
 // make no difference that can be measured.  The kernel waits for loads most of
-// the time: with the terms tested against the row's length the exact sums cost
-// 3-5 % of a solve, with padding coefficients of 0 instead (CG, 331,776 tetrahedra,
-// FP64) 54.8 ms before, 57.6 and 53.4; (mixed GMRES(50), 310,000 hexahedra) 34.7, 36.3
-// and 35.5.
+// the time, so the sums cost little: a solve with plain sums and with these, CG on
+// 331,776 tetrahedra in FP64 54.9 and 53.1 ms, mixed GMRES(50) on 310,000 hexahedra
+// 36.4 and 36.2, on 6.0 M hexahedra 828.7 and 841.6 (the conversions of FP32).  They
+// cost 3-5 % with the terms tested against the row's length, in place of padding
+// coefficients of 0, and the row's input added before the slots were on their way.
 template <class T>
 struct RowSum;
 
@@ -140,11 +141,12 @@ struct RowSum<double> {
   }
 };
 
-// adds a row's terms u = lane, lane + Lanes, ... (W of them, slots `step` apart;
-// padding: coefficient 0 times the row's own input)
+// adds o x0 and then a row's terms u = lane, lane + Lanes, ... (W of them, slots
+// `step` apart; padding: coefficient 0 times the row's own input).  (The additions
+// come after the last load: one that waits for x0 first holds the slots up.)
 template <class T, int W>
 __device__ __forceinline__ void ilu_terms(const int* __restrict__ col, const T* __restrict__ coef, const T* buf,
-                                          size_t q0, int step, RowSum<T>& s) {
+                                          size_t q0, int step, T o, T x0, RowSum<T>& s) {
   T v[W], x[W];
   int c[W];
 #pragma unroll
@@ -154,13 +156,14 @@ __device__ __forceinline__ void ilu_terms(const int* __restrict__ col, const T* 
   }
 #pragma unroll
   for (int u = 0; u < W; ++u) x[u] = buf[c[u]];
+  s.add(o, x0);
 #pragma unroll
   for (int u = 0; u < W; ++u) s.add(v[u], x[u]);
 }
 
-// (own: the coefficient of each row's own input, null: 1; rcase: the case of
-// each row of a batch, whose finished cases' rows are left out)
-template <class T, bool Wide>
+// (own: the coefficient of each row's own input in the upper sweep, 1 in the lower;
+// rcase: the case of each row of a batch, whose finished cases' rows are left out)
+template <class T, bool Wide, bool Upper>
 __global__ void __launch_bounds__(kBlock) k_ilu_group(IluLaunch g, const int* __restrict__ col,
                                                       const T* __restrict__ coef,
                                                       const T* __restrict__ own, T* buf, int n, const KState* st,
@@ -189,22 +192,24 @@ __global__ void __launch_bounds__(kBlock) k_ilu_group(IluLaunch g, const int* __
   if (st && st[rcase ? rcase[p] : blockIdx.y].reason) return;
   const int step = nrows * lanes;
   const size_t q0 = static_cast<size_t>(off) + i;
+  T o = T(1), x0 = buf[p];
+  if constexpr (Upper) o = own[p];
+  if constexpr (Wide) x0 = lane == 0 ? x0 : T(0);
   RowSum<T> z;
-  if (lane == 0) z.add(own ? own[p] : T(1), buf[p]);
   if (cls == 0) {
-    ilu_terms<T, 3>(col, coef, buf, q0, step, z);
+    ilu_terms<T, 3>(col, coef, buf, q0, step, o, x0, z);
   } else if (cls == 1) {
-    ilu_terms<T, 6>(col, coef, buf, q0, step, z);
+    ilu_terms<T, 6>(col, coef, buf, q0, step, o, x0, z);
   } else if (cls == 2) {
-    ilu_terms<T, 10>(col, coef, buf, q0, step, z);
+    ilu_terms<T, 10>(col, coef, buf, q0, step, o, x0, z);
   } else if constexpr (Wide) {
     switch (cls) {
-      case 3: ilu_terms<T, 15>(col, coef, buf, q0, step, z); break;
-      case 4: ilu_terms<T, 8>(col, coef, buf, q0, step, z); break;
-      case 5: ilu_terms<T, 16>(col, coef, buf, q0, step, z); break;
+      case 3: ilu_terms<T, 15>(col, coef, buf, q0, step, o, x0, z); break;
+      case 4: ilu_terms<T, 8>(col, coef, buf, q0, step, o, x0, z); break;
+      case 5: ilu_terms<T, 16>(col, coef, buf, q0, step, o, x0, z); break;
       default:
         for (int j = 0; j < width; j += 16 * kTermBatch)
-          ilu_terms<T, kTermBatch>(col, coef, buf, q0 + static_cast<size_t>(j / 16) * step, step, z);
+          ilu_terms<T, kTermBatch>(col, coef, buf, q0 + static_cast<size_t>(j / 16) * step, step, o, j ? T(0) : x0, z);
         break;
     }
     if (lanes > 1) {
@@ -383,7 +388,7 @@ void ilu_factor(const CsrView<T>& A, int nnz, const IluLevels& lv, T* lu, hipStr
 }
 
 // one sweep, group by group, on buf: n inputs, then n results
-template <class T>
+template <class T, bool Upper>
 void ilu_sweep(const IluSweep& w, const T* coef, const T* own, T* buf, const KState* st, int rep, hipStream_t s) {
   for (size_t g = 0; g + 1 < w.group.size(); ++g) {
     IluLaunch a{};
@@ -401,7 +406,7 @@ void ilu_sweep(const IluSweep& w, const T* coef, const T* own, T* buf, const KSt
       blocks += grid_for(static_cast<long>(u.nrows) * kTermLanes[c], b);
     }
     const bool wide = w.subs[w.group[g + 1] - 1].cls >= kNarrowClasses;
-    hipLaunchKernelGGL((wide ? k_ilu_group<T, true> : k_ilu_group<T, false>), dim3(blocks, rep), dim3(b), 0, s, a,
+    hipLaunchKernelGGL((wide ? k_ilu_group<T, true, Upper> : k_ilu_group<T, false, Upper>), dim3(blocks, rep), dim3(b), 0, s, a,
                        w.col, coef, own, buf, w.n, st, w.rcase);
   }
 }
@@ -436,9 +441,9 @@ void ilu_apply(const CsrView<T>& A, const IluLevels& lv, const T* lu, const T* r
   // r into the lower order, the lower sweep, its result into the upper
   // order, the upper sweep, z back into the natural order
   hipLaunchKernelGGL((k_scatter<T, 0>), gn, dim3(kBlock), 0, s, n, lv.lpos, r, n1, zl, 2 * n1, st_move);
-  ilu_sweep<T>(lv.lower, static_cast<const T*>(w->ilu_lcoef), static_cast<const T*>(nullptr), zl, st, rep, s);
+  ilu_sweep<T, false>(lv.lower, static_cast<const T*>(w->ilu_lcoef), static_cast<const T*>(nullptr), zl, st, rep, s);
   hipLaunchKernelGGL((k_scatter<T, 1>), gn, dim3(kBlock), 0, s, n, lv.l2u, zl + n, 2 * n1, zu, 2 * n1, st_move);
-  ilu_sweep<T>(lv.upper, static_cast<const T*>(w->ilu_ucoef), static_cast<const T*>(w->ilu_own), zu, st, rep, s);
+  ilu_sweep<T, true>(lv.upper, static_cast<const T*>(w->ilu_ucoef), static_cast<const T*>(w->ilu_own), zu, st, rep, s);
   if (dot)
     hipLaunchKernelGGL((k_gather_at<T, 2, true>), gn, dim3(kBlock), 0, s, n, lv.upos, zu + n, z, st, r, dot);
   else
